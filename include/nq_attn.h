@@ -399,8 +399,8 @@ int64_t nq_qk_norm_rope_bwd_workspace_bytes(int B, int S, int H, int D);
  * gradient dy of y = rope(rmsnorm(x) * weight), writes dx and the weight
  * gradient dweight (fp32, D elements, fully written).  The blocks store
  * partial sums of dweight in the workspace
- * (nq_qk_norm_rope_bwd_workspace_bytes), which a second launch adds in block
- * order: dweight is the same bit for bit on every run.  weight / dweight
+ * (nq_qk_norm_rope_bwd_workspace_bytes), which a second launch adds in a
+ * fixed order: dweight is the same bit for bit on every run.  weight / dweight
  * NULL: no norm (workspace unused); cos_tab NULL: no rotation.  Positions as
  * in nq_qk_norm_rope.  x, dy, dx: (B, H, S, D) with strides {batch, head,
  * seq}.

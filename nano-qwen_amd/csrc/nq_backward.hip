@@ -657,7 +657,7 @@ static hipError_t launch_bwd(const BwdParams& p, int nw, bool causal, hipStream_
 // the forward row kernel (D/16 lanes, a lane owns 8 elements and their
 // rotate-half partners).  dw is accumulated per block in LDS and each block
 // stores its partial sum in the workspace; a second launch adds the partials
-// in block order, so dw is the same bit for bit on every run (no atomics).
+// in a fixed order, so dw is the same bit for bit on every run (no atomics).
 struct NormBwdParams {
   const void* x;
   int64_t xsb, xsh, xss;
@@ -749,23 +749,25 @@ __global__ __launch_bounds__(256) void norm_rope_bwd_kernel(NormBwdParams p) {
   }
 }
 
-// dw[d] = sum of the nblk partials in block order: 256 threads, thread t adds
-// blocks t / D, t / D + 256 / D, ... of column t % D, then the 256 / D column
-// sums are added in thread order.
+// dw[d] = sum of the nblk per-block partials, in a fixed order (64 row slots,
+// then a butterfly over them): the same bits on every run.  Latency-bound (at
+// most 512 KiB, in L2), so it is split by columns: workgroup x owns columns
+// 4x .. 4x+3, thread t adds partials t/4, t/4 + 64, ... of column t%4, all its
+// loads independent.  One workgroup for all D columns, each thread adding up to
+// 512 partials, took 122 us at 1024 partials x D = 128; this takes 4.5 us.
 template <int D>
 __global__ __launch_bounds__(256) void norm_dw_reduce_kernel(const float* ws, int nblk, float* dw) {
-  constexpr int LANES = 256 / D;
-  __shared__ float part[LANES][D];
-  const int d = threadIdx.x % D, l = threadIdx.x / D;
+  __shared__ float part[4][4];
+  const int c = threadIdx.x & 3, lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  const float* col = ws + 4 * blockIdx.x + c;
   float t = 0.f;
-  for (int i = l; i < nblk; i += LANES) t += ws[(int64_t)i * D + d];
-  part[l][d] = t;
+#pragma unroll 8
+  for (int i = threadIdx.x >> 2; i < nblk; i += 64) t += col[(int64_t)i * D];
+#pragma unroll
+  for (int m = 4; m < 64; m <<= 1) t += __shfl_xor(t, m, 64);
+  if (lane < 4) part[wave][c] = t;
   __syncthreads();
-  if (l == 0) {
-    float s = 0.f;
-    for (int i = 0; i < LANES; ++i) s += part[i][d];
-    dw[d] = s;
-  }
+  if (threadIdx.x < 4) dw[4 * blockIdx.x + c] = (part[0][c] + part[1][c]) + (part[2][c] + part[3][c]);
 }
 
 }  // namespace nq
@@ -962,7 +964,7 @@ extern "C" int nq_qk_norm_rope_bwd(const void* x, const int64_t* x_strides, cons
     constexpr int DD = decltype(dc)::value;
     if (dtype == NQ_DTYPE_BF16) hipLaunchKernelGGL((norm_rope_bwd_kernel<bf16, DD>), grid, dim3(256), 0, st, p);
     else hipLaunchKernelGGL((norm_rope_bwd_kernel<float, DD>), grid, dim3(256), 0, st, p);
-    if (weight) hipLaunchKernelGGL((norm_dw_reduce_kernel<DD>), dim3(1), dim3(256), 0, st, p.ws, nblk, dweight);
+    if (weight) hipLaunchKernelGGL((norm_dw_reduce_kernel<DD>), dim3(DD / 4), dim3(256), 0, st, p.ws, nblk, dweight);
     return 0;
   });
   return nq_check_launch(hipGetLastError());

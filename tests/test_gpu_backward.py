@@ -175,6 +175,26 @@ def test_norm_rope_backward_against_fp64_autograd(dtype, D):
     torch.testing.assert_close(dw.double().cpu(), wd.grad, rtol=tol, atol=tol * float(wd.grad.abs().max()))
 
 
+@pytest.mark.parametrize("blocks", [1, 2, 63, 64, 65, 513, 1024])
+@pytest.mark.parametrize("D", [32, 128])
+def test_norm_weight_gradient_sum_over_blocks(D, blocks):
+    """The second launch adds one partial per 256 / (D/16) rows: counts around its 64 row slots, and the cap."""
+    say(f"norm weight gradient D={D} blocks={blocks}")
+    S = blocks * (4096 // D) - (1 if blocks > 1 else 0)  # the last block one row short
+    x = randn(1, 1, S, D, seed=535).to(DEV)
+    dy = randn(1, 1, S, D, seed=536).to(DEV)
+    w = (1 + 0.1 * randn(D, seed=537)).to(DEV)
+    _, dw = ops.qk_norm_rope_backward(x, dy, weight=w, eps=1e-6)
+    xd = x.double()
+    terms = dy.double() * xd * torch.rsqrt(xd.square().mean(-1, keepdim=True) + 1e-6)
+    # each term carries a few roundings (the norm's rsqrt among them), then a
+    # chain of rows-per-slot + 32 + 16 + 8 additions: (8 + 64) * 2^-24 of the
+    # terms' magnitudes bounds it
+    bound = 72 * 2.0 ** -24 * terms.abs().sum((0, 1, 2))
+    assert bool(((dw.double() - terms.sum((0, 1, 2))).abs() <= bound).all())
+    assert torch.equal(dw, ops.qk_norm_rope_backward(x, dy, weight=w, eps=1e-6)[1])
+
+
 def test_flash_attention_mirror_autograd():
     say("flash_attention autograd")
     B, H, S, D = 2, 4, 96, 64
