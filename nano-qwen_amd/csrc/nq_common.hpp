@@ -186,10 +186,11 @@ __device__ __forceinline__ void store8<float>(float* p, floatx8 v) {
   *reinterpret_cast<floatx4*>(p + 4) = floatx4{v[4], v[5], v[6], v[7]};
 }
 
+// two consecutive elements, p a multiple of two elements
 template <typename T>
 __device__ __forceinline__ void store2(T* p, float a, float b) {
-  p[0] = (T)a;
-  p[1] = (T)b;
+  typedef T pair __attribute__((ext_vector_type(2)));
+  *reinterpret_cast<pair*>(p) = pair{(T)a, (T)b};
 }
 
 template <typename T>

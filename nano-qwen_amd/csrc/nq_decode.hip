@@ -51,6 +51,8 @@ constexpr int DC_WAVES = DC_THREADS / 64;
 constexpr int DC_STEP = 32;      // keys per wave step
 constexpr int DC_WG_PER_CU = 1;  // resident workgroups per CU for the persistent grid
 constexpr int DC_MAX_WAVES = 1024;  // persistent grid cap: 256 CUs x 1 workgroup x 4 waves
+constexpr int DC_MERGE_MAX_THREADS = 1024;
+constexpr int DC_MERGE_WIDE_PARTIALS = 16;  // launched waves per row from which a row's merge takes 1024 threads
 
 struct DecodeParams {
   const void* q;
@@ -76,6 +78,7 @@ struct DecodeParams {
   int q_pos0;
   int B, Hq, Hkv, G, NG, max_len;
   int rows_per_batch;  // Hkv * NG
+  int hs;              // the merge's heads per slice: 2^hs >= min(G, 16)
   int nwaves;          // waves launched
   int span;            // steps per wave; 0 = split N evenly over nwaves
   float scale_log2;
@@ -558,9 +561,11 @@ decode_stream_kernel(DecodeParams p) {
     } else {
       const int64_t slot = w + r;
       float* so = p.ws_o + (slot * 16 + c16) * D;
+      if (hvalid) {  // the merge reads no other heads
 #pragma unroll
-      for (int dd = 0; dd < NDO; ++dd) *reinterpret_cast<floatx4*>(so + dd * 16 + grp * 4) = oacc[dd];
-      if (grp == 0) *reinterpret_cast<floatx2*>(p.ws_ml + (slot * 16 + c16) * 2) = floatx2{m_i, l_i};
+        for (int dd = 0; dd < NDO; ++dd) *reinterpret_cast<floatx4*>(so + dd * 16 + grp * 4) = oacc[dd];
+        if (grp == 0) *reinterpret_cast<floatx2*>(p.ws_ml + (slot * 16 + c16) * 2) = floatx2{m_i, l_i};
+      }
     }
 
     q += nseg;
@@ -575,33 +580,36 @@ decode_stream_kernel(DecodeParams p) {
 
 // One workgroup per row (batch, kv head, head group): combines the partials
 // of the waves that covered the row, or writes zeros for a row without keys.
-// Thread t owns head t / 16 of the group and DPT consecutive dims.
+// 16 threads hold a head (D/16 consecutive dims each); the workgroup's threads
+// make up slices of the row's 2^p.hs heads, and slice i takes partials i,
+// i + slices, ...: the partials' round trips to memory overlap, and the slices
+// meet in LDS, each thread then adding them for two output dims.  Latency-bound
+// (a few MB in all).  With one slice of 16 heads, B1 32/8 heads with 1500 keys
+// (48 partials a row, 4 heads) took 11.5 us; 16 slices of 4 heads take 5.0 us.
 template <int D, typename T>
-__global__ void __launch_bounds__(DC_THREADS) decode_merge_kernel(DecodeParams p) {
+__global__ void __launch_bounds__(DC_MERGE_MAX_THREADS) decode_merge_kernel(DecodeParams p) {
   constexpr int DPT = D / 16;  // dims per thread (8, 4 or 2)
+  extern __shared__ float merge_lds[];
   const int64_t r = blockIdx.x;
   const int b = (int)(r / p.rows_per_batch), j = (int)(r % p.rows_per_batch);
   const int kvh = j / p.NG, hg = j % p.NG;
-  const int hq = threadIdx.x >> 4, d0 = (threadIdx.x & 15) * DPT;
-  const int gh = hg * 16 + hq;
+  const int heads = 1 << p.hs, slots = blockDim.x >> 4, slices = slots >> p.hs;
+  const int slot = threadIdx.x >> 4, d0 = (threadIdx.x & 15) * DPT;
+  const int hq = slot & (heads - 1), slice = slot >> p.hs;
+  const int nh = min(heads, p.G - hg * 16);  // valid heads of the group
   // the row's first and last covering wave, read through the scalar path
   // alongside lens[b] (a row without keys never uses them)
   const int64_t wf = ld_uniform(p.ws_rw, r * 2), wl = ld_uniform(p.ws_rw, r * 2 + 1);
   const int len = uniform(batch_len(p, b));
   if (p.lens_out && j == 0 && threadIdx.x == 0) p.lens_out[b] = len < 0 ? p.lens[b] : p.lens[b] + 1;
-  T* orow = reinterpret_cast<T*>(p.o) + b * p.osb + (int64_t)(kvh * p.G + (gh < p.G ? gh : 0)) * p.osh + d0;
+  T* out = reinterpret_cast<T*>(p.o) + b * p.osb + (int64_t)(kvh * p.G + hg * 16) * p.osh;
   if (len <= 0) {  // no keys: zeros; a length out of range: NaN
-    if (gh < p.G) {
-      const float f = len < 0 ? __builtin_nanf("") : 0.f;
-      if constexpr (DPT == 8) store8<T>(orow, floatx8{f, f, f, f, f, f, f, f});
-      else if constexpr (DPT == 4) store4<T>(orow, floatx4{f, f, f, f});
-      else store2<T>(orow, f, f);
-    }
+    const float f = len < 0 ? __builtin_nanf("") : 0.f;
+    for (int t = threadIdx.x; t < nh * (D / 2); t += blockDim.x)
+      store2<T>(out + (t / (D / 2)) * p.osh + (t % (D / 2)) * 2, f, f);
     return;
   }
-  if (wf == wl || gh >= p.G) return;  // one wave covered the row and wrote it
-  const float* ml = p.ws_ml + ((wf + r) * 16 + hq) * 2;
-  const float* po = p.ws_o + ((wf + r) * 16 + hq) * D + d0;
+  if (wf == wl) return;  // one wave covered the row and wrote it
   const int ns = (int)(wl - wf + 1);
   // one pass with a running max, so every partial's (m, l) and outputs are
   // loaded together (every partial holds at least one key: its m is finite)
@@ -609,38 +617,74 @@ __global__ void __launch_bounds__(DC_THREADS) decode_merge_kernel(DecodeParams p
   float acc[DPT];
 #pragma unroll
   for (int e = 0; e < DPT; ++e) acc[e] = 0.f;
+  const float* ml = p.ws_ml + ((wf + r) * 16 + hq) * 2;
+  const float* po = p.ws_o + ((wf + r) * 16 + hq) * D + d0;
+  auto add = [&](int first, auto stride) {
 #pragma unroll 4
-  for (int i = 0; i < ns; ++i) {
-    const floatx2 m_l = *reinterpret_cast<const floatx2*>(ml + i * 32);
-    float o[DPT];
-    if constexpr (DPT == 2) {
-      const floatx2 o2 = *reinterpret_cast<const floatx2*>(po + (int64_t)i * 16 * D);
-      o[0] = o2[0];
-      o[1] = o2[1];
-    } else {
+    for (int i = first; i < ns; i += stride) {
+      const floatx2 m_l = *reinterpret_cast<const floatx2*>(ml + i * 32);
+      float o[DPT];
+      if constexpr (DPT == 2) {
+        const floatx2 o2 = *reinterpret_cast<const floatx2*>(po + (int64_t)i * 16 * D);
+        o[0] = o2[0];
+        o[1] = o2[1];
+      } else {
 #pragma unroll
-      for (int e = 0; e < DPT; e += 4) {
-        const floatx4 o4 = *reinterpret_cast<const floatx4*>(po + (int64_t)i * 16 * D + e);
+        for (int e = 0; e < DPT; e += 4) {
+          const floatx4 o4 = *reinterpret_cast<const floatx4*>(po + (int64_t)i * 16 * D + e);
 #pragma unroll
-        for (int k = 0; k < 4; ++k) o[e + k] = o4[k];
+          for (int k = 0; k < 4; ++k) o[e + k] = o4[k];
+        }
       }
-    }
-    const float Mn = fmaxf(M, m_l[0]);
-    const float a = fast_exp2(M - Mn);  // 0 for the first partial
-    const float sc = fast_exp2(m_l[0] - Mn);
-    wsum = wsum * a + m_l[1] * sc;
+      const float Mn = fmaxf(M, m_l[0]);
+      const float a = fast_exp2(M - Mn);  // 0 for the first partial
+      const float sc = fast_exp2(m_l[0] - Mn);
+      wsum = wsum * a + m_l[1] * sc;
 #pragma unroll
-    for (int e = 0; e < DPT; ++e) acc[e] = acc[e] * a + o[e] * sc;
-    M = Mn;
+      for (int e = 0; e < DPT; ++e) acc[e] = acc[e] * a + o[e] * sc;
+      M = Mn;
+    }
+  };
+  if (slices == 1) {
+    if (hq >= nh) return;
+    add(0, std::integral_constant<int, 1>{});
+    const float inv = 1.0f / wsum;
+    T* orow = out + hq * p.osh + d0;
+    if constexpr (DPT == 8) {
+      store8<T>(orow, floatx8{acc[0] * inv, acc[1] * inv, acc[2] * inv, acc[3] * inv,
+                              acc[4] * inv, acc[5] * inv, acc[6] * inv, acc[7] * inv});
+    } else if constexpr (DPT == 4) {
+      store4<T>(orow, floatx4{acc[0] * inv, acc[1] * inv, acc[2] * inv, acc[3] * inv});
+    } else {
+      store2<T>(orow, acc[0] * inv, acc[1] * inv);
+    }
+    return;
   }
-  const float inv = 1.0f / wsum;
-  if constexpr (DPT == 8) {
-    store8<T>(orow, floatx8{acc[0] * inv, acc[1] * inv, acc[2] * inv, acc[3] * inv,
-                            acc[4] * inv, acc[5] * inv, acc[6] * inv, acc[7] * inv});
-  } else if constexpr (DPT == 4) {
-    store4<T>(orow, floatx4{acc[0] * inv, acc[1] * inv, acc[2] * inv, acc[3] * inv});
-  } else {
-    store2<T>(orow, acc[0] * inv, acc[1] * inv);
+  if (hq < nh) add(slice, slices);
+  // slot (slice, head): D sums, then its max and weight (a slice without
+  // partials: M = -inf, weight 0)
+  float* mine = merge_lds + slot * (D + 2);
+#pragma unroll
+  for (int e = 0; e < DPT; e += 2) *reinterpret_cast<floatx2*>(mine + d0 + e) = floatx2{acc[e], acc[e + 1]};
+  if (d0 == 0) *reinterpret_cast<floatx2*>(mine + D) = floatx2{M, wsum};
+  __syncthreads();
+  const int used = min(slices, ns);  // slices that hold partials
+  for (int t = threadIdx.x; t < nh * (D / 2); t += blockDim.x) {
+    const int h = t / (D / 2), d = (t % (D / 2)) * 2;
+    const float* s0 = merge_lds + h * (D + 2);
+    const int step = heads * (D + 2);
+    float top = s0[D];
+    for (int i = 1; i < used; ++i) top = fmaxf(top, s0[i * step + D]);
+    float sum = 0.f, a0 = 0.f, a1 = 0.f;
+    for (int i = 0; i < used; ++i) {
+      const float* si = s0 + i * step;
+      const float f = fast_exp2(si[D] - top);
+      sum = __builtin_fmaf(si[D + 1], f, sum);
+      a0 = __builtin_fmaf(si[d], f, a0);
+      a1 = __builtin_fmaf(si[d + 1], f, a1);
+    }
+    const float inv = 1.0f / sum;
+    store2<T>(out + h * p.osh + d, a0 * inv, a1 * inv);
   }
 }
 
@@ -689,7 +733,12 @@ static hipError_t launch_decode(DecodeParams p, hipStream_t st) {
   hipError_t e = hipGetLastError();
   if (e != hipSuccess) return e;
   const int64_t rows = (int64_t)p.B * p.rows_per_batch;
-  hipLaunchKernelGGL((decode_merge_kernel<D, T>), dim3((unsigned)rows), dim3(DC_THREADS), 0, st, p);
+  // 16 waves per row while the rows are few (each then has many partials, and
+  // the CUs are idle anyway), four where a row has a handful: at 4 waves a row
+  // (B64, 4 kv heads, G = 16) 16 waves took 6.3 us and four 5.4
+  const int threads = rows * DC_MERGE_WIDE_PARTIALS <= p.nwaves ? DC_MERGE_MAX_THREADS : DC_THREADS;
+  hipLaunchKernelGGL((decode_merge_kernel<D, T>), dim3((unsigned)rows), dim3(threads),
+                     (threads / 16) * (D + 2) * sizeof(float), st, p);
   return hipGetLastError();
 }
 
@@ -736,6 +785,7 @@ static int decode_setup(DecodeParams& p, const void* q, const int64_t* q_strides
   p.B = B; p.Hq = Hq; p.Hkv = Hkv; p.G = Hq / Hkv; p.NG = (p.G + 15) / 16;
   p.max_len = max_len;
   p.rows_per_batch = Hkv * p.NG;
+  while ((1 << p.hs) < (p.G < 16 ? p.G : 16)) ++p.hs;
   p.span = dc_span(chunk);
   const int64_t nw = dc_waves(B, Hkv, p.NG, max_len, chunk);
   if (nw / DC_WAVES > 0x7fffffff) return nq_fail(NQ_ERR_INVALID, "chunk %d too small for these sizes", chunk);

@@ -144,3 +144,26 @@ def test_qwen3_235b_decode_full_size():
                           vc[b:b + 1, :, :L].float().cpu(), lens[b:b + 1], q_weight=qw,
                           eps=1e-6, cos=cos, sin=sin, q_pos=lens[b:b + 1].long() - 1)
         assert_bf16_close(o[b:b + 1], ref, f"235B b={b} len={L}")
+
+
+@pytest.mark.parametrize("keys,chunk", [(1, 0), (33, 0), (129, 32), (1500, 0), (5000, 32)])
+@pytest.mark.parametrize("Hq,Hkv", [(2, 2), (3, 1), (8, 2), (16, 1), (32, 1)])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+def test_decode_merge_of_many_partials(dtype, Hq, Hkv, keys, chunk):
+    """Few rows cut into one to ~160 partials: the merge's slices of 1 to 16
+    heads, with fewer partials than slices, as many, and several each."""
+    if dtype == torch.float32 and 128 % (Hq // Hkv):
+        pytest.skip("fp32 takes group sizes that divide 128")
+    say(f"decode merge G={Hq // Hkv} keys={keys} chunk={chunk} {dtype}")
+    for D in (32, 64, 128):
+        lens = torch.tensor([keys], dtype=torch.int32)
+        q = randn(1, Hq, D, seed=91, dtype=dtype)
+        kc = randn(1, Hkv, keys, D, seed=92, dtype=dtype)
+        vc = randn(1, Hkv, keys, D, seed=93, dtype=dtype)
+        qw = 1 + 0.02 * randn(D, seed=94)
+        cos, sin = rope_tables(D, keys, 1e6)
+        o = nq.attention_decode(q.to(DEV), kc.to(DEV), vc.to(DEV), lens.to(DEV), max_len=keys, chunk=chunk,
+                                q_weight=qw.to(DEV), eps=1e-6, cos=cos.to(DEV), sin=sin.to(DEV))
+        ref = decode_path(q.float(), kc.float(), vc.float(), lens, q_weight=qw, eps=1e-6, cos=cos, sin=sin,
+                          q_pos=lens.long() - 1)
+        assert_close_for(dtype, o, ref, f"D={D}")
