@@ -199,6 +199,9 @@ int nq_attn_prefill_paged_fwd(const void* q, const int64_t* q_strides, const voi
  */
 int64_t nq_attn_decode_workspace_bytes(int B, int Hq, int Hkv, int D, int max_len, int chunk);
 
+/* Or'd into the dtype of nq_attn_decode_fwd and nq_attn_decode_paged_fwd. */
+#define NQ_DECODE_F32_SPLIT 0x100
+
 /*
  * Single-token decode attention against a ragged KV cache.
  *
@@ -217,7 +220,10 @@ int64_t nq_attn_decode_workspace_bytes(int B, int Hq, int Hkv, int D, int max_le
  * o: output (B, Hq, D) with strides {batch, head}.
  * workspace: device buffer of at least
  *   nq_attn_decode_workspace_bytes(B, Hq, Hkv, D, max_len, chunk) bytes for
- *   bf16 caches; fp32 caches keep no partials and ignore it (NULL allowed).
+ *   bf16 caches.  fp32 caches ignore it (NULL allowed) and then walk each
+ *   sequence's keys with one workgroup per kv head; with dtype
+ *   NQ_DTYPE_F32 | NQ_DECODE_F32_SPLIT they use it as bf16 caches do, and
+ *   split the keys over the device.
  * Requires Hq / Hkv <= 16 or a multiple of 16.
  */
 int nq_attn_decode_fwd(const void* q, const int64_t* q_strides, const void* k_cache,

@@ -228,8 +228,56 @@ __device__ __forceinline__ int64_t wave_begin(const DecodeParams& p, int64_t N, 
   const int64_t total = split_weight(We);
   return N * DC_ODD_W >= total ? split_weight(w) * N / total : w * N / We;
 }
+
+// A wave's walk over its range of steps, one row segment at a time, for the fp32
+// stream kernel.  (The bf16 one keeps the same walk in its own variables: through
+// this struct it ran 1.2% slower at B64, 64/4 heads, up to 32768 keys.)
+struct Walk {
+  int64_t q, q1;      // the range's next step and its end
+  int b, j, ls, nb;   // batch, row within it, first step within the row, steps of a row
+  int lens_lane;      // lens of up to 64 batch rows, one per lane: no memory round trip at a row boundary
+  bool lens_in_reg;
+
+  __device__ __forceinline__ int len_of(const DecodeParams& p, int bb) const {
+    return lens_in_reg ? __builtin_amdgcn_readlane(lens_lane, bb) : uniform(batch_len(p, bb));
+  }
+  __device__ __forceinline__ int steps_of(const DecodeParams& p, int bb) const {
+    const int l = len_of(p, bb);
+    return l > 0 ? (l + DC_STEP - 1) / DC_STEP : 0;
+  }
+  // false: wave w has no steps
+  __device__ __forceinline__ bool start(const DecodeParams& p, int lane, int64_t w) {
+    const int64_t N = lane_value_i64(total_steps(p, lane), 0);
+    if (N == 0) return false;
+    const int64_t We = waves_used(p, N);
+    if (w >= We) return false;
+    q = wave_begin(p, N, We, w);
+    q1 = wave_begin(p, N, We, w + 1);
+    if (q >= q1) return false;
+    lens_in_reg = p.B <= 64;
+    lens_lane = lens_in_reg && lane < p.B ? batch_len(p, lane) : 0;
+    int64_t before;
+    find_batch(p, lane, q, b, before);
+    nb = steps_of(p, b);
+    j = (int)((q - before) / nb);
+    ls = (int)((q - before) % nb);
+    return true;
+  }
+  // past a segment of nseg steps; false at the end of the range
+  __device__ __forceinline__ bool next(const DecodeParams& p, int nseg) {
+    q += nseg;
+    if (q >= q1) return false;
+    ls = 0;
+    if (++j == p.rows_per_batch) {
+      j = 0;
+      do nb = steps_of(p, ++b); while (nb == 0 && b + 1 < p.B);  // q < q1: a batch with keys follows
+    }
+    return true;
+  }
+};
+
 // ---------------------------------------------------------------- kernels
-// bf16 caches (fp32 caches run the fp32 prefill kernel at S = 1)
+// bf16 caches
 template <int D, typename T, bool PAGED, bool APPEND>
 __global__ void __attribute__((amdgpu_flat_work_group_size(DC_THREADS, DC_THREADS), amdgpu_waves_per_eu(DC_WG_PER_CU)))
 decode_stream_kernel(DecodeParams p) {
@@ -578,6 +626,312 @@ decode_stream_kernel(DecodeParams p) {
   }
 }
 
+// fp32 caches: the same schedule and partials, fp32 arithmetic throughout on
+// v_mfma_f32_16x16x4_f32 (heads on the N side), and no LDS tile: the order in
+// which the MFMA's k index walks the head dims (scores) and its rows the output
+// dims is free, so it is chosen to make each lane's operands 16 consecutive
+// bytes of the cache rows.
+//   S^T = K Q^T: k-slot g of MFMA (u, e) is dim 16u + 4g + e, so lane (key c,
+//     slot g) loads K[c][16u + 4g .. +4]: 64 contiguous bytes per row and load.
+//   O^T += V^T P^T: MFMA i takes key 4g + i in k-slot g, the key of the lane's
+//     own score i; output row r of block (dd, e) is dim 64dd + VW r + e, so the
+//     lane loads V[4g + i][64dd + VW r .. + VW]: whole rows per load.
+// Bound by HBM like the bf16 kernel: the padding to 16 heads costs MFMA work
+// for ~19 TB/s at any D.  K of the next step is loaded once the scores are done
+// with this one's registers, V after the output.  Without a split (one
+// workgroup per kv head, the fp32 prefill kernel at S = 1) B4 8/2 heads D64
+// with 300..2048 keys took 210 us; this takes 10.3 us and the merge 4.8.
+template <int D>
+__device__ __forceinline__ floatx4 mfma16_f32(float a, float b, floatx4 c) {
+  return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0);
+}
+
+template <int D, bool PAGED, bool APPEND>
+__global__ void __attribute__((amdgpu_flat_work_group_size(DC_THREADS, DC_THREADS), amdgpu_waves_per_eu(DC_WG_PER_CU)))
+decode_stream_f32_kernel(DecodeParams p) {
+  constexpr int NU = D / 16;              // 16-byte K pieces per lane and 16 keys
+  constexpr int VW = D >= 64 ? 4 : D / 16;  // V floats per lane and load
+  constexpr int NDD = D / (16 * VW);      // V loads per key
+  constexpr int LPR = D / 16;             // lanes holding one appended row
+  typedef float vpiece __attribute__((ext_vector_type(VW)));
+  __shared__ __attribute__((aligned(16))) float newrow[DC_WAVES][2][D];
+
+  const int lane = threadIdx.x & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int64_t w = (int64_t)blockIdx.x * DC_WAVES + wave;
+  Walk at;
+  if (!at.start(p, lane, w)) return;
+  const int c16 = lane & 15, grp = lane >> 4, sub = lane % LPR;
+  const int krow = (int)(c16 * p.kst * 4) + grp * 16, vrow = (int)(grp * 4 * p.vst * 4) + c16 * VW * 4;
+  const int kst = (int)(p.kst * 4), vst = (int)(p.vst * 4);
+
+  while (true) {
+    const int b = at.b, ls = at.ls, nb = at.nb;
+    const int len = at.len_of(p, b);
+    const int kvh = at.j / p.NG, hg = at.j % p.NG;
+    const int nseg = (int)min((int64_t)(nb - ls), at.q1 - at.q);
+    const bool whole = ls == 0 && nseg == nb;
+    const int kbeg = ls * DC_STEP;
+    const int kend = min(len, (ls + nseg) * DC_STEP);
+    const bool tail = APPEND && kend == len;  // the appended key is this segment's last
+    const int kend_ld = tail ? kend - 1 : kend;
+
+    // block-table entries [wbase, wbase + 64) of this row, one per lane
+    int wbase = 0, win = 0;
+    auto load_window = [&](int first) {
+      const int npg = (kend + p.page - 1) / p.page;
+      wbase = first;
+      win = first + lane < npg ? p.bt[b * p.bts + first + lane] : 0;
+    };
+    if constexpr (PAGED) load_window(kbeg / p.page);
+    const float* kbase = reinterpret_cast<const float*>(p.kc) + kvh * p.ksh;
+    const float* vbase = reinterpret_cast<const float*>(p.vc) + kvh * p.vsh;
+    // the rows of one step: a descriptor that ends after the segment's last
+    // cached key (rows past it read as zeros)
+    BufRsrc krs, vrs;
+    auto step_rows = [&](int k0) {
+      int64_t slab = b, row = k0;
+      if constexpr (PAGED) {  // a step never crosses a page
+        const int pg = k0 / p.page;
+        if (pg - wbase >= 64) load_window(pg);
+        slab = __builtin_amdgcn_readlane(win, pg - wbase);
+        row = k0 - pg * p.page;
+      }
+      const int n = min(kend_ld, k0 + DC_STEP) - k0;
+      krs = make_rsrc(kbase + slab * p.ksb + row * p.kst, n > 0 ? (uint32_t)((n - 1) * kst + D * 4) : 0u);
+      vrs = make_rsrc(vbase + slab * p.vsb + row * p.vst, n > 0 ? (uint32_t)((n - 1) * vst + D * 4) : 0u);
+    };
+    floatx4 kr[2][NU];
+    vpiece vr[2][4][NDD];
+    auto load_k = [&]() {
+#pragma unroll
+      for (int kb = 0; kb < 2; ++kb)
+#pragma unroll
+        for (int u = 0; u < NU; ++u)
+          kr[kb][u] = __builtin_bit_cast(
+              floatx4, __builtin_amdgcn_raw_buffer_load_b128(krs, krow, kb * 16 * kst + u * 64, DC_AUX_NT));
+    };
+    auto load_v = [&]() {
+#pragma unroll
+      for (int kb = 0; kb < 2; ++kb)
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+#pragma unroll
+          for (int dd = 0; dd < NDD; ++dd) {
+            const int so = (kb * 16 + i) * vst + dd * 256;
+            if constexpr (VW == 4)
+              vr[kb][i][dd] = __builtin_bit_cast(vpiece, __builtin_amdgcn_raw_buffer_load_b128(vrs, vrow, so, DC_AUX_NT));
+            else
+              vr[kb][i][dd] = __builtin_bit_cast(vpiece, __builtin_amdgcn_raw_buffer_load_b64(vrs, vrow, so, DC_AUX_NT));
+          }
+    };
+
+    // ---- the query: lane (head c16, slot grp) holds dims 16u + 4grp + e, so
+    // the rotate-half partner of piece u is the lane's piece u + NU/2
+    const int gh = hg * 16 + c16;
+    const bool hvalid = gh < p.G;
+    const float* qrow = reinterpret_cast<const float*>(p.q) + b * p.qsb + (kvh * p.G + (hvalid ? gh : 0)) * p.qsh;
+    floatx4 x[NU], wq[NU], cs[NU / 2], sn[NU / 2];
+#pragma unroll
+    for (int u = 0; u < NU; ++u) x[u] = *reinterpret_cast<const floatx4*>(qrow + u * 16 + grp * 4);
+    if (p.qw) {
+#pragma unroll
+      for (int u = 0; u < NU; ++u) wq[u] = *reinterpret_cast<const floatx4*>(p.qw + u * 16 + grp * 4);
+    }
+    const int pos =
+        p.cos_tab ? table_row(p.q_pos ? ld_uniform(p.q_pos, b) : (p.q_pos0 >= 0 ? p.q_pos0 : len - 1), p.max_pos) : 0;
+    if (p.cos_tab) {
+      const float nan = __builtin_nanf("");
+#pragma unroll
+      for (int u = 0; u < NU / 2; ++u) {
+        const int64_t o = (int64_t)(pos < 0 ? 0 : pos) * (D / 2) + u * 16 + grp * 4;
+        cs[u] = *reinterpret_cast<const floatx4*>(p.cos_tab + o);
+        sn[u] = *reinterpret_cast<const floatx4*>(p.sin_tab + o);
+        if (pos < 0) cs[u] = sn[u] = floatx4{nan, nan, nan, nan};
+      }
+    }
+    // ---- the appended row, in the row kernel's layout and arithmetic: chunks
+    // sub and sub + D/16 per lane
+    floatx8 ka1{}, ka2{}, va1{}, va2{}, kw1{}, kw2{}, kc1{}, ks1{};
+    if (tail) {
+      const float* ks = reinterpret_cast<const float*>(p.kn) + b * p.knsb + kvh * p.knsh + sub * 8;
+      const float* vs = reinterpret_cast<const float*>(p.vn) + b * p.vnsb + kvh * p.vnsh + sub * 8;
+      ka1 = Vec8<float>::load_f32(ks);
+      ka2 = Vec8<float>::load_f32(ks + D / 2);
+      va1 = Vec8<float>::load_f32(vs);
+      va2 = Vec8<float>::load_f32(vs + D / 2);
+      if (p.kw) {
+        kw1 = Vec8<float>::load_f32(p.kw + sub * 8);
+        kw2 = Vec8<float>::load_f32(p.kw + D / 2 + sub * 8);
+      }
+      if (p.cos_tab) {
+        kc1 = load_tab8(p.cos_tab, pos, D / 2, sub * 8);
+        ks1 = load_tab8(p.sin_tab, pos, D / 2, sub * 8);
+      }
+    }
+    step_rows(kbeg);
+    load_k();
+    load_v();
+
+    if (tail) {
+      if (p.kw) norm_row<D>(ka1, ka2, kw1, kw2, p.eps);
+      if (p.cos_tab) rope_row(ka1, ka2, kc1, ks1);
+      if (lane < LPR) {
+        float* nk = newrow[wave][0] + sub * 8;
+        float* nv = newrow[wave][1] + sub * 8;
+        store8<float>(nk, ka1);
+        store8<float>(nk + D / 2, ka2);
+        store8<float>(nv, va1);
+        store8<float>(nv + D / 2, va2);
+        if (hg == 0) {  // one wave per (batch, kv head) writes the row; none of this launch reads it
+          const int t = len - 1;
+          int64_t slab = b, row = t;
+          if constexpr (PAGED) {
+            slab = p.bt[b * p.bts + t / p.page];
+            row = t % p.page;
+          }
+          float* kd = reinterpret_cast<float*>(p.kc) + slab * p.ksb + kvh * p.ksh + row * p.kst + sub * 8;
+          float* vd = reinterpret_cast<float*>(p.vc) + slab * p.vsb + kvh * p.vsh + row * p.vst + sub * 8;
+          store8<float>(kd, ka1);
+          store8<float>(kd + D / 2, ka2);
+          store8<float>(vd, va1);
+          store8<float>(vd + D / 2, va2);
+        }
+      }
+    }
+    if (p.qw) {
+      float ss = 0.f;
+#pragma unroll
+      for (int u = 0; u < NU; ++u)
+#pragma unroll
+        for (int e = 0; e < 4; ++e) ss = __builtin_fmaf(x[u][e], x[u][e], ss);
+      ss += shfl_xor_f(ss, 16);
+      ss += shfl_xor_f(ss, 32);
+      const float r = rsqrtf(ss / (float)D + p.eps);
+#pragma unroll
+      for (int u = 0; u < NU; ++u) x[u] = (x[u] * r) * wq[u];
+    }
+    if (p.cos_tab) {
+#pragma unroll
+      for (int u = 0; u < NU / 2; ++u) {
+        const floatx4 x1 = x[u], x2 = x[u + NU / 2];
+        // fused multiply-adds written out here and below: every instance rounds alike
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+          x[u][e] = __builtin_fmaf(x1[e], cs[u][e], -(x2[e] * sn[u][e]));
+          x[u + NU / 2][e] = __builtin_fmaf(x2[e], cs[u][e], x1[e] * sn[u][e]);
+        }
+      }
+    }
+
+    float m_i = -INFINITY, l_i = 0.f;
+    floatx4 oacc[NDD][VW];
+#pragma unroll
+    for (int dd = 0; dd < NDD; ++dd)
+#pragma unroll
+      for (int e = 0; e < VW; ++e) oacc[dd][e] = floatx4{};
+
+    for (int s = 0; s < nseg; ++s) {
+      const int k0 = kbeg + s * DC_STEP;
+      if (tail && s == nseg - 1) {  // the appended row replaces the zeros loaded for it
+        const int rr = len - 1 - k0;
+#pragma unroll
+        for (int kb = 0; kb < 2; ++kb) {
+          if (kb * 16 + c16 == rr) {
+#pragma unroll
+            for (int u = 0; u < NU; ++u)
+              kr[kb][u] = *reinterpret_cast<const floatx4*>(newrow[wave][0] + u * 16 + grp * 4);
+          }
+#pragma unroll
+          for (int i = 0; i < 4; ++i)
+            if (kb * 16 + grp * 4 + i == rr) {
+#pragma unroll
+              for (int dd = 0; dd < NDD; ++dd)
+                vr[kb][i][dd] = *reinterpret_cast<const vpiece*>(newrow[wave][1] + dd * 64 + c16 * VW);
+            }
+        }
+      }
+      floatx4 sc[2] = {floatx4{}, floatx4{}};
+#pragma unroll
+      for (int u = 0; u < NU; ++u)
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+          sc[0] = mfma16_f32<D>(kr[0][u][e], x[u][e], sc[0]);
+          sc[1] = mfma16_f32<D>(kr[1][u][e], x[u][e], sc[1]);
+        }
+      if (s + 1 < nseg) {
+        step_rows(k0 + DC_STEP);
+        load_k();
+      }
+      if (k0 + DC_STEP > kend) {
+#pragma unroll
+        for (int kb = 0; kb < 2; ++kb)
+#pragma unroll
+          for (int i = 0; i < 4; ++i)
+            if (k0 + kb * 16 + grp * 4 + i >= kend) sc[kb][i] = -INFINITY;
+      }
+      float mx = -INFINITY;
+#pragma unroll
+      for (int kb = 0; kb < 2; ++kb)
+#pragma unroll
+        for (int i = 0; i < 4; ++i) mx = fmaxf(mx, sc[kb][i]);
+      mx = fmaxf(mx, shfl_xor_f(mx, 16));
+      mx = fmaxf(mx, shfl_xor_f(mx, 32));
+      const float m_new = fmaxf(m_i, mx * p.scale_log2);  // finite: a step holds a key below kend
+      const float alpha = fast_exp2(m_i - m_new);
+      float rs = 0.f;
+#pragma unroll
+      for (int kb = 0; kb < 2; ++kb)
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+          sc[kb][i] = fast_exp2(__builtin_fmaf(sc[kb][i], p.scale_log2, -m_new));
+          rs += sc[kb][i];
+        }
+      l_i = __builtin_fmaf(l_i, alpha, rs);
+      m_i = m_new;
+#pragma unroll
+      for (int dd = 0; dd < NDD; ++dd)
+#pragma unroll
+        for (int e = 0; e < VW; ++e) oacc[dd][e] *= alpha;
+#pragma unroll
+      for (int kb = 0; kb < 2; ++kb)
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+#pragma unroll
+          for (int dd = 0; dd < NDD; ++dd)
+#pragma unroll
+            for (int e = 0; e < VW; ++e)
+              oacc[dd][e] = mfma16_f32<D>(vr[kb][i][dd][e], sc[kb][i], oacc[dd][e]);
+      if (s + 1 < nseg) load_v();
+    }
+
+    // ---- flush: lane (head c16), block (dd, e), row 4grp + i = dim 64dd + VW (4grp + i) + e
+    l_i += shfl_xor_f(l_i, 16);
+    l_i += shfl_xor_f(l_i, 32);
+    const int64_t r = ((int64_t)b * p.Hkv + kvh) * p.NG + hg;
+    if (lane == 0) {
+      if (ls == 0) p.ws_rw[r * 2] = (int32_t)w;
+      if (ls + nseg == nb) p.ws_rw[r * 2 + 1] = (int32_t)w;
+    }
+    if (hvalid) {
+      const int64_t slot = w + r;
+      float* out = whole ? reinterpret_cast<float*>(p.o) + b * p.osb + (int64_t)(kvh * p.G + gh) * p.osh
+                         : p.ws_o + (slot * 16 + c16) * D;
+      const float f = whole ? 1.0f / l_i : 1.0f;
+#pragma unroll
+      for (int dd = 0; dd < NDD; ++dd)
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+          vpiece v;
+#pragma unroll
+          for (int e = 0; e < VW; ++e) v[e] = oacc[dd][e][i] * f;
+          *reinterpret_cast<vpiece*>(out + dd * 64 + VW * (grp * 4 + i)) = v;
+        }
+      if (!whole && grp == 0) *reinterpret_cast<floatx2*>(p.ws_ml + (slot * 16 + c16) * 2) = floatx2{m_i, l_i};
+    }
+    if (!at.next(p, nseg)) break;
+  }
+}
 // One workgroup per row (batch, kv head, head group): combines the partials
 // of the waves that covered the row, or writes zeros for a row without keys.
 // 16 threads hold a head (D/16 consecutive dims each); the workgroup's threads
@@ -707,7 +1061,9 @@ static int64_t dc_workspace(int B, int Hq, int Hkv, int D, int max_len, int chun
 
 template <int D, typename T, bool PAGED, bool APPEND>
 static hipError_t launch_decode(DecodeParams p, hipStream_t st) {
-  auto kern = decode_stream_kernel<D, T, PAGED, APPEND>;
+  void (*kern)(DecodeParams);
+  if constexpr (std::is_same<T, float>::value) kern = decode_stream_f32_kernel<D, PAGED, APPEND>;
+  else kern = decode_stream_kernel<D, T, PAGED, APPEND>;
   if (p.span == 0) {
     // persistent grid: as many waves as stay resident at once (<= DC_MAX_WAVES),
     // worked out once per device and kernel variant
@@ -747,9 +1103,14 @@ static hipError_t launch_decode(DecodeParams p, hipStream_t st) {
 static int decode_setup(DecodeParams& p, const void* q, const int64_t* q_strides, const int64_t* k_strides,
                         const int64_t* v_strides, void* o, const int64_t* o_strides, void* workspace,
                         int64_t workspace_bytes, int B, int Hq, int Hkv, int D, int max_len, int chunk,
-                        int dtype, const float* q_weight, float eps, const float* cos_tab,
+                        int& dtype, const float* q_weight, float eps, const float* cos_tab,
                         const float* sin_tab, int max_pos, const int32_t* q_pos, int q_pos0, float sm_scale) {
   if (!head_dim_ok(D)) return nq_fail(NQ_ERR_UNSUPPORTED, "head_dim must be 32, 64 or 128, got %d", D);
+  // partials in the workspace: always for bf16, on request for fp32 (whose
+  // callers otherwise pass none, or one that other calls may be using)
+  const bool f32_split = dtype == (NQ_DTYPE_F32 | NQ_DECODE_F32_SPLIT);
+  if (f32_split) dtype = NQ_DTYPE_F32;
+  const bool partials = dtype == NQ_DTYPE_BF16 || f32_split;
   if (!nq_dtype_ok(dtype)) return nq_fail(NQ_ERR_UNSUPPORTED, "unknown dtype code %d", dtype);
   if (B <= 0 || Hq <= 0 || Hkv <= 0 || max_len <= 0)
     return nq_fail(NQ_ERR_INVALID, "sizes must be positive (B=%d Hq=%d Hkv=%d max_len=%d)", B, Hq, Hkv, max_len);
@@ -769,11 +1130,8 @@ static int decode_setup(DecodeParams& p, const void* q, const int64_t* q_strides
     return nq_fail(NQ_ERR_INVALID, "cos and sin tables go together, with max_pos > 0");
   if (k_strides[2] < D || v_strides[2] < D)
     return nq_fail(NQ_ERR_INVALID, "cache rows must not overlap (seq stride >= head_dim)");
-  // fp32 caches run the fp32 prefill kernel at S = 1, which keeps no partials:
-  // the workspace is neither required nor read there
-  const bool f32 = dtype == NQ_DTYPE_F32;
   const int64_t need = dc_workspace(B, Hq, Hkv, D, max_len, chunk);
-  if (!f32 && (workspace == nullptr || workspace_bytes < need))
+  if (partials && (workspace == nullptr || workspace_bytes < need))
     return nq_fail(NQ_ERR_WORKSPACE, "workspace of %lld bytes required, %lld given", (long long)need,
                    (long long)workspace_bytes);
   p.q = q; p.qsb = q_strides[0]; p.qsh = q_strides[1];
@@ -790,7 +1148,7 @@ static int decode_setup(DecodeParams& p, const void* q, const int64_t* q_strides
   const int64_t nw = dc_waves(B, Hkv, p.NG, max_len, chunk);
   if (nw / DC_WAVES > 0x7fffffff) return nq_fail(NQ_ERR_INVALID, "chunk %d too small for these sizes", chunk);
   p.nwaves = (int)nw;
-  if (!f32) {
+  if (partials) {
     p.ws_o = reinterpret_cast<float*>(workspace);
     p.ws_ml = p.ws_o + (nw + (int64_t)B * p.rows_per_batch) * 16 * D;
     p.ws_rw = reinterpret_cast<int32_t*>(p.ws_ml + (nw + (int64_t)B * p.rows_per_batch) * 16 * 2);
@@ -800,12 +1158,11 @@ static int decode_setup(DecodeParams& p, const void* q, const int64_t* q_strides
   return NQ_OK;
 }
 
-// ---------------------------------------------------------------- fp32 caches
-// An fp32 cache keeps fp32 arithmetic (the reference's SDPA runs in the input
-// dtype): the append, when fused, is its own launch, then the fp32 MFMA
-// attention kernel of the prefill runs with S = 1 over each sequence's keys
-// (its per-sequence lengths and block table), with the same length, position
-// and NaN rules as the bf16 path.  The workspace is not used.
+// ---------------------------------------------------------------- fp32 caches, no workspace
+// Without a workspace an fp32 decode cannot split its keys: the append, when
+// fused, is its own launch, then the fp32 MFMA attention kernel of the prefill
+// runs with S = 1 over each sequence's keys (its per-sequence lengths and block
+// table), with the same length, position and NaN rules.
 
 // The new token's K (QK-Normed with kw, rotated at the query's position) and
 // V to row lens[b] of the paged cache, and lens_out[b] = lens[b] + 1; a
@@ -843,7 +1200,6 @@ __global__ void __launch_bounds__(256) decode_append_f32_kernel(DecodeParams p) 
 }
 
 static int decode_launch_f32(const DecodeParams& d, int D, bool paged, bool append, void* stream) {
-  if (128 % d.G) return nq_fail(NQ_ERR_UNSUPPORTED, "fp32 decode: GQA group size %d must divide 128", d.G);
   hipStream_t st = reinterpret_cast<hipStream_t>(stream);
   if (append) {
     const int64_t threads = (int64_t)d.B * d.Hkv * (D / 16);
@@ -875,8 +1231,17 @@ static int decode_launch_f32(const DecodeParams& d, int D, bool paged, bool appe
 
 template <bool PAGED, bool APPEND>
 static int decode_launch(const DecodeParams& p, int D, int dtype, void* stream) {
-  if (dtype == NQ_DTYPE_F32) return decode_launch_f32(p, D, PAGED, APPEND, stream);
   hipStream_t st = reinterpret_cast<hipStream_t>(stream);
+  if (dtype == NQ_DTYPE_F32) {
+    // the group sizes the form without a split takes, whichever one runs
+    if (128 % p.G) return nq_fail(NQ_ERR_UNSUPPORTED, "fp32 decode: GQA group size %d must divide 128", p.G);
+    // the split addresses a step's 32 rows with 32-bit byte offsets
+    const bool split =
+        p.ws_o && p.kst * 4 * DC_STEP <= 0x7fffffff && p.vst * 4 * DC_STEP <= 0x7fffffff;
+    if (!split) return decode_launch_f32(p, D, PAGED, APPEND, stream);
+    return nq_check_launch(
+        with_head_dim(D, [&](auto dc) { return launch_decode<decltype(dc)::value, float, PAGED, APPEND>(p, st); }));
+  }
   const hipError_t e =
       with_head_dim(D, [&](auto dc) { return launch_decode<decltype(dc)::value, bf16, PAGED, APPEND>(p, st); });
   return nq_check_launch(e);
@@ -1032,7 +1397,7 @@ extern "C" int nq_attn_decode_paged_fwd_noalloc(
   if (!head_dim_ok(D)) return nq_fail(NQ_ERR_UNSUPPORTED, "head_dim must be 32, 64 or 128, got %d", D);
   if (B <= 0 || Hq <= 0 || Hkv <= 0 || max_len <= 0 || Hq % Hkv)
     return nq_fail(NQ_ERR_INVALID, "invalid sizes (B=%d Hq=%d Hkv=%d max_len=%d)", B, Hq, Hkv, max_len);
-  // fp32 caches keep no partials (the workspace is unused), so any size is served
+  // fp32 caches run without a split here (the workspace is unused), so any size is served
   const int64_t need = dtype == NQ_DTYPE_F32 ? 0 : dc_workspace(B, Hq, Hkv, D, max_len, chunk);
   if (need > NQ_DECODE_SCRATCH_BYTES)
     return nq_fail(NQ_ERR_WORKSPACE,

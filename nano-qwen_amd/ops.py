@@ -471,6 +471,19 @@ def decode_workspace_bytes(B: int, Hq: int, Hkv: int, D: int, max_len: int, chun
     return int(_lib.load().nq_attn_decode_workspace_bytes(B, Hq, Hkv, D, max_len, chunk))
 
 
+def _decode_workspace(workspace: Optional[torch.Tensor], dt: int, B: int, Hq: int, Hkv: int, D: int,
+                      max_len: int, chunk: int, dev):
+    """The workspace of a decode's partials (the caller's when it is large enough), and the
+    call's dtype code.  An fp32 decode takes one of its own: its callers may hand the same
+    workspace to calls that overlap, which an fp32 cache never read."""
+    need = decode_workspace_bytes(B, Hq, Hkv, D, max_len, chunk)
+    if dt == _lib.NQ_DTYPE_F32:
+        return torch.empty(max(need, 16), dtype=torch.uint8, device=dev), dt | _lib.NQ_DECODE_F32_SPLIT
+    if workspace is None or workspace.numel() * workspace.element_size() < need:
+        workspace = torch.empty(max(need, 16), dtype=torch.uint8, device=dev)
+    return workspace, dt
+
+
 def attention_decode(q: torch.Tensor, k_cache: torch.Tensor, v_cache: torch.Tensor,
                      lens: Optional[torch.Tensor] = None, *, max_len: int,
                      q_weight: Optional[torch.Tensor] = None, eps: float = 1e-6,
@@ -505,11 +518,8 @@ def attention_decode(q: torch.Tensor, k_cache: torch.Tensor, v_cache: torch.Tens
     if out is None:
         out = torch.empty(B, Hq, D, dtype=q.dtype, device=q.device)
     dev = q.device
-    # fp32 caches keep no partials: the library neither needs nor reads a workspace
-    need = 0 if q.dtype == torch.float32 else decode_workspace_bytes(B, Hq, Hkv, D, max_len, chunk)
-    if need > 0 and (workspace is None or workspace.numel() * workspace.element_size() < need):
-        workspace = torch.empty(need, dtype=torch.uint8, device=dev)
-    wbytes = 0 if workspace is None else workspace.numel() * workspace.element_size()
+    workspace, dt = _decode_workspace(workspace, dt, B, Hq, Hkv, D, max_len, chunk, dev)
+    wbytes = workspace.numel() * workspace.element_size()
     cos_t, sin_t, max_pos = _tables(cos, sin, dev)
     lens_t = _i32(lens, dev)
     qp = _decode_q_pos(q_pos, q_pos0, B, max_pos, dev)
@@ -664,11 +674,8 @@ def attention_decode_paged(q: torch.Tensor, k_pool: torch.Tensor, v_pool: torch.
             raise ValueError("lens_out must not alias lens")
     if out is None:
         out = torch.empty(B, Hq, D, dtype=q.dtype, device=dev)
-    # fp32 caches keep no partials: the library neither needs nor reads a workspace
-    need = 0 if q.dtype == torch.float32 else decode_workspace_bytes(B, Hq, Hkv, D, max_len, chunk)
-    if need > 0 and (workspace is None or workspace.numel() * workspace.element_size() < need):
-        workspace = torch.empty(need, dtype=torch.uint8, device=dev)
-    wbytes = 0 if workspace is None else workspace.numel() * workspace.element_size()
+    workspace, dt = _decode_workspace(workspace, dt, B, Hq, Hkv, D, max_len, chunk, dev)
+    wbytes = workspace.numel() * workspace.element_size()
     cos_t, sin_t, max_pos = _tables(cos, sin, dev)
     qp = _decode_q_pos(q_pos, q_pos0, B, max_pos, dev)
     qw, kw = _f32(q_weight, dev), _f32(k_weight, dev)
