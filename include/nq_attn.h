@@ -191,6 +191,27 @@ int nq_attn_prefill_paged_fwd(const void* q, const int64_t* q_strides, const voi
                               void* stream);
 
 /*
+ * The prefill with a workspace.  A launch with too few query blocks to fill the
+ * device (a short chunk after a long history, a small batch) then splits each
+ * block's keys over several workgroups, whose fp32 partials a second launch
+ * adds (no counterpart in the reference).  nq_attn_prefill_workspace_bytes
+ * gives the bytes needed (16-byte aligned), 0 where the keys are not split: the
+ * workspace is then not used, and NULL is accepted anywhere for no split.
+ * block_table NULL: k and v are dense as in nq_attn_prefill_fwd; else they are
+ * pools as in nq_attn_prefill_paged_fwd.  The other arguments are theirs.
+ */
+int64_t nq_attn_prefill_workspace_bytes(int B, int Hq, int Hkv, int S, int T, int D, int dtype);
+int nq_attn_prefill_ws_fwd(const void* q, const int64_t* q_strides, const void* k,
+                           const int64_t* k_strides, const void* v, const int64_t* v_strides,
+                           const int32_t* block_table, int64_t bt_stride, int page_size, void* o,
+                           const int64_t* o_strides, float* lse, void* workspace,
+                           int64_t workspace_bytes, int B, int Hq, int Hkv, int S, int T, int D,
+                           int dtype, const float* q_weight, float eps, const float* cos_tab,
+                           const float* sin_tab, int max_pos, const int32_t* q_pos,
+                           const int32_t* q_pos_base, int q_pos0, int causal, float sm_scale,
+                           void* stream);
+
+/*
  * Bytes of fp32 workspace nq_attn_decode_fwd needs for these sizes (no
  * counterpart in the reference, whose decode allocates inside torch).
  * max_len bounds every lens[b].  chunk = 0 spreads the cache evenly over a

@@ -70,6 +70,17 @@ SIGNATURES = {
         _p, _p, _i32,                                # q_pos, q_pos_base, q_pos0
         _i32, _f32, _p,                              # causal, sm_scale, stream
     ]),
+    "nq_attn_prefill_workspace_bytes": (_i64, [_i32] * 7),  # B, Hq, Hkv, S, T, D, dtype
+    "nq_attn_prefill_ws_fwd": (_i32, [
+        _p, _i64p, _p, _i64p, _p, _i64p,             # q, k, v (+ strides)
+        _p, _i64, _i32,                              # block_table, bt_stride, page_size
+        _p, _i64p, _p, _p, _i64,                     # o, o_strides, lse, workspace, bytes
+        _i32, _i32, _i32, _i32, _i32, _i32, _i32,    # B, Hq, Hkv, S, T, D, dtype
+        _p, _f32,                                    # q_weight, eps
+        _p, _p, _i32,                                # cos, sin, max_pos
+        _p, _p, _i32,                                # q_pos, q_pos_base, q_pos0
+        _i32, _f32, _p,                              # causal, sm_scale, stream
+    ]),
     "nq_attn_prefill_bias_fwd": (_i32, [
         _p, _i64p, _p, _i64p, _p, _i64p, _p, _i64p,  # q, k, v, o (+ strides)
         _p, _p,                                      # lse, key_lens

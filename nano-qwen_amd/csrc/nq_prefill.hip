@@ -105,6 +105,32 @@ __device__ __forceinline__ int key_perm32(int r) {
   return (r & ~12) | ((r & 4) << 1) | ((r & 8) >> 1);
 }
 
+// ---- split keys.  A query block's tiles [0, ntiles) start at those whose first
+// key every row of the block sees, so that no row of a split is without a
+// finite score; these are dealt to the splits in equal runs, and the tiles
+// after them (the block's diagonal) stay with the last run.
+// The keys [kofs, kend) of split s; false: it has none.
+template <bool CAUSAL>
+__device__ __forceinline__ bool pf_split(const PrefillParams& p, int q0, int s, int& kofs, int& kend) {
+  const int front = q0 + p.T - p.S;  // the first row's last key
+  const int nstart = CAUSAL ? front / PF_BN + 1 : (p.T + PF_BN - 1) / PF_BN;
+  const int run = (nstart + p.nsplit - 1) / p.nsplit;
+  if (s * run >= nstart) return false;
+  kofs = s * run * PF_BN;
+  kend = (s + 1) * run >= nstart ? p.T : (s + 1) * run * PF_BN;
+  return true;
+}
+// Slot of (query block, pair, wave)'s first split in the workspace: per slot
+// NDO x 4 x 64 float4 of O in the accumulators' lane order; after all of them
+// 32 (max, sum) pairs per slot.
+__device__ __forceinline__ int64_t pf_split_slot(const PrefillParams& p, int qblk, int pair, int wave, int nw) {
+  return (((int64_t)qblk * p.B * p.Hkv + pair) * nw + wave) * p.nsplit;
+}
+__device__ __forceinline__ floatx2* pf_split_ml(const PrefillParams& p, int D, int nw) {
+  return reinterpret_cast<floatx2*>(p.ws + (int64_t)p.nqb * p.B * p.Hkv * nw * p.nsplit * (32 * D));
+}
+static int64_t pf_split_bytes(int64_t wgs, int nsplit, int D) { return wgs * 4 * nsplit * (32 * D + 64) * (int64_t)sizeof(float); }
+
 template <int D, int NW>
 struct PfTile {
   static constexpr int ROW_BYTES = D * 2;
@@ -125,7 +151,13 @@ struct PfTile {
 // to every score tile before the row max, so every step takes the masked
 // path; a row may then see no finite score in its first tiles (or in none),
 // which the running max starts from a placeholder for (below).
-template <int D, typename T, bool CAUSAL, bool FUSE_Q, int NW, bool PAGED = false, bool BIAS = false>
+// SPLIT: the key tiles of a query block are dealt to p.nsplit workgroups
+// (pf_split), each of which leaves its unnormalised O, row max and row sum in
+// the workspace for prefill_merge_kernel.  Without it a launch of 128 workgroups
+// (B1, 500 queries on 12345 paged keys, 32/8 heads) ran 277 us on half the CUs;
+// with four runs each and the merge 121 us, 851 TFLOP/s.
+template <int D, typename T, bool CAUSAL, bool FUSE_Q, int NW, bool PAGED = false, bool BIAS = false,
+          bool SPLIT = false>
 __global__ void __attribute__((amdgpu_flat_work_group_size(64 * NW, 64 * NW),
                                amdgpu_waves_per_eu(2, 2)))
 prefill_kernel(PrefillParams p) {
@@ -150,7 +182,12 @@ prefill_kernel(PrefillParams p) {
   const int npairs = p.B * p.Hkv;
   const int L = blockIdx.x;
   int qrank, pair;
-  if (npairs % 8 == 0 && p.nqb >= 128) {
+  int split = 0;
+  if (SPLIT) {
+    pair = L % npairs;
+    split = L / npairs % p.nsplit;
+    qrank = L / (npairs * p.nsplit);
+  } else if (npairs % 8 == 0 && p.nqb >= 128) {
     const int xcd = L & 7, k = L >> 3;
     pair = (k / p.nqb) * 8 + xcd;
     qrank = k % p.nqb;
@@ -161,10 +198,17 @@ prefill_kernel(PrefillParams p) {
   const int qblk = CAUSAL ? (p.nqb - 1 - qrank) : qrank;
   const int b = pair / p.Hkv, kvh = pair % p.Hkv;
   const int q0 = qblk * p.BM;
-  const int coff = p.T - p.S;
+  // SPLIT: keys are counted from this workgroup's first one (kofs)
+  int kofs = 0, coff = p.T - p.S;
   // keys of this sequence (key padding: fewer than T)
-  const int Tk = pf_keys(p, b);
-  if (Tk <= 0) {  // no keys: zeros; a length out of range: NaN
+  int Tk = pf_keys(p, b);
+  if constexpr (SPLIT) {
+    int kend;
+    if (!pf_split<CAUSAL>(p, q0, split, kofs, kend)) return;
+    Tk = kend - kofs;
+    coff -= kofs;
+  }
+  if (!SPLIT && Tk <= 0) {  // no keys: zeros; a length out of range: NaN
     const float f = Tk < 0 ? __builtin_nanf("") : 0.f;
     for (int r = threadIdx.x; r < 32 * NW; r += 64 * NW) {
       const int g = r % p.G, qi = q0 + r / p.G;
@@ -181,9 +225,9 @@ prefill_kernel(PrefillParams p) {
   // K/V are bf16 in memory: they go to LDS unconverted.  A paged pool's base
   // is its kv head's slice of page 0 (pages are added per tile).
   const unsigned char* kbase = reinterpret_cast<const unsigned char*>(
-      reinterpret_cast<const bf16*>(p.k) + (PAGED ? 0 : b * p.ksb) + kvh * p.ksh);
+      reinterpret_cast<const bf16*>(p.k) + (PAGED ? 0 : b * p.ksb + (SPLIT ? kofs * p.kss : 0)) + kvh * p.ksh);
   const unsigned char* vbase = reinterpret_cast<const unsigned char*>(
-      reinterpret_cast<const bf16*>(p.v) + (PAGED ? 0 : b * p.vsb) + kvh * p.vsh);
+      reinterpret_cast<const bf16*>(p.v) + (PAGED ? 0 : b * p.vsb + (SPLIT ? kofs * p.vss : 0)) + kvh * p.vsh);
   const int64_t krow_bytes = p.kss * 2, vrow_bytes = p.vss * 2;
   const int64_t kpage_bytes = p.ksb * 2, vpage_bytes = p.vsb * 2;
 
@@ -207,7 +251,7 @@ prefill_kernel(PrefillParams p) {
       // in page pi1 from row r1 (page % 32 == 0, key0 % 64 == 0); the block
       // table is read through the scalar path, only for rows below Tk
       const int key0 = tile * PF_BN;
-      const int pi0 = key0 / p.page, r0 = key0 - pi0 * p.page;
+      const int pi0 = (kofs + key0) / p.page, r0 = kofs + key0 - pi0 * p.page;
       const bool same = r0 + 32 < p.page;
       const int r1 = same ? r0 + 32 : 0;
       const int64_t btb = (int64_t)b * p.bts;
@@ -693,6 +737,20 @@ prefill_kernel(PrefillParams p) {
   }
 
   l_i = xor32_sum(l_i);
+  if constexpr (SPLIT) {
+    // in the lane order of the accumulators: every store is 1 KiB of the workspace
+    const int64_t grp = pf_split_slot(p, qblk, pair, wave, NW) + split;
+    const int sl = fresh_lane();
+    floatx4* po = reinterpret_cast<floatx4*>(p.ws) + grp * (NDO * 4 * 64) + sl;
+#pragma unroll
+    for (int dd = 0; dd < NDO; ++dd)
+#pragma unroll
+      for (int gq = 0; gq < 4; ++gq)
+        po[(dd * 4 + gq) * 64] = floatx4{oacc[dd][gq * 4 + 0], oacc[dd][gq * 4 + 1], oacc[dd][gq * 4 + 2],
+                                         oacc[dd][gq * 4 + 3]};
+    if (sl < 32) pf_split_ml(p, D, NW)[grp * 32 + sl] = floatx2{m_i, l_i};
+    return;
+  }
   // (BIAS: a row the bias masks entirely has l = 0 and gets zeros, as SDPA gives)
   const float inv_l = (BIAS && !(l_i > 0.f)) ? 0.f : 1.f / l_i;
 
@@ -738,6 +796,72 @@ prefill_kernel(PrefillParams p) {
   }
 }
 
+// Adds the partials of a split prefill: a workgroup takes the 32 rows of one
+// wave, wave dd of it their dims 32dd .. 32dd + 31 in the accumulators' lane
+// order, then the rows go out through LDS as in the kernel's own epilogue.
+// Reads nsplit x fp32 O once: HBM- or L2-bound.
+template <int D, bool CAUSAL>
+__global__ void __launch_bounds__(2 * D) prefill_merge_kernel(PrefillParams p) {
+  constexpr int NDO = D / 32, NW = 4;
+  using Tl = PfTile<D, NW>;
+  __shared__ __attribute__((aligned(16))) unsigned char stage[32 * Tl::ROW_BYTES];
+  const int lane = threadIdx.x & 63, dd = threadIdx.x >> 6;
+  const int r32 = lane & 31, hh = lane >> 5;
+  const int npairs = p.B * p.Hkv;
+  const int wave = blockIdx.x % NW, wg = blockIdx.x / NW;
+  const int qblk = wg / npairs, pair = wg % npairs;
+  const int b = pair / p.Hkv, kvh = pair % p.Hkv;
+  const int q0 = qblk * p.BM;
+  int k0, k1, ns = 1;  // splits that hold keys: the first always does
+  while (ns < p.nsplit && pf_split<CAUSAL>(p, q0, ns, k0, k1)) ++ns;
+  const int64_t grp = pf_split_slot(p, qblk, pair, wave, NW);
+  const floatx2* ml = pf_split_ml(p, D, NW) + grp * 32 + r32;
+  const floatx4* po = reinterpret_cast<const floatx4*>(p.ws) + grp * (NDO * 4 * 64) + dd * 256 + lane;
+  float M = -INFINITY;
+  for (int s = 0; s < ns; ++s) M = fmaxf(M, ml[s * 32][0]);
+  float l = 0.f;
+  floatx4 o[4] = {floatx4{}, floatx4{}, floatx4{}, floatx4{}};
+#pragma unroll 2
+  for (int s = 0; s < ns; ++s) {
+    const floatx2 m_l = ml[s * 32];
+    const float w = fast_exp2(m_l[0] - M);
+    l = __builtin_fmaf(m_l[1], w, l);
+#pragma unroll
+    for (int gq = 0; gq < 4; ++gq) o[gq] += po[(int64_t)s * (NDO * 4 * 64) + gq * 64] * w;
+  }
+  const float inv_l = 1.f / l;
+#pragma unroll
+  for (int gq = 0; gq < 4; ++gq)
+    *reinterpret_cast<bf16x4*>(stage + r32 * Tl::ROW_BYTES + Tl::k_chunk(r32, dd * 4 + gq) * 16 + hh * 8) =
+        __builtin_convertvector(o[gq] * inv_l, bf16x4);
+  __syncthreads();
+  constexpr int OCH = D / 8;
+  for (int i = threadIdx.x; i < 32 * OCH; i += 2 * D) {
+    const int r = i / OCH, c = i % OCH;
+    const int Rw = wave * 32 + r, qr = q0 + Rw / p.G;
+    if (qr < p.S)
+      *reinterpret_cast<bf16x8*>(reinterpret_cast<bf16*>(p.o) + b * p.osb + (kvh * p.G + Rw % p.G) * p.osh +
+                                 (int64_t)qr * p.oss + c * 8) =
+          *reinterpret_cast<const bf16x8*>(stage + r * Tl::ROW_BYTES + Tl::k_chunk(r, c) * 16);
+  }
+  if (p.lse && threadIdx.x < 32) {
+    const int eR = wave * 32 + r32, eq = q0 + eR / p.G;
+    if (eq < p.S) p.lse[((int64_t)b * p.Hq + kvh * p.G + eR % p.G) * p.S + eq] = (M + __log2f(l)) * kLn2;
+  }
+}
+
+template <int D, bool CAUSAL>
+static hipError_t launch_prefill_split(const PrefillParams& p, hipStream_t st) {
+  const int64_t wgs = (int64_t)p.nqb * p.B * p.Hkv;
+  const dim3 grid((unsigned)(wgs * p.nsplit)), block(256);
+  if (p.bt) hipLaunchKernelGGL((prefill_kernel<D, bf16, CAUSAL, true, 4, true, false, true>), grid, block, 0, st, p);
+  else hipLaunchKernelGGL((prefill_kernel<D, bf16, CAUSAL, true, 4, false, false, true>), grid, block, 0, st, p);
+  const hipError_t e = hipGetLastError();
+  if (e != hipSuccess) return e;
+  hipLaunchKernelGGL((prefill_merge_kernel<D, CAUSAL>), dim3((unsigned)(wgs * 4)), dim3(2 * D), 0, st, p);
+  return hipGetLastError();
+}
+
 template <int D, typename T, int NW>
 static hipError_t launch_prefill_nw(const PrefillParams& p, bool causal, bool fuse, hipStream_t st) {
   dim3 grid((unsigned)(p.nqb * p.B * p.Hkv));
@@ -779,6 +903,31 @@ static hipError_t launch_prefill(const PrefillParams& p, int nw, bool causal, bo
 
 using namespace nq;
 
+// 4-wave workgroups of a launch.
+static int64_t prefill_wgs4(int B, int Hq, int Hkv, int S) {
+  const int BM = 128 / (Hq / Hkv);
+  return BM > 0 ? (int64_t)B * Hkv * ((S + BM - 1) / BM) : 0;
+}
+
+// Workgroups per query block that the keys are split over: as many as the
+// device holds, two per CU.  A launch of up to half a workgroup per CU gains
+// from runs of 6 tiles on (B1 32/8 heads D128, 16 queries on 1000 keys: 19.7 ->
+// 17.2 us; 500 on 12345: 180 -> 112), up to 16 of them (16 queries on 12000 keys:
+// 165 us whole, 36 at 15 runs, 46 at 31, whose merge takes longer).  Above that a
+// split only puts a second workgroup on each CU: 2 x 500 queries on 2000 keys,
+// 32/4 heads, 35 tiles in two went 45.8 -> 50.7 us, 250 tiles 327 -> 307.
+constexpr int PF_SPLIT_SLOTS = 512, PF_SPLIT_MAX = 16;
+static int prefill_splits(int B, int Hq, int Hkv, int S, int T) {
+  if (128 % (Hq / Hkv)) return 1;
+  const int64_t wgs = prefill_wgs4(B, Hq, Hkv, S);
+  const int64_t fit = PF_SPLIT_SLOTS / wgs;
+  const int tiles = wgs <= PF_SPLIT_SLOTS / 4 ? 6 : 32;
+  const int64_t most = (T - S / 2) / (PF_BN * tiles);  // T - S/2: a causal row's keys on average
+  int64_t n = fit < most ? fit : most;
+  if (n > PF_SPLIT_MAX) n = PF_SPLIT_MAX;
+  return n > 1 ? (int)n : 1;
+}
+
 // Shared by the dense, paged and bias entry points: bt == NULL for dense K/V,
 // bias == NULL for none.
 static int prefill_entry(const void* q, const int64_t* q_strides, const void* k, const int64_t* k_strides,
@@ -787,7 +936,8 @@ static int prefill_entry(const void* q, const int64_t* q_strides, const void* k,
                          void* o, const int64_t* o_strides, float* lse, const int32_t* key_lens, int B, int Hq,
                          int Hkv, int S, int T, int D, int dtype, const float* q_weight, float eps,
                          const float* cos_tab, const float* sin_tab, int max_pos, const int32_t* q_pos,
-                         const int32_t* q_pos_base, int q_pos0, int causal, float sm_scale, void* stream) {
+                         const int32_t* q_pos_base, int q_pos0, int causal, float sm_scale, void* workspace,
+                         int64_t workspace_bytes, void* stream) {
   // head_dim 256 (kernels/flash_attn.py:106): plain bf16 attention only
   const bool wide = D == 256;
   if (wide && (dtype != NQ_DTYPE_BF16 || q_weight || cos_tab || key_lens || bias || bt))
@@ -867,9 +1017,37 @@ static int prefill_entry(const void* q, const int64_t* q_strides, const void* k,
   const int nw = (128 % G == 0 && (wide_wgs < PF_WIDE_MIN_WGS || D == 32 || bias)) ? 4 : 8;
   p.BM = 32 * nw / G;
   p.nqb = (S + p.BM - 1) / p.BM;
+  p.nsplit = workspace && !key_lens && !bias ? prefill_splits(B, Hq, Hkv, S, T) : 1;
+  if (p.nsplit > 1) {
+    const int64_t need = pf_split_bytes((int64_t)p.nqb * B * Hkv, p.nsplit, D);
+    if (workspace_bytes < need || !nq_aligned16(workspace))
+      return nq_fail(NQ_ERR_WORKSPACE, "workspace of %lld bytes (16-byte aligned) required, %lld given",
+                     (long long)need, (long long)workspace_bytes);
+    p.ws = reinterpret_cast<float*>(workspace);
+    return nq_check_launch(with_head_dim(D, [&](auto dc) {
+      constexpr int DD = decltype(dc)::value;
+      return causal ? launch_prefill_split<DD, true>(p, st) : launch_prefill_split<DD, false>(p, st);
+    }));
+  }
   const hipError_t e =
       with_head_dim(D, [&](auto dc) { return launch_prefill<decltype(dc)::value, bf16>(p, nw, causal, fuse, st); });
   return nq_check_launch(e);
+}
+
+extern "C" int64_t nq_attn_prefill_workspace_bytes(int B, int Hq, int Hkv, int S, int T, int D, int dtype) {
+  if (B <= 0 || Hq <= 0 || Hkv <= 0 || S <= 0 || T <= 0 || Hq % Hkv || !head_dim_ok(D) || dtype != NQ_DTYPE_BF16)
+    return 0;
+  const int ns = prefill_splits(B, Hq, Hkv, S, T);
+  return ns > 1 ? pf_split_bytes(prefill_wgs4(B, Hq, Hkv, S), ns, D) : 0;
+}
+
+static int check_pages(int64_t bt_stride, int page_size, int T) {
+  if (page_size <= 0 || page_size % 32)
+    return nq_fail(NQ_ERR_UNSUPPORTED, "page_size must be a positive multiple of 32, got %d", page_size);
+  if (T > 0 && bt_stride < (T + page_size - 1) / page_size)
+    return nq_fail(NQ_ERR_INVALID, "bt_stride %lld holds fewer than the %d pages of T %d", (long long)bt_stride,
+                   (T + page_size - 1) / page_size, T);
+  return NQ_OK;
 }
 
 extern "C" int nq_attn_prefill_fwd(const void* q, const int64_t* q_strides, const void* k,
@@ -884,7 +1062,26 @@ extern "C" int nq_attn_prefill_fwd(const void* q, const int64_t* q_strides, cons
   nq_clear_error();
   return prefill_entry(q, q_strides, k, k_strides, v, v_strides, nullptr, 0, 0, nullptr, nullptr, o, o_strides, lse,
                        key_lens, B, Hq, Hkv, S, T, D, dtype, q_weight, eps, cos_tab, sin_tab, max_pos, q_pos,
-                       q_pos_base, q_pos0, causal, sm_scale, stream);
+                       q_pos_base, q_pos0, causal, sm_scale, nullptr, 0, stream);
+}
+
+extern "C" int nq_attn_prefill_ws_fwd(const void* q, const int64_t* q_strides, const void* k,
+                                      const int64_t* k_strides, const void* v, const int64_t* v_strides,
+                                      const int32_t* block_table, int64_t bt_stride, int page_size, void* o,
+                                      const int64_t* o_strides, float* lse, void* workspace,
+                                      int64_t workspace_bytes, int B, int Hq, int Hkv, int S, int T, int D,
+                                      int dtype, const float* q_weight, float eps, const float* cos_tab,
+                                      const float* sin_tab, int max_pos, const int32_t* q_pos,
+                                      const int32_t* q_pos_base, int q_pos0, int causal, float sm_scale,
+                                      void* stream) {
+  nq_clear_error();
+  if (block_table) {
+    const int rc = check_pages(bt_stride, page_size, T);
+    if (rc != NQ_OK) return rc;
+  }
+  return prefill_entry(q, q_strides, k, k_strides, v, v_strides, block_table, bt_stride, page_size, nullptr, nullptr,
+                       o, o_strides, lse, nullptr, B, Hq, Hkv, S, T, D, dtype, q_weight, eps, cos_tab, sin_tab,
+                       max_pos, q_pos, q_pos_base, q_pos0, causal, sm_scale, workspace, workspace_bytes, stream);
 }
 
 extern "C" int nq_attn_prefill_bias_fwd(const void* q, const int64_t* q_strides, const void* k,
@@ -899,7 +1096,7 @@ extern "C" int nq_attn_prefill_bias_fwd(const void* q, const int64_t* q_strides,
   if (!bias) return nq_fail(NQ_ERR_INVALID, "nq_attn_prefill_bias_fwd needs the bias");
   return prefill_entry(q, q_strides, k, k_strides, v, v_strides, nullptr, 0, 0, bias, bias_strides, o, o_strides,
                        lse, key_lens, B, Hq, Hkv, S, T, D, dtype, q_weight, eps, cos_tab, sin_tab, max_pos, q_pos,
-                       q_pos_base, q_pos0, causal, sm_scale, stream);
+                       q_pos_base, q_pos0, causal, sm_scale, nullptr, 0, stream);
 }
 
 extern "C" int nq_attn_prefill_paged_fwd(const void* q, const int64_t* q_strides, const void* k_pool,
@@ -913,12 +1110,10 @@ extern "C" int nq_attn_prefill_paged_fwd(const void* q, const int64_t* q_strides
                                          int q_pos0, int causal, float sm_scale, void* stream) {
   nq_clear_error();
   if (!block_table) return nq_fail(NQ_ERR_INVALID, "a paged prefill needs the block table");
-  if (page_size <= 0 || page_size % 32)
-    return nq_fail(NQ_ERR_UNSUPPORTED, "page_size must be a positive multiple of 32, got %d", page_size);
-  if (T > 0 && bt_stride < (T + page_size - 1) / page_size)
-    return nq_fail(NQ_ERR_INVALID, "bt_stride %lld holds fewer than the %d pages of T %d", (long long)bt_stride,
-                   (T + page_size - 1) / page_size, T);
+  const int rc = check_pages(bt_stride, page_size, T);
+  if (rc != NQ_OK) return rc;
   return prefill_entry(q, q_strides, k_pool, k_pool_strides, v_pool, v_pool_strides, block_table, bt_stride,
                        page_size, nullptr, nullptr, o, o_strides, lse, nullptr, B, Hq, Hkv, S, T, D, dtype, q_weight,
-                       eps, cos_tab, sin_tab, max_pos, q_pos, q_pos_base, q_pos0, causal, sm_scale, stream);
+                       eps, cos_tab, sin_tab, max_pos, q_pos, q_pos_base, q_pos0, causal, sm_scale, nullptr, 0,
+                       stream);
 }

@@ -45,6 +45,10 @@ struct PrefillParams {
   // contiguous and readable up to T rounded up to a multiple of 8
   const void* bias;
   int64_t bsb, bsh, bss;
+  // keys split over nsplit workgroups per query block (bf16 form; 1 = none),
+  // whose partials go to ws
+  int nsplit;
+  float* ws;
 };
 
 // Keys of sequence b (-1: a length out of range).

@@ -374,10 +374,22 @@ def attention_prefill(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, *,
         call = KernelCall(_lib.load().nq_attn_prefill_bias_fwd, args, len(args) - 1, "nq_attn_prefill_bias_fwd",
                           keep + (bias.bias,), (out, lse) if return_lse else out)
     else:
-        args = head + tail
-        call = KernelCall(_lib.load().nq_attn_prefill_fwd, args, len(args) - 1, "nq_attn_prefill_fwd",
-                          keep, (out, lse) if return_lse else out)
+        ws = _prefill_workspace(B, Hq, Hkv, S, T, D, dt, dev) if kl is None else None
+        if ws is not None:
+            args = head[:6] + (None, 0, 0) + head[6:9] + (_ptr(ws), ws.numel()) + tail
+            call = KernelCall(_lib.load().nq_attn_prefill_ws_fwd, args, len(args) - 1, "nq_attn_prefill_ws_fwd",
+                              keep + (ws,), (out, lse) if return_lse else out)
+        else:
+            args = head + tail
+            call = KernelCall(_lib.load().nq_attn_prefill_fwd, args, len(args) - 1, "nq_attn_prefill_fwd",
+                              keep, (out, lse) if return_lse else out)
     return call if plan else call.launch()
+
+
+def _prefill_workspace(B, Hq, Hkv, S, T, D, dt, dev) -> Optional[torch.Tensor]:
+    """The workspace of a prefill whose keys are split over the device; None when they are not."""
+    need = int(_lib.load().nq_attn_prefill_workspace_bytes(B, Hq, Hkv, S, T, D, dt))
+    return torch.empty(need, dtype=torch.uint8, device=dev) if need > 0 else None
 
 
 def _check_bias(bias: AttnBias, B: int, Hq: int, S: int, T: int, dtype: torch.dtype, transpose: bool = False):
@@ -435,14 +447,17 @@ def attention_prefill_paged(q: torch.Tensor, k_pool: torch.Tensor, v_pool: torch
     pb = _i32(pos_base, dev)
     qw = _f32(q_weight, dev)
     st = _lib.strides3
+    ws = _prefill_workspace(B, Hq, Hkv, S, int(T), D, dt, dev)
+    name = "nq_attn_prefill_paged_fwd" if ws is None else "nq_attn_prefill_ws_fwd"
     args = (
         _ptr(q), st(q.stride()[:3]), _ptr(k_pool), st(k_pool.stride()[:3]), _ptr(v_pool),
         st(v_pool.stride()[:3]), _ptr(bt), bt.stride(0), P, _ptr(out), st(out.stride()[:3]), _ptr(lse),
+        *(() if ws is None else (_ptr(ws), ws.numel())),
         B, Hq, Hkv, S, int(T), D, dt, _ptr(qw), float(eps), _ptr(cos_t), _ptr(sin_t), max_pos,
         _ptr(pos), _ptr(pb), int(pos_offset), int(bool(causal)),
         float(sm_scale) if sm_scale is not None else 0.0, _stream(q))
-    call = KernelCall(_lib.load().nq_attn_prefill_paged_fwd, args, len(args) - 1, "nq_attn_prefill_paged_fwd",
-                      (q, k_pool, v_pool, bt, cos_t, sin_t, pos, pb, qw), (out, lse) if return_lse else out)
+    call = KernelCall(getattr(_lib.load(), name), args, len(args) - 1, name,
+                      (q, k_pool, v_pool, bt, cos_t, sin_t, pos, pb, qw, ws), (out, lse) if return_lse else out)
     return call if plan else call.launch()
 
 

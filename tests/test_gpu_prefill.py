@@ -4,6 +4,7 @@ import pytest
 import torch
 
 import nano_qwen_amd as nq
+from nano_qwen_amd import ops
 from oracle import attention, attention_path, rms_norm, rope_tables, rotate_half
 from tests.helpers import assert_bf16_close, assert_close_for, assert_fp32_close, randn, say
 
@@ -353,3 +354,48 @@ def test_staged_tables_match_per_token_positions_at_8_waves():
     o_ids5, _ = nq.attention_prefill(q, k, v, position_ids=torch.arange(S, device=DEV)[None, :].expand(B, S) + 5,
                                      **kw)
     assert torch.equal(o_off, o_ids5), f"max |diff| {(o_off.float() - o_ids5.float()).abs().max().item():.3e}"
+
+
+@pytest.mark.parametrize("paged", [False, True])
+@pytest.mark.parametrize("causal", [True, False])
+@pytest.mark.parametrize("Hq,Hkv,D,S,T", [
+    (8, 2, 128, 1, 1599),      # one query row, two runs
+    (8, 2, 128, 33, 1600),     # a block's diagonal inside one tile
+    (8, 2, 64, 500, 5003),     # several query blocks, the last one short
+    (2, 2, 128, 129, 1664),    # 128 positions a block: the diagonal spans three tiles
+    (32, 1, 32, 70, 12345),    # 4 positions a block, many runs
+    (4, 2, 128, 3100, 3100),   # a whole prompt: the first blocks have fewer tiles than runs
+])
+def test_split_keys_prefill(Hq, Hkv, D, S, T, causal, paged):
+    """Launches with few query blocks split their keys; every other row of the pages is NaN."""
+    say(f"split prefill Hq={Hq} Hkv={Hkv} D={D} S={S} T={T} causal={causal} paged={paged}")
+    assert ops._lib.load().nq_attn_prefill_workspace_bytes(1, Hq, Hkv, S, T, D, 0) > 0
+    q = randn(1, Hq, S, D, seed=401, dtype=torch.bfloat16)
+    k = randn(1, Hkv, T, D, seed=402, dtype=torch.bfloat16)
+    v = randn(1, Hkv, T, D, seed=403, dtype=torch.bfloat16)
+    w = 1 + 0.02 * randn(D, seed=404)
+    cos, sin = rope_tables(D, T, 1e6)
+    args = dict(q_weight=w.to(DEV), eps=1e-6, cos=cos.to(DEV), sin=sin.to(DEV), pos_offset=T - S, causal=causal,
+                return_lse=True)
+    if paged:
+        P = 96
+        n = -(-T // P)
+        kp, vp = (torch.full((n + 1, Hkv, P, D), float("nan"), dtype=torch.bfloat16, device=DEV) for _ in range(2))
+        bt = torch.randperm(n + 1, generator=torch.Generator().manual_seed(405))[:n].to(torch.int32)
+        for src, pool in ((k, kp), (v, vp)):
+            for i in range(n):
+                rows = src[0, :, i * P:(i + 1) * P].to(DEV)
+                pool[int(bt[i]), :, :rows.shape[1]] = rows
+        o, lse = ops.attention_prefill_paged(q.to(DEV), kp, vp, bt.view(1, n).to(DEV), T=T, **args)
+    else:
+        o, lse = ops.attention_prefill(q.to(DEV), k.to(DEV), v.to(DEV), **args)
+    qh = rotate_half(rms_norm(q.double(), w.double(), 1e-6, compute_dtype=torch.float64),
+                     cos.double()[T - S:], sin.double()[T - S:])
+    sc = qh.view(1, Hkv, -1, S, D) @ k.double()[:, :, None].transpose(-1, -2) / D ** 0.5
+    if causal:
+        sc = sc.masked_fill(torch.arange(T) > torch.arange(S)[:, None] + T - S, float("-inf"))
+    ref = (torch.softmax(sc, -1) @ v.double()[:, :, None]).view(1, Hq, S, D)
+    assert_bf16_close(o, ref, "split o")
+    # scores carry Q-hat's bf16 rounding: 2^-9 relative over D products of unit
+    # variance, so a row's LSE moves by a few 2^-9 at most
+    torch.testing.assert_close(lse.cpu().double(), torch.logsumexp(sc, -1).view(1, Hq, S), rtol=0, atol=2e-2)
