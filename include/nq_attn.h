@@ -366,6 +366,15 @@ int nq_attn_merge(void* o, const int64_t* o_strides, float* lse, const void* o_p
  * and read by its second.
  */
 int64_t nq_attn_bwd_workspace_bytes(int B, int Hq, int S);
+/*
+ * Bytes with which nq_attn_bwd also splits the work of dK/dV: a key block's
+ * query rows over several workgroups, whose fp32 partial sums a further launch
+ * adds in a fixed order.  At least nq_attn_bwd_workspace_bytes, and equal to it
+ * where nothing is gained (long key ranges that fill the device evenly).  With
+ * a smaller workspace (or one that is not 16-byte aligned) nothing is split.
+ */
+int64_t nq_attn_bwd_split_workspace_bytes(int B, int Hq, int Hkv, int S, int T, int D, int dtype,
+                                          int causal);
 
 /*
  * Attention backward (FlashAttention-2 with the forward's LSE): the gradient

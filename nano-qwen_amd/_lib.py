@@ -143,6 +143,7 @@ SIGNATURES = {
         _i32, _i32, _i32, _i32, _i32,                # B, H, S, D, dtype
         _p,                                          # stream
     ]),
+    "nq_attn_bwd_split_workspace_bytes": (_i64, [_i32] * 8),  # B, Hq, Hkv, S, T, D, dtype, causal
     "nq_attn_bwd_workspace_bytes": (_i64, [_i32, _i32, _i32]),
     "nq_attn_bwd": (_i32, [
         _p, _i64p, _p, _i64p, _p, _i64p,             # q, k, v (+ strides)

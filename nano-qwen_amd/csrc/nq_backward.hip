@@ -43,7 +43,7 @@ namespace nq {
 
 constexpr int BW_BN = 64;     // keys per tile (dQ kernel)
 constexpr int BW_BQ = 32;     // query rows per tile (dK/dV kernel)
-constexpr int BW_KEYS = 128;  // keys per dK/dV workgroup (32 per wave)
+constexpr int BW_KEYS = BW_SPLIT_KEYS;  // keys per dK/dV workgroup (32 per wave)
 constexpr int64_t BW_DQ_WIDE_MIN_WGS = 2048;  // 8-wave dQ workgroups needed to prefer them
 constexpr int BW_XCD_MIN_BLOCKS = 64;  // blocks per pair from which each XCD takes whole pairs
 
@@ -352,8 +352,9 @@ __global__ void __launch_bounds__(64 * NW, 8 / NW) bwd_dq_kernel(BwdParams p) {
 }
 
 // ---------------------------------------------------------------- dK, dV
-// D = 64 fits three workgroups per CU (168 VGPRs), D = 128 two
-template <int D, typename T, bool CAUSAL, bool BIAS = false>
+// D = 64 fits three workgroups per CU (168 VGPRs), D = 128 two.
+// SPLIT: the steps of a key block in up to p.nsplit runs (nq_backward.hpp).
+template <int D, typename T, bool CAUSAL, bool BIAS = false, bool SPLIT = false>
 __global__ void __launch_bounds__(256, D == 64 ? 3 : 2) bwd_dkdv_kernel(BwdParams p) {
   using L = BwTile<D>;
   constexpr int NDB = D / 16, NDO = D / 32;
@@ -376,9 +377,13 @@ __global__ void __launch_bounds__(256, D == 64 ? 3 : 2) bwd_dkdv_kernel(BwdParam
   // first; with a pair count that is a multiple of 8 a pair's blocks still
   // land on one XCD.
   const int npairs = p.B * p.Hkv;
-  int kblk, pair;
+  int kblk, pair, split = 0;
   const int nkb = gridDim.x / npairs;
-  if (npairs % 8 == 0 && nkb >= BW_XCD_MIN_BLOCKS) {
+  if (SPLIT) {
+    pair = blockIdx.x % npairs;
+    split = blockIdx.x / npairs % p.nsplit;
+    kblk = blockIdx.x / (npairs * p.nsplit);
+  } else if (npairs % 8 == 0 && nkb >= BW_XCD_MIN_BLOCKS) {
     const int x = blockIdx.x & 7, k = blockIdx.x >> 3;
     pair = (k / nkb) * 8 + x;
     kblk = k % nkb;
@@ -394,9 +399,13 @@ __global__ void __launch_bounds__(256, D == 64 ? 3 : 2) bwd_dkdv_kernel(BwdParam
 
   // the work list: (query tile qt, head g) for queries that see a key of this
   // block (q + coff >= k0); none when the whole block is padding
-  const int qstart = CAUSAL ? max(0, k0 - p.coff) / BW_BQ * BW_BQ : 0;
-  const int nqt = (qstart < p.S && k0 < Tk) ? (p.S - qstart + BW_BQ - 1) / BW_BQ : 0;
-  const int niter = p.G * nqt;
+  const int qstart = bw_first_query(p, CAUSAL, k0, BW_BQ);
+  const int steps = bw_steps(p, CAUSAL, b, k0);
+  const int nqt = steps / p.G;
+  const int runs = SPLIT ? bw_runs(p, steps) : 1;
+  if (SPLIT && split >= runs) return;
+  const int it0 = split * p.run;  // this run's first step
+  const int niter = SPLIT ? min(p.run, steps - it0) : steps;
   // bf16 Q / dO tiles: this wave's DMA instruction i fills LDS bytes
   // [(wave + 4i) * 1024, +1024), the lane's 16 bytes lying in tile row
   // dr0 + i * DSTEP at the same swizzled chunk for every i (the swizzle
@@ -447,8 +456,10 @@ __global__ void __launch_bounds__(256, D == 64 ? 3 : 2) bwd_dkdv_kernel(BwdParam
       qt -= BW_BQ;
     }
   };
-  const int qtop = qstart + (nqt - 1) * BW_BQ;  // the last query tile
-  int gn = 0, qtn = qtop;  // the next step to stage
+  // the first step's tile (the last one of the block) and head
+  const int qtop = qstart + (nqt - 1 - (SPLIT ? it0 / p.G : 0)) * BW_BQ;
+  const int gtop = SPLIT ? it0 % p.G : 0;
+  int gn = gtop, qtn = qtop;  // the next step to stage
   // V of the block's keys stays in LDS (read as the B operand of dP each
   // step); K of the lane's key is held in registers (B operand of S).  Both
   // stagings are waited for at the top of the first iteration (a workgroup
@@ -491,7 +502,7 @@ __global__ void __launch_bounds__(256, D == 64 ? 3 : 2) bwd_dkdv_kernel(BwdParam
 #pragma unroll
   for (int dd = 0; dd < NDO; ++dd) dkacc[dd] = dvacc[dd] = floatx16{};
 
-  int gcur = 0, qnext = qtop;
+  int gcur = gtop, qnext = qtop;
   for (int it = 0; it < niter; ++it) {
     const int qt = qnext;  // this step's query tile
     const int gstep = gcur;  // and head
@@ -607,9 +618,15 @@ __global__ void __launch_bounds__(256, D == 64 ? 3 : 2) bwd_dkdv_kernel(BwdParam
     }
   }
 
-  if (key >= p.T) return;
-  T* dko = reinterpret_cast<T*>(p.dk) + b * p.dksb + kvh * p.dksh + (int64_t)key * p.dkss;
-  T* dvo = reinterpret_cast<T*>(p.dv) + b * p.dvsb + kvh * p.dvsh + (int64_t)key * p.dvss;
+  if (SPLIT && runs > 1) {
+    bw_store_part<D>(p, kblk, pair, split, wave, fresh_lane(), dkacc, dvacc);
+    return;
+  }
+  const int el = fresh_lane(), ehh = el >> 5;  // no lane value held through the loop: it would spill
+  const int ekey = k0 + wave * 32 + (el & 31);
+  if (ekey >= p.T) return;
+  T* dko = reinterpret_cast<T*>(p.dk) + b * p.dksb + kvh * p.dksh + (int64_t)ekey * p.dkss;
+  T* dvo = reinterpret_cast<T*>(p.dv) + b * p.dvsb + kvh * p.dvsh + (int64_t)ekey * p.dvss;
 #pragma unroll
   for (int dd = 0; dd < NDO; ++dd)
 #pragma unroll
@@ -617,8 +634,8 @@ __global__ void __launch_bounds__(256, D == 64 ? 3 : 2) bwd_dkdv_kernel(BwdParam
       floatx4 tk = {dkacc[dd][gq * 4] * p.scale, dkacc[dd][gq * 4 + 1] * p.scale, dkacc[dd][gq * 4 + 2] * p.scale,
                     dkacc[dd][gq * 4 + 3] * p.scale};
       floatx4 tv = {dvacc[dd][gq * 4], dvacc[dd][gq * 4 + 1], dvacc[dd][gq * 4 + 2], dvacc[dd][gq * 4 + 3]};
-      store4<T>(dko + dd * 32 + gq * 8 + hh * 4, tk);
-      store4<T>(dvo + dd * 32 + gq * 8 + hh * 4, tv);
+      store4<T>(dko + dd * 32 + gq * 8 + ehh * 4, tk);
+      store4<T>(dvo + dd * 32 + gq * 8 + ehh * 4, tv);
     }
 }
 
@@ -638,16 +655,20 @@ static hipError_t launch_bwd(const BwdParams& p, int nw, bool causal, hipStream_
     }
     return hipGetLastError();
   }
+  const dim3 gs(gk.x * p.nsplit);
   if (causal) {
     if (nw == 8) hipLaunchKernelGGL((bwd_dq_kernel<D, T, true, 8>), gq, bq, 0, st, p);
     else hipLaunchKernelGGL((bwd_dq_kernel<D, T, true, 4>), gq, bq, 0, st, p);
-    hipLaunchKernelGGL((bwd_dkdv_kernel<D, T, true>), gk, dim3(256), 0, st, p);
+    if (p.nsplit > 1) hipLaunchKernelGGL((bwd_dkdv_kernel<D, T, true, false, true>), gs, dim3(256), 0, st, p);
+    else hipLaunchKernelGGL((bwd_dkdv_kernel<D, T, true>), gk, dim3(256), 0, st, p);
   } else {
     if (nw == 8) hipLaunchKernelGGL((bwd_dq_kernel<D, T, false, 8>), gq, bq, 0, st, p);
     else hipLaunchKernelGGL((bwd_dq_kernel<D, T, false, 4>), gq, bq, 0, st, p);
-    hipLaunchKernelGGL((bwd_dkdv_kernel<D, T, false>), gk, dim3(256), 0, st, p);
+    if (p.nsplit > 1) hipLaunchKernelGGL((bwd_dkdv_kernel<D, T, false, false, true>), gs, dim3(256), 0, st, p);
+    else hipLaunchKernelGGL((bwd_dkdv_kernel<D, T, false>), gk, dim3(256), 0, st, p);
   }
-  return hipGetLastError();
+  const hipError_t e = hipGetLastError();
+  return e == hipSuccess && p.nsplit > 1 ? launch_dkdv_merge<D, T>(p, causal, st) : e;
 }
 
 // ---------------------------------------------------------------- QK-Norm + RoPE backward
@@ -779,6 +800,41 @@ extern "C" int64_t nq_attn_bwd_workspace_bytes(int B, int Hq, int S) {
   return (int64_t)B * Hq * ((S + 31) / 32) * 64 * (int64_t)sizeof(float);
 }
 
+// How dK/dV splits the key blocks' steps when there are fewer blocks than CUs:
+// runs of the length that gives every resident workgroup the same work (at least
+// DKDV_MIN_RUN steps, ~25 us), where some block is longer than that.  fp32 B2
+// S1000 8/2 heads D64, 32 blocks of up to 128 steps: 666 us whole, 93 + 6 for the
+// merge in runs of 16.  From a block per CU on the sums keep the query order, so
+// that a sequence's gradients do not depend on the batch it is in.
+struct DkdvSplit { int nsplit, run; };
+constexpr int DKDV_MIN_RUN = 16;
+static DkdvSplit dkdv_split(int B, int Hq, int Hkv, int S, int T, int D, int dtype, bool causal) {
+  const int G = Hq / Hkv, nkb = (T + BW_KEYS - 1) / BW_KEYS;
+  int64_t total = 0, most = 0;
+  for (int i = 0; i < nkb; ++i) {
+    const int lo = i * BW_KEYS - (T - S), q = causal && lo > 0 ? lo / BW_BQ * BW_BQ : 0;
+    const int64_t steps = q < S ? (int64_t)G * ((S - q + BW_BQ - 1) / BW_BQ) : 0;
+    total += steps;
+    if (steps > most) most = steps;
+  }
+  // resident workgroups: 256 CUs x (bf16 D = 64: 3, else 2; fp32: 1)
+  const int slots = 256 * (dtype == NQ_DTYPE_F32 ? 1 : (D == 64 ? 3 : 2));
+  const int64_t even = (total * B * Hkv + slots - 1) / slots;
+  const int64_t run = even > DKDV_MIN_RUN ? even : DKDV_MIN_RUN;
+  if ((int64_t)nkb * B * Hkv >= 256 || run >= most || most > 0x7fffffff) return {1, 1};
+  return {(int)((most + run - 1) / run), (int)run};
+}
+
+extern "C" int64_t nq_attn_bwd_split_workspace_bytes(int B, int Hq, int Hkv, int S, int T, int D, int dtype,
+                                                     int causal) {
+  const int64_t base = nq_attn_bwd_workspace_bytes(B, Hq, S);
+  if (base == 0 || Hkv <= 0 || T <= 0 || Hq % Hkv || !head_dim_ok(D) || !nq_dtype_ok(dtype)) return base;
+  const DkdvSplit sp = dkdv_split(B, Hq, Hkv, S, T, D, dtype, causal != 0);
+  if (sp.nsplit == 1) return base;
+  const int64_t nkb = (T + BW_KEYS - 1) / BW_KEYS;
+  return base + nkb * B * Hkv * sp.nsplit * (BW_KEYS * 2 * (int64_t)D * (int64_t)sizeof(float));
+}
+
 // Shared by nq_attn_bwd and nq_attn_bwd_bias (bias == NULL: none).
 static int bwd_entry(const void* q, const int64_t* q_strides, const void* k, const int64_t* k_strides,
                      const void* v, const int64_t* v_strides, const void* o, const int64_t* o_strides,
@@ -867,6 +923,16 @@ static int bwd_entry(const void* q, const int64_t* q_strides, const void* k, con
   p.scale = sm_scale > 0.f ? sm_scale : 1.0f / sqrtf((float)D);
   p.scale_log2 = p.scale * kLog2e;
   hipStream_t st = reinterpret_cast<hipStream_t>(stream);
+  p.nsplit = p.run = 1;
+  if (!wide && !bias && nq_aligned16(workspace) &&
+      workspace_bytes >= nq_attn_bwd_split_workspace_bytes(B, Hq, Hkv, S, T, D, dtype, causal)) {
+    const DkdvSplit sp = dkdv_split(B, Hq, Hkv, S, T, D, dtype, causal != 0);
+    if ((int64_t)((T + BW_KEYS - 1) / BW_KEYS) * B * Hkv * sp.nsplit < (1LL << 29)) {
+      p.nsplit = sp.nsplit;
+      p.run = sp.run;
+      p.part = p.ws + need / (int64_t)sizeof(float);  // need is a multiple of 256
+    }
+  }
   if (wide) {
     p.nqb = (S + 63) / 64;
     if ((int64_t)p.nqb * B * Hq >= (1LL << 31) || (int64_t)((T + 63) / 64) * B * Hkv >= (1LL << 31))

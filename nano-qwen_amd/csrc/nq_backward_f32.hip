@@ -215,7 +215,8 @@ __global__ void __launch_bounds__(64 * BF32_NW) bwd_dq_f32_kernel(BwdParams p) {
 }
 
 // ---------------------------------------------------------------------------
-template <int D, bool CAUSAL, bool BIAS = false>
+// SPLIT: the steps of a key block in up to p.nsplit runs (nq_backward.hpp).
+template <int D, bool CAUSAL, bool BIAS = false, bool SPLIT = false>
 __global__ void __launch_bounds__(64 * BF32_NW) bwd_dkdv_f32_kernel(BwdParams p) {
   using L = BwF32<D>;
   constexpr int NT = D / 2, NDO = D / 32;
@@ -227,7 +228,9 @@ __global__ void __launch_bounds__(64 * BF32_NW) bwd_dkdv_f32_kernel(BwdParams p)
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   const int r32 = lane & 31, hh = lane >> 5;
   const int npairs = p.B * p.Hkv;
-  const int pair = blockIdx.x % npairs, kblk = blockIdx.x / npairs;  // lowest keys (most work) first
+  const int pair = blockIdx.x % npairs;
+  const int split = SPLIT ? blockIdx.x / npairs % p.nsplit : 0;
+  const int kblk = blockIdx.x / (npairs * (SPLIT ? p.nsplit : 1));  // lowest keys (most work) first
   const int b = pair / p.Hkv, kvh = pair % p.Hkv;
   const int k0 = kblk * KEYS;
   const int key = k0 + wave * 32 + r32;  // this lane's key column
@@ -257,16 +260,31 @@ __global__ void __launch_bounds__(64 * BF32_NW) bwd_dkdv_f32_kernel(BwdParams p)
 #pragma unroll
   for (int dd = 0; dd < NDO; ++dd) dkacc[dd] = dvacc[dd] = floatx16{};
 
-  // query rows that see any of this workgroup's keys: s + coff >= k0
-  const int sbeg = CAUSAL ? max(0, k0 - p.coff) / BF32_TILE * BF32_TILE : 0;
+  // the work list: query tiles that see any of this workgroup's keys (s + coff
+  // >= k0), head by head; a wave without attended keys still stages them
+  const int sbeg = bw_first_query(p, CAUSAL, k0, BF32_TILE);
+  const int steps = bw_steps(p, CAUSAL, b, k0);
+  const int nqt = steps / p.G;
+  const int runs = SPLIT ? bw_runs(p, steps) : 1;
+  if (SPLIT && split >= runs) return;
+  const int it0 = split * p.run;
+  const int niter = SPLIT ? min(p.run, steps - it0) : steps;
   TileCopy<D> qc, dc;
-  for (int g = 0; g < p.G; ++g) {
+  int g = SPLIT && nqt ? it0 / nqt : 0, s0 = sbeg + (SPLIT && nqt ? it0 % nqt * BF32_TILE : 0);
+  auto fetch = [&](int gf, int sf) {
+    const int head = kvh * p.G + gf;
+    qc.fetch(reinterpret_cast<const float*>(p.q) + b * p.qsb + head * p.qsh, p.qss, sf, p.S);
+    dc.fetch(reinterpret_cast<const float*>(p.dout) + b * p.dosb + head * p.dosh, p.doss, sf, p.S);
+  };
+  if (niter > 0) fetch(g, s0);
+  for (int it = 0; it < niter; ++it) {
     const int head = kvh * p.G + g;
-    const float* qbase = reinterpret_cast<const float*>(p.q) + b * p.qsb + head * p.qsh;
-    const float* dbase = reinterpret_cast<const float*>(p.dout) + b * p.dosb + head * p.dosh;
-    for (int s0 = sbeg; s0 < p.S; s0 += BF32_TILE) {
-      qc.fetch(qbase, p.qss, s0, p.S);
-      dc.fetch(dbase, p.doss, s0, p.S);
+    int gn = g, sn = s0 + BF32_TILE;  // the next step
+    if (sn >= p.S) {
+      sn = sbeg;
+      ++gn;
+    }
+    {
       __syncthreads();  // every wave is done with the previous tile
       qc.stash(qt);
       dc.stash(dot);
@@ -277,6 +295,7 @@ __global__ void __launch_bounds__(64 * BF32_NW) bwd_dkdv_f32_kernel(BwdParams p)
         dlts[threadIdx.x] = s < p.S ? p.ws[wi + 32] : 0.f;
       }
       __syncthreads();
+      if (it + 1 < niter) fetch(gn, sn);  // lands under this step's products
       // S = Q K^T and dP = dO V^T (MFMA row = query row r32 of the tile)
       floatx16 s = floatx16{}, dp = floatx16{};
 #pragma unroll
@@ -323,6 +342,12 @@ __global__ void __launch_bounds__(64 * BF32_NW) bwd_dkdv_f32_kernel(BwdParams p)
         }
       }
     }
+    g = gn;
+    s0 = sn;
+  }
+  if (SPLIT && runs > 1) {
+    bw_store_part<D>(p, kblk, pair, split, wave, lane, dkacc, dvacc);
+    return;
   }
   if (!kvalid) return;
   float* dkrow = reinterpret_cast<float*>(p.dk) + b * p.dksb + kvh * p.dksh + (int64_t)key * p.dkss;
@@ -355,14 +380,18 @@ static hipError_t launch_f32(const BwdParams& p, bool causal, hipStream_t st) {
     }
     return hipGetLastError();
   }
+  const dim3 gs(gk.x * p.nsplit);
   if (causal) {
     hipLaunchKernelGGL((bwd_dq_f32_kernel<D, true>), gq, block, 0, st, p);
-    hipLaunchKernelGGL((bwd_dkdv_f32_kernel<D, true>), gk, block, 0, st, p);
+    if (p.nsplit > 1) hipLaunchKernelGGL((bwd_dkdv_f32_kernel<D, true, false, true>), gs, block, 0, st, p);
+    else hipLaunchKernelGGL((bwd_dkdv_f32_kernel<D, true>), gk, block, 0, st, p);
   } else {
     hipLaunchKernelGGL((bwd_dq_f32_kernel<D, false>), gq, block, 0, st, p);
-    hipLaunchKernelGGL((bwd_dkdv_f32_kernel<D, false>), gk, block, 0, st, p);
+    if (p.nsplit > 1) hipLaunchKernelGGL((bwd_dkdv_f32_kernel<D, false, false, true>), gs, block, 0, st, p);
+    else hipLaunchKernelGGL((bwd_dkdv_f32_kernel<D, false>), gk, block, 0, st, p);
   }
-  return hipGetLastError();
+  const hipError_t e = hipGetLastError();
+  return e == hipSuccess && p.nsplit > 1 ? launch_dkdv_merge<D, float>(p, causal, st) : e;
 }
 
 hipError_t launch_bwd_f32(const BwdParams& p, int D, bool causal, hipStream_t st) {

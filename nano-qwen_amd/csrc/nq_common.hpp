@@ -219,6 +219,17 @@ __device__ __forceinline__ float xor32_sum(float v) {
   return __uint_as_float(r[0]) + __uint_as_float(r[1]);
 }
 
+// This lane's index (0..63), computed afresh (volatile, so the compiler cannot
+// reuse an earlier value): code after the main loop derives its lane-dependent
+// values from it instead of keeping them live through the loop, where they
+// would be spilled and reloaded (and a reload, counted by vmcnt like the tile
+// loads in flight, waits for those loads too).
+__device__ __forceinline__ int fresh_lane() {
+  int l;
+  asm volatile("v_mbcnt_lo_u32_b32 %0, -1, 0\n\tv_mbcnt_hi_u32_b32 %0, -1, %0" : "=v"(l));
+  return l;
+}
+
 __device__ __forceinline__ float fast_exp2(float x) { return __builtin_amdgcn_exp2f(x); }
 
 // c + the sum of the 8 bf16 values of v, in fp32, with v_dot2_f32_bf16 against

@@ -89,17 +89,6 @@ __device__ __forceinline__ void static_for(F&& f) {
 }
 
 
-// This lane's index (0..63), computed afresh (volatile, so the compiler cannot
-// reuse an earlier value): code after the main loop derives its lane-dependent
-// values from it instead of keeping them live through the loop, where they
-// would be spilled and reloaded (and a reload, counted by vmcnt like the tile
-// loads in flight, waits for those loads too).
-__device__ __forceinline__ int fresh_lane() {
-  int l;
-  asm volatile("v_mbcnt_lo_u32_b32 %0, -1, 0\n\tv_mbcnt_hi_u32_b32 %0, -1, %0" : "=v"(l));
-  return l;
-}
-
 // MFMA row r of a 32-key block holds key sigma(r): bits 2 and 3 swapped.
 __device__ __forceinline__ int key_perm32(int r) {
   return (r & ~12) | ((r & 4) << 1) | ((r & 8) >> 1);

@@ -782,8 +782,10 @@ def attention_backward(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, o: tor
     dk = torch.empty(B, T, Hkv, D, dtype=q.dtype, device=dev).transpose(1, 2)
     dv = torch.empty(B, T, Hkv, D, dtype=q.dtype, device=dev).transpose(1, 2)
     lib = _lib.load()
-    need = int(lib.nq_attn_bwd_workspace_bytes(B, Hq, S))
-    if workspace is None or workspace.numel() * workspace.element_size() < need:
+    if workspace is None or (workspace.numel() * workspace.element_size()
+                             < int(lib.nq_attn_bwd_workspace_bytes(B, Hq, S))):
+        # with room for the partial sums of dK/dV, whose steps a small launch splits
+        need = int(lib.nq_attn_bwd_split_workspace_bytes(B, Hq, Hkv, S, T, D, _code(q), int(bool(causal))))
         workspace = torch.empty(need, dtype=torch.uint8, device=dev)
     st = _lib.strides3
     head = (_ptr(q), st(q.stride()[:3]), _ptr(k), st(k.stride()[:3]), _ptr(v), st(v.stride()[:3]),

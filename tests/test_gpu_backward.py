@@ -407,3 +407,45 @@ def test_attention_backward_full_size(B, Hq, Hkv, S):
             rq, rk, rv = _fp32_grads_on_device(q[b, hs], k[b, kvh], v[b, kvh], do[b, hs])
             for got, ref, name in ((dq[b, hs], rq, "dq"), (dk[b, kvh], rk, "dk"), (dv[b, kvh], rv, "dv")):
                 _close_rel(got, ref, f"{name} b={b} kvh={kvh}")
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("causal", [True, False])
+@pytest.mark.parametrize("Hq,Hkv,D,S,T", [
+    (8, 2, 64, 545, 545),    # 5 key blocks; runs that end inside a tile's group of heads
+    (2, 2, 128, 1000, 1090), # T > S, one head per group
+    (16, 1, 32, 160, 160),   # 16 heads per tile: a run inside the heads of one tile
+    (4, 1, 128, 513, 513),   # a last block of one key, which has a single run
+])
+def test_split_dkdv_backward(Hq, Hkv, D, S, T, causal, dtype):
+    """Launches of few key blocks split their steps into runs; each block's rows are the sum of its runs."""
+    say(f"split dK/dV Hq={Hq} Hkv={Hkv} D={D} S={S} T={T} causal={causal} {dtype}")
+    lib = ops._lib.load()
+    base = lib.nq_attn_bwd_workspace_bytes(1, Hq, S)
+    assert lib.nq_attn_bwd_split_workspace_bytes(1, Hq, Hkv, S, T, D, ops._code(torch.empty(0, dtype=dtype)),
+                                                 int(causal)) > base
+    q = randn(1, Hq, S, D, seed=581, dtype=dtype)
+    k = randn(1, Hkv, T, D, seed=582, dtype=dtype)
+    v = randn(1, Hkv, T, D, seed=583, dtype=dtype)
+    do = randn(1, Hq, S, D, seed=584, dtype=dtype)
+    dv = lambda t: t.to(DEV)  # noqa: E731
+    o, lse = ops.attention_prefill(dv(q), dv(k), dv(v), causal=causal, return_lse=True)
+    lens = torch.tensor([T - 150 if T > 200 else T], dtype=torch.int32)
+    split = ops.attention_backward(dv(q), dv(k), dv(v), o, dv(do), lse, causal=causal)
+    _, rq, rk, rv = _ref_grads(q, k, v, do, causal)
+    for name, got, ref in zip(("dq", "dk", "dv"), split, (rq, rk, rv)):
+        _close_rel(got, ref, name, dtype)
+    # the same steps in one run each (a workspace without room for partials):
+    # the order of fp32 additions is all that differs
+    ws = torch.empty(base, dtype=torch.uint8, device=DEV)
+    whole = ops.attention_backward(dv(q), dv(k), dv(v), o, dv(do), lse, causal=causal, workspace=ws)
+    assert torch.equal(split[0], whole[0])
+    for a, b in zip(split[1:], whole[1:]):
+        _close_rel(a, b, "split against whole", dtype)
+    # key padding: blocks of padding alone have no steps and zero gradients
+    o, lse = ops.attention_prefill(dv(q), dv(k), dv(v), causal=causal, key_lens=dv(lens), return_lse=True)
+    split = ops.attention_backward(dv(q), dv(k), dv(v), o, dv(do), lse, causal=causal, key_lens=dv(lens))
+    whole = ops.attention_backward(dv(q), dv(k), dv(v), o, dv(do), lse, causal=causal, key_lens=dv(lens), workspace=ws)
+    for a, b in zip(split[1:], whole[1:]):
+        _close_rel(a, b, "padded split against whole", dtype)
+        assert not a[:, :, int(lens[0]):].any()
