@@ -17,6 +17,9 @@
  *     accumulation.  fp32 data in nq_attn_prefill_fwd: products on fp32 MFMA
  *     (the reference's SDPA keeps the input dtype).  Norm, RoPE and softmax
  *     arithmetic is fp32 everywhere.
+ *   - norm weights are fp32.  NQ_QWEIGHT_BF16 / NQ_KWEIGHT_BF16 or'd into the
+ *     dtype (dtype_in) of a call on bf16 data say that its q_weight (or weight)
+ *     / k_weight points to bf16 values instead, 16-byte aligned.
  *   - head_dim must be 32, 64 or 128 (the reference's configs use 32 and 128).
  *     kernels/flash_attn.py:106 also allows 16 and 256: nq_attn_prefill_fwd
  *     and nq_attn_bwd take 256 for plain bf16 attention (no QK-Norm/RoPE
@@ -49,6 +52,8 @@ extern "C" {
 
 #define NQ_DTYPE_BF16 0
 #define NQ_DTYPE_F32 1
+#define NQ_QWEIGHT_BF16 0x200
+#define NQ_KWEIGHT_BF16 0x400
 
 /* Library version, e.g. 100 for 0.1.0. */
 int nq_version(void);

@@ -22,6 +22,8 @@ NQ_ERR_WORKSPACE = 3
 NQ_DTYPE_BF16 = 0
 NQ_DTYPE_F32 = 1
 NQ_DECODE_F32_SPLIT = 0x100
+NQ_QWEIGHT_BF16 = 0x200
+NQ_KWEIGHT_BF16 = 0x400
 
 _p = ctypes.c_void_p
 _i32 = ctypes.c_int

@@ -686,7 +686,8 @@ struct NormBwdParams {
   int64_t ysb, ysh, yss;
   void* dx;
   int64_t dsb, dsh, dss;
-  const float* w;
+  const float* w;  // bf16 when w16
+  int w16;
   float* dw;
   float* ws;  // per-block partial dw, gridDim.x x D
   int B, H, S;
@@ -708,8 +709,11 @@ __global__ __launch_bounds__(256) void norm_rope_bwd_kernel(NormBwdParams p) {
   const int64_t nrows = (int64_t)p.B * p.H * p.S;
   floatx8 w1{}, w2{}, a1{}, a2{};
   if (p.w) {
-    w1 = Vec8<float>::load_f32(p.w + sub * 8);
-    w2 = Vec8<float>::load_f32(p.w + D / 2 + sub * 8);
+    Weight8 r1, r2;
+    r1.load(p.w, p.w16, sub * 8);
+    r2.load(p.w, p.w16, D / 2 + sub * 8);
+    w1 = r1.value(p.w16);
+    w2 = r2.value(p.w16);
   }
   for (int64_t row = (int64_t)blockIdx.x * RPB + slot; row < nrows; row += (int64_t)gridDim.x * RPB) {
     const int s = (int)(row % p.S);
@@ -994,6 +998,8 @@ extern "C" int nq_qk_norm_rope_bwd(const void* x, const int64_t* x_strides, cons
                                    float eps, const float* cos_tab, const float* sin_tab, int max_pos,
                                    const int32_t* pos, const int32_t* pos_base, int pos0, void* stream) {
   nq_clear_error();
+  int w16 = 0, k16 = 0;
+  if ((dtype & ~NQ_QWEIGHT_BF16) == NQ_DTYPE_BF16) dtype = nq_take_weight_flags(dtype, &w16, &k16);
   if (!head_dim_ok(D)) return nq_fail(NQ_ERR_UNSUPPORTED, "head_dim must be 32, 64 or 128, got %d", D);
   if (!nq_dtype_ok(dtype)) return nq_fail(NQ_ERR_UNSUPPORTED, "unknown dtype code %d", dtype);
   if (B <= 0 || S <= 0 || H <= 0) return nq_fail(NQ_ERR_INVALID, "sizes must be positive");
@@ -1019,7 +1025,7 @@ extern "C" int nq_qk_norm_rope_bwd(const void* x, const int64_t* x_strides, cons
   p.x = x; p.xsb = x_strides[0]; p.xsh = x_strides[1]; p.xss = x_strides[2];
   p.dy = dy; p.ysb = dy_strides[0]; p.ysh = dy_strides[1]; p.yss = dy_strides[2];
   p.dx = dx; p.dsb = dx_strides[0]; p.dsh = dx_strides[1]; p.dss = dx_strides[2];
-  p.w = weight; p.dw = dweight; p.ws = reinterpret_cast<float*>(workspace);
+  p.w = weight; p.w16 = w16; p.dw = dweight; p.ws = reinterpret_cast<float*>(workspace);
   p.B = B; p.H = H; p.S = S; p.eps = eps;
   p.cos_tab = cos_tab; p.sin_tab = sin_tab; p.max_pos = max_pos;
   p.pos = pos; p.pos_base = pos_base; p.pos0 = pos0;

@@ -257,6 +257,27 @@ __device__ __forceinline__ float row_sum(float v) {
   return v;
 }
 
+// 8 norm weights stored as fp32 or (w16) bf16, both 16-byte aligned.  The load
+// takes two 16-byte pieces either way and no branch, so a prologue's loads still
+// go out together; value() decodes what arrived.
+struct Weight8 {
+  uint32_t __attribute__((ext_vector_type(4))) a, b;
+  __device__ __forceinline__ void load(const void* w, bool w16, int i) {
+    const unsigned char* p = reinterpret_cast<const unsigned char*>(w) + i * (w16 ? 2 : 4);
+    a = *reinterpret_cast<const decltype(a)*>(p);
+    b = *reinterpret_cast<const decltype(b)*>(p + (w16 ? 0 : 16));
+  }
+  __device__ __forceinline__ floatx8 value(bool w16) const {
+    floatx8 v;
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      v[e] = __uint_as_float(w16 ? (e & 1 ? a[e / 2] & 0xffff0000u : a[e / 2] << 16) : a[e]);
+      v[4 + e] = __uint_as_float(w16 ? (e & 1 ? a[2 + e / 2] & 0xffff0000u : a[2 + e / 2] << 16) : b[e]);
+    }
+    return v;
+  }
+};
+
 // Head dims every kernel is built for, and the host-side switch that calls
 // f(std::integral_constant<int, D>) for the one asked for.
 constexpr bool head_dim_ok(int D) { return D == 32 || D == 64 || D == 128; }

@@ -69,7 +69,8 @@ struct DecodeParams {
   float* ws_o;   // (slots, 16, D) unnormalised partial outputs
   float* ws_ml;  // (slots, 16, 2) running max (log2 units) and sum
   int32_t* ws_rw;  // (rows, 2) first and last wave that covered each row
-  const float* qw;
+  const float* qw;  // bf16 when q16
+  int q16, k16;
   float eps;
   const float* cos_tab;
   const float* sin_tab;
@@ -379,7 +380,8 @@ decode_stream_kernel(DecodeParams p) {
     // rope_row: lane `sub` of each group of LPR lanes holds chunks sub and
     // sub + D/16 of the row
     const int sub = lane % LPR;
-    floatx8 ka1{}, ka2{}, va1{}, va2{}, kw1{}, kw2{}, kc1{}, ks1{};
+    floatx8 ka1{}, ka2{}, va1{}, va2{}, kc1{}, ks1{};
+    Weight8 kw1{}, kw2{};
     if (tail) {
       const T* ks = reinterpret_cast<const T*>(p.kn) + b * p.knsb + kvh * p.knsh + sub * 8;
       const T* vs = reinterpret_cast<const T*>(p.vn) + b * p.vnsb + kvh * p.vnsh + sub * 8;
@@ -388,8 +390,8 @@ decode_stream_kernel(DecodeParams p) {
       va1 = Vec8<T>::load_f32(vs);
       va2 = Vec8<T>::load_f32(vs + D / 2);
       if (p.kw) {
-        kw1 = Vec8<float>::load_f32(p.kw + sub * 8);
-        kw2 = Vec8<float>::load_f32(p.kw + D / 2 + sub * 8);
+        kw1.load(p.kw, p.k16, sub * 8);
+        kw2.load(p.kw, p.k16, D / 2 + sub * 8);
       }
     }
 
@@ -402,12 +404,13 @@ decode_stream_kernel(DecodeParams p) {
     // in the same lane (d blocks dq and dq + NDQ/2); for D = 32 (one d block)
     // element d of lanes 0..31 pairs with d + 16 of lanes 32..63
     constexpr int NCS = NDQ >= 2 ? NDQ / 2 : 1;
-    floatx8 xf[NDQ], wq[NDQ], cs[NCS], sn[NCS];
+    floatx8 xf[NDQ], cs[NCS], sn[NCS];
+    Weight8 wq[NDQ];
 #pragma unroll
     for (int dq = 0; dq < NDQ; ++dq) xf[dq] = Vec8<T>::load_f32(qrow + dq * 32 + grp * 8);
     if (p.qw) {
 #pragma unroll
-      for (int dq = 0; dq < NDQ; ++dq) wq[dq] = Vec8<float>::load_f32(p.qw + dq * 32 + grp * 8);
+      for (int dq = 0; dq < NDQ; ++dq) wq[dq].load(p.qw, p.q16, dq * 32 + grp * 8);
     }
     const int pos =
         p.cos_tab ? table_row(p.q_pos ? ld_uniform(p.q_pos, b) : (p.q_pos0 >= 0 ? p.q_pos0 : len - 1), p.max_pos) : 0;
@@ -456,7 +459,7 @@ decode_stream_kernel(DecodeParams p) {
     // kernel, so the cached row matches its K-hat bit for bit), written back
     // by one wave per (batch, kv head); no wave of this launch reads that row
     if (tail) {
-      if (p.kw) norm_row<D>(ka1, ka2, kw1, kw2, p.eps);
+      if (p.kw) norm_row<D>(ka1, ka2, kw1.value(p.k16), kw2.value(p.k16), p.eps);
       if (p.cos_tab) rope_row(ka1, ka2, kc1, ks1);
       if (hg == 0 && lane < LPR) {
         const int t = len - 1;
@@ -487,9 +490,11 @@ decode_stream_kernel(DecodeParams p) {
         ss += shfl_xor_f(ss, 32);
         const float r = rsqrtf(ss / (float)D + p.eps);
 #pragma unroll
-        for (int dq = 0; dq < NDQ; ++dq)
+        for (int dq = 0; dq < NDQ; ++dq) {
+          const floatx8 wv = wq[dq].value(p.q16);
 #pragma unroll
-          for (int e = 0; e < 8; ++e) xf[dq][e] = xf[dq][e] * r * wq[dq][e];
+          for (int e = 0; e < 8; ++e) xf[dq][e] = xf[dq][e] * r * wv[e];
+        }
       }
       if (p.cos_tab) {
         if constexpr (NDQ >= 2) {
@@ -1108,6 +1113,7 @@ static int decode_setup(DecodeParams& p, const void* q, const int64_t* q_strides
   if (!head_dim_ok(D)) return nq_fail(NQ_ERR_UNSUPPORTED, "head_dim must be 32, 64 or 128, got %d", D);
   // partials in the workspace: always for bf16, on request for fp32 (whose
   // callers otherwise pass none, or one that other calls may be using)
+  if ((dtype & ~(NQ_QWEIGHT_BF16 | NQ_KWEIGHT_BF16)) == NQ_DTYPE_BF16) dtype = nq_take_weight_flags(dtype, &p.q16, &p.k16);
   const bool f32_split = dtype == (NQ_DTYPE_F32 | NQ_DECODE_F32_SPLIT);
   if (f32_split) dtype = NQ_DTYPE_F32;
   const bool partials = dtype == NQ_DTYPE_BF16 || f32_split;

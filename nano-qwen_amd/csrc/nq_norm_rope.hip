@@ -32,7 +32,8 @@ struct RowJob {
   void* dst;
   int64_t sb, sh, ss;   // source strides (elements)
   int64_t db, dh, ds;   // destination strides (elements)
-  const float* weight;  // RMSNorm weight (D) or null
+  const float* weight;  // RMSNorm weight (D) or null; bf16 when w16
+  int w16;
   int H;
   int rope;             // apply RoPE
   int norm;             // apply RMSNorm
@@ -96,9 +97,11 @@ __global__ __launch_bounds__(256) void norm_rope_rows_kernel(RowParams p) {
   unsigned char* const wslot = smem + wave * ROW_WAVE_LDS;  // weight
   unsigned char* const tslot = wslot + 1024;                // table chunks
   const int64_t nrows = (int64_t)p.B * jb.H * p.S;
-  // lane l stages weight values [4 (l % (D/4)), +4): the slot holds the
-  // weight (repeated for D < 256); waited for with the first row
-  if (jb.norm) global_load_lds16(jb.weight + (lane % (D / 4)) * 4, wslot);
+  // lane l stages the weight's 16-byte piece l % pieces: the slot holds the
+  // weight, repeated; waited for with the first row
+  const bool w16 = jb.w16;
+  if (jb.norm)
+    global_load_lds16(reinterpret_cast<const unsigned char*>(jb.weight) + (lane % (w16 ? D / 8 : D / 4)) * 16, wslot);
   // explicit or per-batch positions need a load before the table row is known;
   // the plain pos0 + s form needs none (a separate loop, so no merged path
   // waits on a position load that was never issued)
@@ -146,14 +149,10 @@ __global__ __launch_bounds__(256) void norm_rope_rows_kernel(RowParams p) {
       wait_vmcnt0();
       const int z = row_opaque_zero();
       if (jb.norm) {
-        const unsigned char* w = wslot + z + sub * 32;
-        const floatx4 a0 = *reinterpret_cast<const floatx4*>(w);
-        const floatx4 a1 = *reinterpret_cast<const floatx4*>(w + 16);
-        const floatx4 b0 = *reinterpret_cast<const floatx4*>(w + D * 2);
-        const floatx4 b1 = *reinterpret_cast<const floatx4*>(w + D * 2 + 16);
-        const floatx8 w1{a0[0], a0[1], a0[2], a0[3], a1[0], a1[1], a1[2], a1[3]};
-        const floatx8 w2{b0[0], b0[1], b0[2], b0[3], b1[0], b1[1], b1[2], b1[3]};
-        norm_row<D>(x1, x2, w1, w2, p.eps);
+        Weight8 w1, w2;
+        w1.load(wslot + z, w16, sub * 8);
+        w2.load(wslot + z, w16, D / 2 + sub * 8);
+        norm_row<D>(x1, x2, w1.value(w16), w2.value(w16), p.eps);
       }
       if (jb.rope) {
         const unsigned char* t = tslot + z + lane * 16;
@@ -222,6 +221,8 @@ static int qk_norm_rope_impl(const void* q, const int64_t* q_strides, void* q_ou
                              const int32_t* kv_row_base, int kv_row0, const int32_t* block_table,
                              int64_t bt_stride, int page_size, void* stream) {
   nq_clear_error();
+  int q16, k16;
+  dtype_in = nq_take_weight_flags(dtype_in, &q16, &k16);
   if (!head_dim_ok(D)) return nq_fail(NQ_ERR_UNSUPPORTED, "head_dim must be 32, 64 or 128, got %d", D);
   if (B <= 0 || S <= 0) return nq_fail(NQ_ERR_INVALID, "B and S must be positive (B=%d S=%d)", B, S);
   if (!nq_dtype_ok(dtype_in) || !nq_dtype_ok(dtype_out))
@@ -239,10 +240,10 @@ static int qk_norm_rope_impl(const void* q, const int64_t* q_strides, void* q_ou
   p.pos = pos; p.pos_base = pos_base; p.pos0 = pos0;
   p.row_base = kv_row_base; p.row0 = kv_row0;
   int nj = 0, max_h = 0;
-  struct In { const void* s; const int64_t* ss; void* d; const int64_t* ds; int H; const float* w; int rope; int rb; const char* name; };
-  In ins[3] = {{q, q_strides, q_out, q_out_strides, Hq, q_weight, 1, 0, "q"},
-               {k, k_strides, k_out, k_out_strides, Hkv, k_weight, 1, 1, "k"},
-               {v, v_strides, v_out, v_out_strides, Hkv, nullptr, 0, 1, "v"}};
+  struct In { const void* s; const int64_t* ss; void* d; const int64_t* ds; int H; const float* w; int w16; int rope; int rb; const char* name; };
+  In ins[3] = {{q, q_strides, q_out, q_out_strides, Hq, q_weight, q16, 1, 0, "q"},
+               {k, k_strides, k_out, k_out_strides, Hkv, k_weight, k16, 1, 1, "k"},
+               {v, v_strides, v_out, v_out_strides, Hkv, nullptr, 0, 0, 1, "v"}};
   for (const In& in : ins) {
     if (!in.s) continue;
     if (!in.d || !in.ss || !in.ds) return nq_fail(NQ_ERR_INVALID, "%s: output and strides required", in.name);
@@ -257,7 +258,7 @@ static int qk_norm_rope_impl(const void* q, const int64_t* q_strides, void* q_ou
     j.src = in.s; j.dst = in.d;
     j.sb = in.ss[0]; j.sh = in.ss[1]; j.ss = in.ss[2];
     j.db = in.ds[0]; j.dh = in.ds[1]; j.ds = in.ds[2];
-    j.weight = in.w; j.H = in.H; j.rope = in.rope && cos_tab != nullptr; j.norm = in.w != nullptr;
+    j.weight = in.w; j.w16 = in.w16; j.H = in.H; j.rope = in.rope && cos_tab != nullptr; j.norm = in.w != nullptr;
     j.use_row_base = in.rb;
     j.heads_inner = in.H > 1 && S > 1 && (in.ss[1] < 0 ? -in.ss[1] : in.ss[1]) < (in.ss[2] < 0 ? -in.ss[2] : in.ss[2]);
     if (in.H > max_h) max_h = in.H;

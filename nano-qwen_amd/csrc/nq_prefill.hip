@@ -390,14 +390,20 @@ prefill_kernel(PrefillParams p) {
       // the same 8, so both halves' values come as wave-uniform loads and each
       // lane selects its own (as vector loads, 16 of them issued at ~220
       // clocks each: 1.8 us of a ~7.5 us prologue at the 1.7B-like shape)
-      const auto* wc = (const __attribute__((address_space(4))) float*)p.qw;  // read-only
+      auto norm = [&](auto weight) {
 #pragma unroll
-      for (int db = 0; db < NDB; ++db)
+        for (int db = 0; db < NDB; ++db)
 #pragma unroll
-        for (int e = 0; e < 8; ++e) {
-          const float w0 = wc[db * 16 + e], w1 = wc[db * 16 + 8 + e];
-          xf[db][e] = xf[db][e] * r * (hh ? w1 : w0);
-        }
+          for (int e = 0; e < 8; ++e)
+            xf[db][e] = xf[db][e] * r * (hh ? weight(db * 16 + 8 + e) : weight(db * 16 + e));
+      };
+      if (p.q16) {  // bf16 weights, two to a word
+        const auto* wc = (const __attribute__((address_space(4))) uint32_t*)p.qw;  // read-only
+        norm([&](int i) { return __uint_as_float(i & 1 ? wc[i / 2] & 0xffff0000u : wc[i / 2] << 16); });
+      } else {
+        const auto* wc = (const __attribute__((address_space(4))) float*)p.qw;
+        norm([&](int i) { return wc[i]; });
+      }
     }
     if (do_rope) {
 #pragma unroll
@@ -927,6 +933,8 @@ static int prefill_entry(const void* q, const int64_t* q_strides, const void* k,
                          const float* cos_tab, const float* sin_tab, int max_pos, const int32_t* q_pos,
                          const int32_t* q_pos_base, int q_pos0, int causal, float sm_scale, void* workspace,
                          int64_t workspace_bytes, void* stream) {
+  int q16 = 0, k16 = 0;  // the key weight is not this call's
+  if ((dtype & ~NQ_QWEIGHT_BF16) == NQ_DTYPE_BF16) dtype = nq_take_weight_flags(dtype, &q16, &k16);
   // head_dim 256 (kernels/flash_attn.py:106): plain bf16 attention only
   const bool wide = D == 256;
   if (wide && (dtype != NQ_DTYPE_BF16 || q_weight || cos_tab || key_lens || bias || bt))
@@ -976,7 +984,7 @@ static int prefill_entry(const void* q, const int64_t* q_strides, const void* k,
   p.ksb = k_strides[0]; p.ksh = k_strides[1]; p.kss = k_strides[2];
   p.vsb = v_strides[0]; p.vsh = v_strides[1]; p.vss = v_strides[2];
   p.osb = o_strides[0]; p.osh = o_strides[1]; p.oss = o_strides[2];
-  p.qw = q_weight; p.eps = eps; p.cos_tab = cos_tab; p.sin_tab = sin_tab; p.max_pos = max_pos;
+  p.qw = q_weight; p.q16 = q16; p.eps = eps; p.cos_tab = cos_tab; p.sin_tab = sin_tab; p.max_pos = max_pos;
   p.q_pos = q_pos; p.q_pos_base = q_pos_base; p.q_pos0 = q_pos0;
   p.B = B; p.Hq = Hq; p.Hkv = Hkv; p.G = G; p.S = S; p.T = T;
   p.kv_lens = key_lens; p.kv_extra = 0; p.kv_max = T;

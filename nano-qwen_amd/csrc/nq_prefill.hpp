@@ -16,7 +16,8 @@ struct PrefillParams {
   int64_t ksb, ksh, kss;
   int64_t vsb, vsh, vss;
   int64_t osb, osh, oss;
-  const float* qw;
+  const float* qw;  // bf16 when q16
+  int q16;
   float eps;
   const float* cos_tab;
   const float* sin_tab;

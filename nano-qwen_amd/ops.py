@@ -94,6 +94,16 @@ def _f32(t: Optional[torch.Tensor], device) -> Optional[torch.Tensor]:
     return t
 
 
+def _norm_weight(t: Optional[torch.Tensor], device, dt: int, flag: int, plan: bool = False):
+    """A norm weight as the kernels read it, and the flag for the call's dtype code: bf16
+    weights of a call on bf16 data as they are (``flag``), others as fp32 (0).  A plan keeps
+    the fp32 copy of the weight it was made with."""
+    if (t is not None and not plan and dt == _lib.NQ_DTYPE_BF16 and t.dtype == torch.bfloat16
+            and t.device == device and t.is_contiguous() and t.data_ptr() % 16 == 0):
+        return t, flag
+    return _f32(t, device), 0
+
+
 def _i32(t: Optional[torch.Tensor], device) -> Optional[torch.Tensor]:
     if t is None:
         return None
@@ -247,7 +257,9 @@ def qk_norm_rope(q: Optional[torch.Tensor] = None, k: Optional[torch.Tensor] = N
     pos = _positions(position_ids, pos_offset, pos_base, B, S, max_pos, dev)
     pb = _i32(pos_base, dev)
     rb = _i32(kv_row_base, dev)
-    qw, kw = _f32(q_weight, dev), _f32(k_weight, dev)
+    qw, qf = _norm_weight(q_weight, dev, dt_in, _lib.NQ_QWEIGHT_BF16, plan)
+    kw, kf = _norm_weight(k_weight, dev, dt_in, _lib.NQ_KWEIGHT_BF16, plan)
+    dt_in |= qf | kf
     lib = _lib.load()
     st = _lib.strides3
     args = (
@@ -360,7 +372,9 @@ def attention_prefill(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, *,
     cos_t, sin_t, max_pos = _tables(cos, sin, dev)
     pos = _positions(position_ids, pos_offset, pos_base, B, S, max_pos, dev)
     pb = _i32(pos_base, dev)
-    qw = _f32(q_weight, dev)
+    ws = _prefill_workspace(B, Hq, Hkv, S, T, D, dt, dev) if bias is None and kl is None else None
+    qw, flag = _norm_weight(q_weight, dev, dt, _lib.NQ_QWEIGHT_BF16, plan)
+    dt |= flag
     st = _lib.strides3
     head = (_ptr(q), st(q.stride()[:3]), _ptr(k), st(k.stride()[:3]), _ptr(v), st(v.stride()[:3]),
             _ptr(out), st(out.stride()[:3]), _ptr(lse), _ptr(kl))
@@ -374,7 +388,6 @@ def attention_prefill(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, *,
         call = KernelCall(_lib.load().nq_attn_prefill_bias_fwd, args, len(args) - 1, "nq_attn_prefill_bias_fwd",
                           keep + (bias.bias,), (out, lse) if return_lse else out)
     else:
-        ws = _prefill_workspace(B, Hq, Hkv, S, T, D, dt, dev) if kl is None else None
         if ws is not None:
             args = head[:6] + (None, 0, 0) + head[6:9] + (_ptr(ws), ws.numel()) + tail
             call = KernelCall(_lib.load().nq_attn_prefill_ws_fwd, args, len(args) - 1, "nq_attn_prefill_ws_fwd",
@@ -445,9 +458,10 @@ def attention_prefill_paged(q: torch.Tensor, k_pool: torch.Tensor, v_pool: torch
     cos_t, sin_t, max_pos = _tables(cos, sin, dev)
     pos = _positions(position_ids, pos_offset, pos_base, B, S, max_pos, dev)
     pb = _i32(pos_base, dev)
-    qw = _f32(q_weight, dev)
-    st = _lib.strides3
     ws = _prefill_workspace(B, Hq, Hkv, S, int(T), D, dt, dev)
+    qw, flag = _norm_weight(q_weight, dev, dt, _lib.NQ_QWEIGHT_BF16, plan)
+    dt |= flag
+    st = _lib.strides3
     name = "nq_attn_prefill_paged_fwd" if ws is None else "nq_attn_prefill_ws_fwd"
     args = (
         _ptr(q), st(q.stride()[:3]), _ptr(k_pool), st(k_pool.stride()[:3]), _ptr(v_pool),
@@ -538,7 +552,8 @@ def attention_decode(q: torch.Tensor, k_cache: torch.Tensor, v_cache: torch.Tens
     cos_t, sin_t, max_pos = _tables(cos, sin, dev)
     lens_t = _i32(lens, dev)
     qp = _decode_q_pos(q_pos, q_pos0, B, max_pos, dev)
-    qw = _f32(q_weight, dev)
+    qw, flag = _norm_weight(q_weight, dev, dt, _lib.NQ_QWEIGHT_BF16, plan)
+    dt |= flag
     q_str = (ctypes.c_int64 * 2)(q.stride(0), q.stride(1))
     o_str = (ctypes.c_int64 * 2)(out.stride(0), out.stride(1))
     st = _lib.strides3
@@ -610,14 +625,14 @@ def kv_append_paged(k: Optional[torch.Tensor], v: Optional[torch.Tensor], k_pool
     pos = _positions(position_ids, pos_offset, pos_base, B, S, max_pos, dev)
     pb = _i32(pos_base, dev)
     rb = _i32(row_base, dev)
-    kw = _f32(k_weight, dev)
+    kw, flag = _norm_weight(k_weight, dev, _code(ref), _lib.NQ_KWEIGHT_BF16, plan)
     st = _lib.strides3
     args = (
         _ptr(k), st(k.stride()[:3]) if k is not None else None,
         _ptr(v), st(v.stride()[:3]) if v is not None else None,
         _ptr(k_pool), st(k_pool.stride()[:3]), _ptr(v_pool), st(v_pool.stride()[:3]),
         _ptr(bt), bt.stride(0), k_pool.shape[2],
-        B, S, Hkv, D, _code(ref), _code(k_pool), _ptr(kw), float(eps),
+        B, S, Hkv, D, _code(ref) | flag, _code(k_pool), _ptr(kw), float(eps),
         _ptr(cos_t), _ptr(sin_t), max_pos, _ptr(pos), _ptr(pb), int(pos_offset),
         _ptr(rb), int(row_offset), _stream(ref))
     call = KernelCall(_lib.load().nq_kv_append_paged, args, len(args) - 1, "nq_kv_append_paged",
@@ -693,7 +708,9 @@ def attention_decode_paged(q: torch.Tensor, k_pool: torch.Tensor, v_pool: torch.
     wbytes = workspace.numel() * workspace.element_size()
     cos_t, sin_t, max_pos = _tables(cos, sin, dev)
     qp = _decode_q_pos(q_pos, q_pos0, B, max_pos, dev)
-    qw, kw = _f32(q_weight, dev), _f32(k_weight, dev)
+    qw, qf = _norm_weight(q_weight, dev, dt, _lib.NQ_QWEIGHT_BF16, plan)
+    kw, kf = _norm_weight(k_weight, dev, dt, _lib.NQ_KWEIGHT_BF16, plan)
+    dt |= qf | kf
     q_str = (ctypes.c_int64 * 2)(q.stride(0), q.stride(1))
     o_str = (ctypes.c_int64 * 2)(out.stride(0), out.stride(1))
     kn_str = vn_str = None
@@ -823,7 +840,8 @@ def qk_norm_rope_backward(x: torch.Tensor, dy: torch.Tensor, *, weight: Optional
     x, dy = _rows_in(x), _rows_in(dy)
     dev = x.device
     dx = torch.empty(B, S, H, D, dtype=x.dtype, device=dev).transpose(1, 2)
-    w = _f32(weight, dev)
+    dt = _code(x)
+    w, flag = _norm_weight(weight, dev, dt, _lib.NQ_QWEIGHT_BF16)
     lib = _lib.load()
     dw, ws, wbytes = None, None, 0
     if w is not None:
@@ -836,7 +854,7 @@ def qk_norm_rope_backward(x: torch.Tensor, dy: torch.Tensor, *, weight: Optional
     st = _lib.strides3
     rc = lib.nq_qk_norm_rope_bwd(
         _ptr(x), st(x.stride()[:3]), _ptr(dy), st(dy.stride()[:3]), _ptr(dx), st(dx.stride()[:3]),
-        _ptr(w), _ptr(dw), _ptr(ws), wbytes, B, S, H, D, _code(x), float(eps), _ptr(cos_t), _ptr(sin_t),
+        _ptr(w), _ptr(dw), _ptr(ws), wbytes, B, S, H, D, dt | flag, float(eps), _ptr(cos_t), _ptr(sin_t),
         max_pos, _ptr(pos), _ptr(pb), int(pos_offset), _stream(x))
     _lib.check(rc, "nq_qk_norm_rope_bwd")
     return dx, dw

@@ -143,3 +143,34 @@ def test_rows_many_passes_and_out_of_range_positions(D, S, dtype, layout):
             torch.testing.assert_close(got[ok], want[ok], rtol=2e-5, atol=2e-5)
         else:
             assert_bf16_close(got[ok], want[ok], name)
+
+
+@pytest.mark.parametrize("D", [32, 64, 128])
+def test_bf16_norm_weights_are_read_as_they_are(D):
+    """Every entry point given bf16 norm weights gives the bits it gives for the same values in fp32."""
+    say(f"bf16 norm weights D={D}")
+    B, S, Hq, Hkv, P = 2, 45, 4, 2, 64
+    dt = torch.bfloat16
+    x = lambda seed, H: randn(B, S, H, D, seed=seed, dtype=dt).to(DEV).transpose(1, 2)  # noqa: E731
+    q, k, v = x(301, Hq), x(302, Hkv), x(303, Hkv)
+    weights = [(1 + 0.1 * randn(D, seed=s)).to(dt).to(DEV) for s in (304, 305)]
+    cos, sin = (t.to(DEV) for t in rope_tables(D, 128, 1e6))
+    args = dict(eps=1e-6, cos=cos, sin=sin)
+    bt = torch.arange(B, dtype=torch.int32, device=DEV).view(B, 1)
+    lens = torch.full((B,), S, dtype=torch.int32, device=DEV)
+
+    def outputs(qw, kw):
+        qh, kh, _ = nq.qk_norm_rope(q=q, k=k, q_weight=qw, k_weight=kw, **args)
+        o = nq.attention_prefill(q, kh, v, q_weight=qw, **args)
+        kp, vp = torch.zeros(B, Hkv, P, D, dtype=dt, device=DEV), torch.zeros(B, Hkv, P, D, dtype=dt, device=DEV)
+        nq.kv_append_paged(k, v, kp, vp, bt, k_weight=kw, **args)
+        op = nq.attention_prefill_paged(q, kp, vp, bt, T=S, q_weight=qw, **args)
+        od = nq.attention_decode(q[:, :, 3], kp, vp, lens, max_len=S, q_weight=qw, **args)
+        kp2, vp2 = kp.clone(), vp.clone()
+        oa = nq.attention_decode_paged(q[:, :, 3], kp2, vp2, bt, lens, max_len=S + 1, k_new=k[:, :, 7].contiguous(),
+                                       v_new=v[:, :, 7].contiguous(), k_weight=kw, q_weight=qw, **args)
+        dx, dw = nq.qk_norm_rope_backward(k, kh, weight=kw, **args)
+        return qh, kh, o, kp, op, od, kp2, oa, dx, dw
+
+    for i, (a, b) in enumerate(zip(outputs(*weights), outputs(*(w.float() for w in weights)))):
+        assert torch.equal(a, b), f"output {i}"
