@@ -145,7 +145,14 @@ struct PfTile {
 // the workspace for prefill_merge_kernel.  Without it a launch of 128 workgroups
 // (B1, 500 queries on 12345 paged keys, 32/8 heads) ran 277 us on half the CUs;
 // with four runs each and the merge 121 us, 851 TFLOP/s.
-template <int D, typename T, bool CAUSAL, bool FUSE_Q, int NW, bool PAGED = false, bool BIAS = false,
+// FUSE: what happens to Q on its load: PF_PLAIN nothing, PF_FUSED QK-Norm and /
+// or RoPE (either skipped when not given), PF_FUSED16 the same with bf16 weights.
+// Dense instances are built for one type of weight: where a branch on it stands
+// between the row's sum of squares and the weights' scalar loads, these are
+// waited for (1.7B-like prefill 152.0 -> 154.7 us).  The paged, bias and split
+// ones branch.
+enum { PF_PLAIN, PF_FUSED, PF_FUSED16 };
+template <int D, typename T, bool CAUSAL, int FUSE, int NW, bool PAGED = false, bool BIAS = false,
           bool SPLIT = false>
 __global__ void __attribute__((amdgpu_flat_work_group_size(64 * NW, 64 * NW),
                                amdgpu_waves_per_eu(2, 2)))
@@ -307,8 +314,8 @@ prefill_kernel(PrefillParams p) {
   // work starts (each load depending on an earlier one's result would cost a
   // round trip of its own).  The table row is resolved before anything is in
   // flight: only explicit per-token positions need a load for it.
-  const bool do_norm = FUSE_Q && p.qw != nullptr;
-  const bool do_rope = FUSE_Q && p.cos_tab != nullptr;
+  const bool do_norm = FUSE != PF_PLAIN && p.qw != nullptr;
+  const bool do_rope = FUSE != PF_PLAIN && p.cos_tab != nullptr;
   int tab_row = 0;
   if (do_rope) tab_row = table_row(row_position(p.q_pos, p.q_pos_base, p.q_pos0, b, qi_c, p.S), p.max_pos);
   // The cos/sin rows of the workgroup's BM consecutive positions are staged in
@@ -390,20 +397,31 @@ prefill_kernel(PrefillParams p) {
       // the same 8, so both halves' values come as wave-uniform loads and each
       // lane selects its own (as vector loads, 16 of them issued at ~220
       // clocks each: 1.8 us of a ~7.5 us prologue at the 1.7B-like shape)
-      auto norm = [&](auto weight) {
+      auto norm16 = [&]() {  // two weights to a word
+        const auto* wc = (const __attribute__((address_space(4))) uint32_t*)p.qw;  // read-only
 #pragma unroll
         for (int db = 0; db < NDB; ++db)
 #pragma unroll
-          for (int e = 0; e < 8; ++e)
-            xf[db][e] = xf[db][e] * r * (hh ? weight(db * 16 + 8 + e) : weight(db * 16 + e));
+          for (int e = 0; e < 8; e += 2) {
+            const uint32_t w0 = wc[db * 8 + e / 2], w1 = wc[db * 8 + 4 + e / 2];
+            const uint32_t w = hh ? w1 : w0;
+            xf[db][e] = xf[db][e] * r * __uint_as_float(w << 16);
+            xf[db][e + 1] = xf[db][e + 1] * r * __uint_as_float(w & 0xffff0000u);
+          }
       };
-      if (p.q16) {  // bf16 weights, two to a word
-        const auto* wc = (const __attribute__((address_space(4))) uint32_t*)p.qw;  // read-only
-        norm([&](int i) { return __uint_as_float(i & 1 ? wc[i / 2] & 0xffff0000u : wc[i / 2] << 16); });
-      } else {
+      auto norm32 = [&]() {
         const auto* wc = (const __attribute__((address_space(4))) float*)p.qw;
-        norm([&](int i) { return wc[i]; });
-      }
+#pragma unroll
+        for (int db = 0; db < NDB; ++db)
+#pragma unroll
+          for (int e = 0; e < 8; ++e) {
+            const float w0 = wc[db * 16 + e], w1 = wc[db * 16 + 8 + e];
+            xf[db][e] = xf[db][e] * r * (hh ? w1 : w0);
+          }
+      };
+      if constexpr (FUSE == PF_FUSED16) norm16();
+      else if ((PAGED || BIAS || SPLIT) && p.q16) norm16();
+      else norm32();
     }
     if (do_rope) {
 #pragma unroll
@@ -845,53 +863,39 @@ __global__ void __launch_bounds__(2 * D) prefill_merge_kernel(PrefillParams p) {
   }
 }
 
-template <int D, bool CAUSAL>
-static hipError_t launch_prefill_split(const PrefillParams& p, hipStream_t st) {
+// Paged pools, biases (4 waves, dense K/V) and split keys have one instance: its
+// norm and rotation are skipped when not given.
+template <int D, int NW, bool CAUSAL>
+static hipError_t launch_prefill_nw(const PrefillParams& p, bool fuse, hipStream_t st) {
   const int64_t wgs = (int64_t)p.nqb * p.B * p.Hkv;
-  const dim3 grid((unsigned)(wgs * p.nsplit)), block(256);
-  if (p.bt) hipLaunchKernelGGL((prefill_kernel<D, bf16, CAUSAL, true, 4, true, false, true>), grid, block, 0, st, p);
-  else hipLaunchKernelGGL((prefill_kernel<D, bf16, CAUSAL, true, 4, false, false, true>), grid, block, 0, st, p);
-  const hipError_t e = hipGetLastError();
-  if (e != hipSuccess) return e;
-  hipLaunchKernelGGL((prefill_merge_kernel<D, CAUSAL>), dim3((unsigned)(wgs * 4)), dim3(2 * D), 0, st, p);
-  return hipGetLastError();
-}
-
-template <int D, typename T, int NW>
-static hipError_t launch_prefill_nw(const PrefillParams& p, bool causal, bool fuse, hipStream_t st) {
-  dim3 grid((unsigned)(p.nqb * p.B * p.Hkv));
-  dim3 block(64 * NW);
-  if (p.bias) {  // an attention bias: 4-wave workgroups, the fused-Q instance, dense K/V
+  const dim3 grid((unsigned)(wgs * p.nsplit)), block(64 * NW);
+  if (p.bias || p.nsplit > 1) {
     if constexpr (NW == 4) {
-      if (causal) hipLaunchKernelGGL((prefill_kernel<D, T, true, true, 4, false, true>), grid, block, 0, st, p);
-      else hipLaunchKernelGGL((prefill_kernel<D, T, false, true, 4, false, true>), grid, block, 0, st, p);
+      if (p.bias) hipLaunchKernelGGL((prefill_kernel<D, bf16, CAUSAL, PF_FUSED, 4, false, true>), grid, block, 0, st, p);
+      else if (p.bt) hipLaunchKernelGGL((prefill_kernel<D, bf16, CAUSAL, PF_FUSED, 4, true, false, true>), grid, block, 0, st, p);
+      else hipLaunchKernelGGL((prefill_kernel<D, bf16, CAUSAL, PF_FUSED, 4, false, false, true>), grid, block, 0, st, p);
+      const hipError_t e = hipGetLastError();
+      if (e != hipSuccess || p.bias) return e;
+      hipLaunchKernelGGL((prefill_merge_kernel<D, CAUSAL>), dim3((unsigned)(wgs * 4)), dim3(2 * D), 0, st, p);
       return hipGetLastError();
     }
     return hipErrorInvalidValue;
   }
-  if (p.bt) {  // paged pools: the fused-Q instance (its norm and rotation are skipped when not given)
-    if (causal) hipLaunchKernelGGL((prefill_kernel<D, T, true, true, NW, true>), grid, block, 0, st, p);
-    else hipLaunchKernelGGL((prefill_kernel<D, T, false, true, NW, true>), grid, block, 0, st, p);
-    return hipGetLastError();
-  }
-  if (causal) {
-    if (fuse) hipLaunchKernelGGL((prefill_kernel<D, T, true, true, NW>), grid, block, 0, st, p);
-    else hipLaunchKernelGGL((prefill_kernel<D, T, true, false, NW>), grid, block, 0, st, p);
-  } else {
-    if (fuse) hipLaunchKernelGGL((prefill_kernel<D, T, false, true, NW>), grid, block, 0, st, p);
-    else hipLaunchKernelGGL((prefill_kernel<D, T, false, false, NW>), grid, block, 0, st, p);
-  }
+  if (p.bt) hipLaunchKernelGGL((prefill_kernel<D, bf16, CAUSAL, PF_FUSED, NW, true>), grid, block, 0, st, p);
+  else if (p.q16) hipLaunchKernelGGL((prefill_kernel<D, bf16, CAUSAL, PF_FUSED16, NW>), grid, block, 0, st, p);
+  else if (fuse) hipLaunchKernelGGL((prefill_kernel<D, bf16, CAUSAL, PF_FUSED, NW>), grid, block, 0, st, p);
+  else hipLaunchKernelGGL((prefill_kernel<D, bf16, CAUSAL, PF_PLAIN, NW>), grid, block, 0, st, p);
   return hipGetLastError();
 }
 
-template <int D, typename T>
+template <int D>
 static hipError_t launch_prefill(const PrefillParams& p, int nw, bool causal, bool fuse, hipStream_t st) {
   if constexpr (D == 32) {
     if (nw != 4) return hipErrorInvalidValue;  // one 1 KiB tile load per wave needs 4 waves
-    return launch_prefill_nw<D, T, 4>(p, causal, fuse, st);
-  } else {
-    return nw == 8 ? launch_prefill_nw<D, T, 8>(p, causal, fuse, st) : launch_prefill_nw<D, T, 4>(p, causal, fuse, st);
+  } else if (nw == 8) {
+    return causal ? launch_prefill_nw<D, 8, true>(p, fuse, st) : launch_prefill_nw<D, 8, false>(p, fuse, st);
   }
+  return causal ? launch_prefill_nw<D, 4, true>(p, fuse, st) : launch_prefill_nw<D, 4, false>(p, fuse, st);
 }
 
 }  // namespace nq
@@ -984,7 +988,7 @@ static int prefill_entry(const void* q, const int64_t* q_strides, const void* k,
   p.ksb = k_strides[0]; p.ksh = k_strides[1]; p.kss = k_strides[2];
   p.vsb = v_strides[0]; p.vsh = v_strides[1]; p.vss = v_strides[2];
   p.osb = o_strides[0]; p.osh = o_strides[1]; p.oss = o_strides[2];
-  p.qw = q_weight; p.q16 = q16; p.eps = eps; p.cos_tab = cos_tab; p.sin_tab = sin_tab; p.max_pos = max_pos;
+  p.qw = q_weight; p.q16 = q16 && q_weight; p.eps = eps; p.cos_tab = cos_tab; p.sin_tab = sin_tab; p.max_pos = max_pos;
   p.q_pos = q_pos; p.q_pos_base = q_pos_base; p.q_pos0 = q_pos0;
   p.B = B; p.Hq = Hq; p.Hkv = Hkv; p.G = G; p.S = S; p.T = T;
   p.kv_lens = key_lens; p.kv_extra = 0; p.kv_max = T;
@@ -1021,13 +1025,9 @@ static int prefill_entry(const void* q, const int64_t* q_strides, const void* k,
       return nq_fail(NQ_ERR_WORKSPACE, "workspace of %lld bytes (16-byte aligned) required, %lld given",
                      (long long)need, (long long)workspace_bytes);
     p.ws = reinterpret_cast<float*>(workspace);
-    return nq_check_launch(with_head_dim(D, [&](auto dc) {
-      constexpr int DD = decltype(dc)::value;
-      return causal ? launch_prefill_split<DD, true>(p, st) : launch_prefill_split<DD, false>(p, st);
-    }));
   }
   const hipError_t e =
-      with_head_dim(D, [&](auto dc) { return launch_prefill<decltype(dc)::value, bf16>(p, nw, causal, fuse, st); });
+      with_head_dim(D, [&](auto dc) { return launch_prefill<decltype(dc)::value>(p, nw, causal, fuse, st); });
   return nq_check_launch(e);
 }
 
