@@ -106,6 +106,27 @@ int nq_rmsnorm(const void* x, int64_t x_row_stride, const void* weight, void* y,
                int dtype_y, float eps, void* stream);
 
 /*
+ * Backward of nq_rmsnorm over contiguous rows, width a multiple of 8 up to 4096:
+ * dy in the promoted dtype of x and weight, dx in x's, dweight in the weight's.
+ * dweight's sum is fp32 over per-workgroup partials in the workspace
+ * (nq_rmsnorm_bwd_workspace_bytes; 0 for sizes not taken), in a fixed order.
+ * Base pointers are 16-byte aligned.
+ */
+int64_t nq_rmsnorm_bwd_workspace_bytes(int64_t rows, int width);
+int nq_rmsnorm_bwd(const void* x, const void* dy, const void* weight, void* dx, void* dweight,
+                   void* workspace, int64_t workspace_bytes, int64_t rows, int width, int dtype_x,
+                   int dtype_w, float eps, void* stream);
+
+/*
+ * The product of model/ffn.py:17-28, y = silu(gate) * up, with silu(gate) rounded
+ * to the dtype, and its gradients, over n contiguous elements (a multiple of 8),
+ * all of one dtype, 16-byte aligned.
+ */
+int nq_swiglu(const void* gate, const void* up, void* y, int64_t n, int dtype, void* stream);
+int nq_swiglu_bwd(const void* gate, const void* up, const void* dy, void* dgate, void* dup, int64_t n,
+                  int dtype, void* stream);
+
+/*
  * Causal / full GQA prefill attention (FlashAttention-2 style forward).
  *
  * Replaces kernels/flash_attn.py:130-143 (flash_attention) and the

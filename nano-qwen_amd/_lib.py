@@ -52,6 +52,14 @@ SIGNATURES = {
         _i64, _i32, _i32, _i32, _i32,                # rows, width, dtype_x, dtype_w, dtype_y
         _f32, _p,                                    # eps, stream
     ]),
+    "nq_rmsnorm_bwd_workspace_bytes": (_i64, [_i64, _i32]),
+    "nq_rmsnorm_bwd": (_i32, [
+        _p, _p, _p, _p, _p, _p, _i64,                # x, dy, weight, dx, dweight, workspace, bytes
+        _i64, _i32, _i32, _i32,                      # rows, width, dtype_x, dtype_w
+        _f32, _p,                                    # eps, stream
+    ]),
+    "nq_swiglu": (_i32, [_p, _p, _p, _i64, _i32, _p]),  # gate, up, y, n, dtype, stream
+    "nq_swiglu_bwd": (_i32, [_p, _p, _p, _p, _p, _i64, _i32, _p]),  # gate, up, dy, dgate, dup, n, dtype, stream
     "nq_attn_prefill_fwd": (_i32, [
         _p, _i64p, _p, _i64p, _p, _i64p, _p, _i64p,  # q, k, v, o (+ strides)
         _p, _p,                                      # lse, key_lens

@@ -69,6 +69,46 @@ class _RMSNormFn(torch.autograd.Function):
         return dx.to(x.dtype), dw, None
 
 
+def layer_rms_norm(x: torch.Tensor, weight: torch.Tensor, eps: float) -> torch.Tensor:
+    """The layer norms' arithmetic (model/norm.py:17-22) as tensor operations."""
+    xf = x.float()
+    y = xf * torch.rsqrt(xf.pow(2).mean(-1, keepdim=True) + eps)
+    return y.to(x.dtype) * weight
+
+
+class LayerRMSNormFn(torch.autograd.Function):
+    """``layer_rms_norm`` on the kernels; for tensors that ``ops.plain_rows`` accepts."""
+
+    @staticmethod
+    def forward(ctx, x, weight, eps: float):
+        ctx.save_for_backward(x, weight)
+        ctx.eps = eps
+        return rms_norm(x, weight, eps)
+
+    @staticmethod
+    def backward(ctx, dy):
+        x, weight = ctx.saved_tensors
+        dyc = dy.contiguous()
+        if torch.is_grad_enabled() or not ops.plain_rows(x, weight, dyc):
+            # a gradient of the gradient, or one under a transform: tensor operations
+            xf = x.float()
+            r = torch.rsqrt(xf.pow(2).mean(-1, keepdim=True) + ctx.eps)
+            n = xf * r
+            g = (dy * weight).to(x.dtype).float()
+            dx = (r * (g - n * (g * n).mean(-1, keepdim=True))).to(x.dtype)
+            return dx, (dy * n.to(x.dtype)).reshape(-1, x.shape[-1]).sum(0).to(weight.dtype), None
+        dx, dw = torch.empty_like(x), torch.empty_like(weight)
+        W = x.shape[-1]
+        rows = x.numel() // W
+        lib = _lib.load()
+        ws = torch.empty(lib.nq_rmsnorm_bwd_workspace_bytes(rows, W), dtype=torch.uint8, device=x.device)
+        rc = lib.nq_rmsnorm_bwd(ops._ptr(x), ops._ptr(dyc), ops._ptr(weight), ops._ptr(dx), ops._ptr(dw),
+                                ops._ptr(ws), ws.numel(), rows, W, ops._code(x), ops._code(weight),
+                                float(ctx.eps), ops._stream(x))
+        _lib.check(rc, "nq_rmsnorm_bwd")
+        return dx, dw, None
+
+
 class RMSNorm(nn.Module):
     def __init__(self, hidden_size: int, eps: float = 1e-6):
         super().__init__()

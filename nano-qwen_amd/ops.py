@@ -18,6 +18,7 @@ import ctypes
 from typing import Optional, Tuple
 
 import torch
+import torch.autograd.forward_ad as _forward_ad
 
 from . import _lib
 
@@ -70,6 +71,24 @@ def _aligned(t: torch.Tensor) -> bool:
     if t.stride(-1) != 1:
         return False
     return all((s * es) % 16 == 0 for s in t.stride()[:-1])
+
+
+def plain_rows(*ts: torch.Tensor) -> bool:
+    """Whether a kernel may stand in for tensor operations on these operands: contiguous
+    bf16 or fp32 tensors of the current device, not empty, 16-byte aligned, rows of whole
+    16-byte pieces, outside tracing, compilation, vmap, forward-mode and dispatch modes
+    (which the tensor operations go through)."""
+    if (torch.compiler.is_compiling() or torch.jit.is_tracing() or _forward_ad._current_level >= 0
+            or torch._C._functorch.peek_interpreter_stack() is not None
+            or torch._C._len_torch_dispatch_stack() > 0):
+        return False
+    for t in ts:
+        if (type(t) not in (torch.Tensor, torch.nn.Parameter) or torch._C._functorch.is_legacy_batchedtensor(t)
+                or not t.is_cuda or t.dtype not in _DTYPES
+                or t.layout != torch.strided or not t.is_contiguous() or t.dim() == 0 or t.numel() == 0
+                or t.shape[-1] % 8 or t.data_ptr() % 16):
+            return False
+    return all(t.device == ts[0].device for t in ts) and ts[0].device.index == torch.cuda.current_device()
 
 
 def _rows_in(t: torch.Tensor) -> torch.Tensor:

@@ -1,0 +1,121 @@
+"""The layer RMSNorm and SwiGLU's product on the kernels, against the same formulas
+in 64 bits with the roundings between the steps that the data types give."""
+
+import pytest
+import torch
+import torch.nn.functional as F
+
+from nano_qwen_amd.model import LayerRMSNorm, SwiGLU, _SwiGLUProduct
+from nano_qwen_amd.norm import layer_rms_norm
+from tests.helpers import randn, say
+
+pytestmark = pytest.mark.gpu
+DEV = "cuda"
+BF, F32 = torch.bfloat16, torch.float32
+
+
+def _close(got, want, dtype, terms, what):
+    # 2-norm: a result passes at most two bf16 roundings of 2^-9 beside the ones
+    # restated; fp32 sums of `terms` terms round by about sqrt(terms) 2^-24
+    lim = 2.0 ** -8 if dtype == BF else 8 * terms ** 0.5 * 2.0 ** -24
+    got, want = got.detach().double().cpu(), want.double()
+    err = float((got - want).norm() / want.norm())
+    assert err <= lim, (what, err, lim)
+
+
+# one, some and all of a lane's chunks; rows below, at and above a workgroup's four and the grid's 2048
+@pytest.mark.parametrize("rows,width", [(1, 8), (3, 256), (5, 512), (4, 520), (2049, 1024), (7, 2048), (2600, 2056),
+                                        (2, 4096)])
+@pytest.mark.parametrize("xdt,wdt", [(BF, BF), (BF, F32), (F32, F32), (F32, BF)])
+def test_layer_rmsnorm(rows, width, xdt, wdt):
+    say(f"layer RMSNorm {rows}x{width} {xdt} {wdt}")
+    x = randn(rows, width, seed=11, dtype=xdt)
+    w = (1 + 0.1 * randn(width, seed=12)).to(wdt)
+    norm = LayerRMSNorm(width, input_kept=True).to(DEV, wdt)
+    with torch.no_grad():
+        norm.weight.copy_(w)
+    xd = x.to(DEV).requires_grad_()
+    y = norm(xd)
+    ydt = torch.promote_types(xdt, wdt)
+    assert y.dtype == ydt and y.grad_fn.name().startswith("LayerRMSNormFn")
+    dy = randn(rows, width, seed=13, dtype=ydt)
+    dx, dw = torch.autograd.grad(y, (xd, norm.weight), dy.to(DEV))
+    with torch.no_grad():
+        assert torch.equal(norm(xd), y)
+    x6, w6, d6 = x.double(), w.double(), dy.double()
+    r = torch.rsqrt(x6.square().mean(-1, keepdim=True) + 1e-6)
+    n = x6 * r
+    g = (d6 * w6).to(xdt).double()
+    _close(y, (n.to(xdt).double() * w6), ydt, width, "y")
+    _close(dx, r * (g - n * (g * n).mean(-1, keepdim=True)), xdt, width, "dx")
+    # a bf16 n may round the other way: 2^-8 of a term now and then
+    _close(dw, (d6 * n.to(xdt).double()).sum(0), BF if BF in (xdt, wdt) else F32, rows, "dw")
+    assert dx.dtype == xdt and dw.dtype == wdt
+
+
+def test_layer_rmsnorm_other_routes():
+    """Calls the kernels do not take give what the tensor operations give."""
+    norm = LayerRMSNorm(64, input_kept=True).to(DEV)
+    x = randn(6, 64, seed=21).to(DEV).requires_grad_()
+    # the gradient of the gradient
+    y = norm(x)
+    (gx,) = torch.autograd.grad(y.square().sum(), x, create_graph=True)
+    (ggx,) = torch.autograd.grad(gx.square().sum(), x)
+    z = layer_rms_norm(x, norm.weight, 1e-6)
+    (hx,) = torch.autograd.grad(z.square().sum(), x, create_graph=True)
+    (hhx,) = torch.autograd.grad(hx.square().sum(), x)
+    torch.testing.assert_close(ggx, hhx, rtol=1e-3, atol=1e-5)
+    # vmap, forward mode, a batch of gradients, a width and a layout the kernels do not take
+    torch.testing.assert_close(torch.vmap(norm)(x[None])[0], z)
+    torch.func.jvp(lambda t: layer_rms_norm(t, norm.weight, 1e-6), (x.detach(),), (x.detach(),))
+    torch.func.jvp(norm, (x.detach(),), (x.detach(),))
+    dys = torch.stack([torch.ones_like(y), 2 * torch.ones_like(y)])
+    (b,) = torch.autograd.grad(norm(x), x, dys, is_grads_batched=True)
+    torch.testing.assert_close(b[1], 2 * b[0])
+    odd = LayerRMSNorm(63).to(DEV)
+    assert odd(x[:, :63]).shape == (6, 63) and norm(x[:0]).shape == (0, 64)
+    xt = randn(64, 6, seed=22).to(DEV).t()
+    assert norm(xt).stride() == layer_rms_norm(xt, norm.weight, 1e-6).stride()
+    # without input_kept the input may change before the backward
+    free = LayerRMSNorm(64).to(DEV, BF)
+    h = randn(6, 64, seed=23, dtype=BF).to(DEV).requires_grad_() * 1
+    out = free(h)
+    h.add_(1)
+    out.sum().backward()
+
+
+@pytest.mark.parametrize("shape", [(1, 8), (3, 683, 8), (2, 5, 6144)])
+@pytest.mark.parametrize("dt", [BF, F32])
+def test_swiglu_product(shape, dt):
+    say(f"SwiGLU product {shape} {dt}")
+    g, u, dy = (randn(*shape, seed=31 + i, dtype=dt) * (3 if i == 0 else 1) for i in range(3))
+    gd, ud = g.to(DEV).requires_grad_(), u.to(DEV).requires_grad_()
+    y = _SwiGLUProduct.apply(gd, ud)
+    dg, du = torch.autograd.grad(y, (gd, ud), dy.to(DEV))
+    g6, u6, d6 = g.double(), u.double(), dy.double()
+    s = torch.sigmoid(g6)
+    silu = (g6 * s).to(dt).double()
+    _close(y, silu * u6, dt, 1, "y")
+    _close(du, d6 * silu, dt, 1, "dup")
+    _close(dg, (d6 * u6).to(dt).double() * s * (1 + g6 * (1 - s)), dt, 1, "dgate")
+
+
+def test_swiglu_other_routes():
+    ffn = SwiGLU(64, 128).to(DEV)
+    x = randn(5, 64, seed=41).to(DEV)
+
+    def plain(t):
+        return ffn.down_proj(F.silu(ffn.gate_proj(t)) * ffn.up_proj(t))
+    torch.testing.assert_close(ffn(x), plain(x))
+    torch.testing.assert_close(torch.vmap(ffn)(x[None])[0], plain(x))
+    for f in (ffn, plain):
+        torch.func.jvp(f, (x,), (x,))
+    xs = x.clone().requires_grad_()
+    res = []
+    for f in (ffn, plain):
+        (a,) = torch.autograd.grad(f(xs).square().sum(), xs, create_graph=True)
+        (b,) = torch.autograd.grad(a.square().sum(), xs)
+        res.append(b)
+    torch.testing.assert_close(res[0], res[1], rtol=1e-3, atol=1e-5)
+    gates = torch.tensor([float("inf"), float("-inf"), float("nan"), 0.0, -100.0, 100.0, 1e30, -1e30], device=DEV)
+    torch.testing.assert_close(_SwiGLUProduct.apply(gates, torch.ones_like(gates)), F.silu(gates), equal_nan=True)
