@@ -213,11 +213,11 @@ def load():
         return lib
 
 
+_Strides3 = ctypes.c_int64 * 3
+
+
 def strides3(vals) -> ctypes.Array:
-    arr = (ctypes.c_int64 * 3)()
-    for i, v in enumerate(vals):
-        arr[i] = int(v)
-    return arr
+    return _Strides3(*vals)
 
 
 def check(rc: int, what: str) -> None:

@@ -31,11 +31,23 @@ def rms_norm(x: torch.Tensor, weight: torch.Tensor, eps: float) -> torch.Tensor:
         rows = rows.contiguous()
     w = weight if weight.is_contiguous() else weight.contiguous()
     y = torch.empty(rows.shape, dtype=out_dtype, device=x.device)
-    rc = _lib.load().nq_rmsnorm(ops._ptr(rows), rows.stride(0), ops._ptr(w), ops._ptr(y), y.stride(0),
-                                rows.shape[0], W, ops._code(rows), ops._code(w), ops._code(y), float(eps),
-                                ops._stream(x))
-    _lib.check(rc, "nq_rmsnorm")
+    _rms_norm_into(rows, w, y, float(eps))
     return y.view(x.shape)
+
+
+def _rms_norm_into(x: torch.Tensor, w: torch.Tensor, y: torch.Tensor, eps: float) -> torch.Tensor:
+    """The launch: x and y hold equally spaced rows (all but the last dim are rows), y contiguous."""
+    W = x.shape[-1]
+    rc = _lib.load().nq_rmsnorm(ops._ptr(x), x.stride(0) if x.dim() == 2 else W, ops._ptr(w), ops._ptr(y), W,
+                                x.numel() // W, W, ops._code(x), ops._code(w), ops._code(y), eps, ops._stream(x))
+    _lib.check(rc, "nq_rmsnorm")
+    return y
+
+
+def plain_rms_norm(x: torch.Tensor, weight: torch.Tensor, eps: float) -> torch.Tensor:
+    """``rms_norm`` of tensors that ``ops.plain_rows`` accepts."""
+    y = torch.empty(x.shape, dtype=torch.promote_types(x.dtype, weight.dtype), device=x.device)
+    return _rms_norm_into(x, weight, y, eps)
 
 
 class _RMSNormFn(torch.autograd.Function):
@@ -83,7 +95,7 @@ class LayerRMSNormFn(torch.autograd.Function):
     def forward(ctx, x, weight, eps: float):
         ctx.save_for_backward(x, weight)
         ctx.eps = eps
-        return rms_norm(x, weight, eps)
+        return plain_rms_norm(x, weight, eps)
 
     @staticmethod
     def backward(ctx, dy):
