@@ -37,6 +37,7 @@
 #include "nq_backward.hpp"
 #include "nq_common.hpp"
 #include "nq_internal.hpp"
+#include "nq_prefill.hpp"
 
 namespace nq {
 
@@ -839,9 +840,17 @@ extern "C" int64_t nq_attn_bwd_split_workspace_bytes(int B, int Hq, int Hkv, int
   const int64_t base = nq_attn_bwd_workspace_bytes(B, Hq, S);
   if (base == 0 || Hkv <= 0 || T <= 0 || Hq % Hkv || !head_dim_ok(D) || !nq_dtype_ok(dtype)) return base;
   const DkdvSplit sp = dkdv_split(B, Hq, Hkv, S, T, D, dtype, causal != 0);
-  if (sp.nsplit == 1) return base;
   const int64_t nkb = (T + BW_KEYS - 1) / BW_KEYS;
-  return base + nkb * B * Hkv * sp.nsplit * (BW_KEYS * 2 * (int64_t)D * (int64_t)sizeof(float));
+  int64_t part = sp.nsplit > 1 ? nkb * B * Hkv * sp.nsplit * (BW_KEYS * 2 * (int64_t)D) : 0;
+  if (dtype == NQ_DTYPE_F32) {  // dQ's partials, in the same memory before dK/dV's
+    const KeyRuns kr = f32_key_runs(B, Hq, Hkv, S, T);
+    if (kr.n > 1) {
+      const int BM = 128 / (Hq / Hkv);
+      const int64_t dq = (int64_t)B * Hkv * ((S + BM - 1) / BM) * kr.n * f32_part(D);
+      if (dq > part) part = dq;
+    }
+  }
+  return base + part * (int64_t)sizeof(float);
 }
 
 // Shared by nq_attn_bwd and nq_attn_bwd_bias (bias == NULL: none).
@@ -932,14 +941,19 @@ static int bwd_entry(const void* q, const int64_t* q_strides, const void* k, con
   p.scale = sm_scale > 0.f ? sm_scale : 1.0f / sqrtf((float)D);
   p.scale_log2 = p.scale * kLog2e;
   hipStream_t st = reinterpret_cast<hipStream_t>(stream);
-  p.nsplit = p.run = 1;
+  p.nsplit = p.run = p.qsplit = p.qrun = 1;
   if (!wide && !bias && nq_aligned16(workspace) &&
       workspace_bytes >= nq_attn_bwd_split_workspace_bytes(B, Hq, Hkv, S, T, D, dtype, causal)) {
     const DkdvSplit sp = dkdv_split(B, Hq, Hkv, S, T, D, dtype, causal != 0);
     if ((int64_t)((T + BW_KEYS - 1) / BW_KEYS) * B * Hkv * sp.nsplit < (1LL << 29)) {
       p.nsplit = sp.nsplit;
       p.run = sp.run;
-      p.part = p.ws + need / (int64_t)sizeof(float);  // need is a multiple of 256
+    }
+    p.part = p.ws + need / (int64_t)sizeof(float);  // need is a multiple of 256
+    if (f32) {
+      const KeyRuns kr = f32_key_runs(B, Hq, Hkv, S, T);
+      p.qsplit = kr.n;
+      p.qrun = kr.len;
     }
   }
   if (wide) {

@@ -40,6 +40,9 @@ struct BwdParams {
   // each (1 = none), whose partial sums go to part
   int nsplit, run;
   float* part;
+  // fp32 dQ: a query block's key tiles split likewise (f32_key_runs), whose
+  // partials use the same memory before it
+  int qsplit, qrun;
 };
 
 // Keys sequence b attends.

@@ -27,6 +27,7 @@
 #include "nq_backward.hpp"
 #include "nq_common.hpp"
 #include "nq_internal.hpp"
+#include "nq_prefill.hpp"
 
 namespace nq {
 
@@ -75,7 +76,9 @@ struct TileCopy {
 // ---------------------------------------------------------------------------
 // BIAS: the forward's additive bias (p.bias) enters every score; a row the
 // bias masks entirely has LSE -inf and P = 0 (its scratch LSE is stored +inf).
-template <int D, bool CAUSAL, bool BIAS = false>
+// SPLIT: a block's key tiles in runs of p.qrun; a block of several leaves its
+// partial dQ for bwd_dq_f32_merge_kernel, its first run writes Delta and the LSE.
+template <int D, bool CAUSAL, bool BIAS = false, bool SPLIT = false>
 __global__ void __launch_bounds__(64 * BF32_NW) bwd_dq_f32_kernel(BwdParams p) {
   using L = BwF32<D>;
   constexpr int NT = D / 2, NDO = D / 32;
@@ -85,18 +88,21 @@ __global__ void __launch_bounds__(64 * BF32_NW) bwd_dq_f32_kernel(BwdParams p) {
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   const int r32 = lane & 31, hh = lane >> 5;
   const int npairs = p.B * p.Hkv;
-  const int pair = blockIdx.x % npairs, qrank = blockIdx.x / npairs;
+  const int pair = blockIdx.x % npairs, split = SPLIT ? blockIdx.x / npairs % p.qsplit : 0;
+  const int qrank = blockIdx.x / npairs / (SPLIT ? p.qsplit : 1);
   const int qblk = CAUSAL ? (p.nqb - 1 - qrank) : qrank;
   const int b = pair / p.Hkv, kvh = pair % p.Hkv;
   const int q0 = qblk * p.BM;
   const int Tk = bw_keys(p, b);  // keys this sequence attends
   const int kv_end = CAUSAL ? min(Tk, q0 + p.BM + p.coff) : Tk;
   const int ntiles = (kv_end + BF32_TILE - 1) / BF32_TILE;
+  const int jbeg = SPLIT ? split * p.qrun : 0, jend = SPLIT ? min(ntiles, jbeg + p.qrun) : ntiles;
+  if (SPLIT && split > 0 && jbeg >= ntiles) return;
   const float* kbase = reinterpret_cast<const float*>(p.k) + b * p.ksb + kvh * p.ksh;
   const float* vbase = reinterpret_cast<const float*>(p.v) + b * p.vsb + kvh * p.vsh;
   TileCopy<D> kc, vc;  // rows past the sequence's keys read as zeros (padding is never read)
-  kc.fetch(kbase, p.kss, 0, Tk);
-  vc.fetch(vbase, p.vss, 0, Tk);
+  kc.fetch(kbase, p.kss, jbeg * BF32_TILE, Tk);
+  vc.fetch(vbase, p.vss, jbeg * BF32_TILE, Tk);
 
   const int R = wave * 32 + r32;
   const int g = R / p.BM, pr = R - g * p.BM;
@@ -130,7 +136,7 @@ __global__ void __launch_bounds__(64 * BF32_NW) bwd_dq_f32_kernel(BwdParams p) {
   }
   float lse2 = p.lse[((int64_t)b * p.Hq + head) * p.S + qi_c] * kLog2e;
   if (BIAS && !(lse2 > -INFINITY)) lse2 = INFINITY;  // no key kept: P = exp2(s - inf) = 0
-  if (qvalid && hh == 0) {
+  if (split == 0 && qvalid && hh == 0) {
     const int64_t wi = bw_ws_index(p, b, head, qi);
     p.ws[wi] = lse2;
     p.ws[wi + 32] = dlt;
@@ -138,7 +144,7 @@ __global__ void __launch_bounds__(64 * BF32_NW) bwd_dq_f32_kernel(BwdParams p) {
   const float* brow = BIAS ? reinterpret_cast<const float*>(p.bias) + b * p.bsb + head * p.bsh +
                                  (int64_t)qi_c * p.bss
                            : nullptr;
-  if (qblk == p.nqb - 1) {  // scratch slots past S: zero
+  if (split == 0 && qblk == p.nqb - 1) {  // scratch slots past S: zero
     const int pad = p.nst * 32 - p.S;
     for (int t = threadIdx.x; t < p.G * 32; t += 64 * BF32_NW) {
       if (t % 32 < pad) {
@@ -152,12 +158,12 @@ __global__ void __launch_bounds__(64 * BF32_NW) bwd_dq_f32_kernel(BwdParams p) {
   floatx16 dqacc[NDO];
 #pragma unroll
   for (int dd = 0; dd < NDO; ++dd) dqacc[dd] = floatx16{};
-  for (int j = 0; j < ntiles; ++j) {
+  for (int j = jbeg; j < jend; ++j) {
     __syncthreads();
     kc.stash(kt);
     vc.stash(vt);
     __syncthreads();
-    if (j + 1 < ntiles) {
+    if (j + 1 < jend) {
       kc.fetch(kbase, p.kss, (j + 1) * BF32_TILE, Tk);
       vc.fetch(vbase, p.vss, (j + 1) * BF32_TILE, Tk);
     }
@@ -202,6 +208,17 @@ __global__ void __launch_bounds__(64 * BF32_NW) bwd_dq_f32_kernel(BwdParams p) {
         dqacc[dd] = mfma_f32x2(L::at(kt, key, dd * 32 + r32), ds[t], dqacc[dd]);
     }
   }
+  if (SPLIT && ntiles > p.qrun) {  // in the accumulators' lane order
+    const int64_t slot = (((int64_t)qblk * npairs + pair) * p.qsplit + split) * BF32_NW + wave;
+    floatx4* po = reinterpret_cast<floatx4*>(p.part) + slot * (NDO * 256) + lane;
+#pragma unroll
+    for (int dd = 0; dd < NDO; ++dd)
+#pragma unroll
+      for (int gq = 0; gq < 4; ++gq)
+        po[(dd * 4 + gq) * 64] = floatx4{dqacc[dd][gq * 4 + 0], dqacc[dd][gq * 4 + 1], dqacc[dd][gq * 4 + 2],
+                                         dqacc[dd][gq * 4 + 3]};
+    return;
+  }
   if (!qvalid) return;
   float* dqrow = reinterpret_cast<float*>(p.dq) + b * p.dqsb + head * p.dqsh + (int64_t)qi * p.dqss;
 #pragma unroll
@@ -212,6 +229,38 @@ __global__ void __launch_bounds__(64 * BF32_NW) bwd_dq_f32_kernel(BwdParams p) {
                          dqacc[dd][gq * 4 + 2] * p.scale, dqacc[dd][gq * 4 + 3] * p.scale};
       *reinterpret_cast<floatx4*>(dqrow + dd * 32 + gq * 8 + hh * 4) = t;
     }
+}
+
+// Adds the partial dQ of the blocks with several runs, in run order: a workgroup
+// takes the 32 rows of one wave, its wave dd their dims 32dd .. 32dd + 31.
+template <int D, bool CAUSAL>
+__global__ void __launch_bounds__(2 * D) bwd_dq_f32_merge_kernel(BwdParams p) {
+  constexpr int NDO = D / 32;
+  const int lane = threadIdx.x & 63, dd = threadIdx.x >> 6;
+  const int npairs = p.B * p.Hkv;
+  const int wave = blockIdx.x % BF32_NW, wg = blockIdx.x / BF32_NW;
+  const int qblk = wg / npairs, pair = wg % npairs;
+  const int b = pair / p.Hkv, kvh = pair % p.Hkv;
+  const int q0 = qblk * p.BM;
+  const int Tk = bw_keys(p, b);
+  const int ntiles = ((CAUSAL ? min(Tk, q0 + p.BM + p.coff) : Tk) + BF32_TILE - 1) / BF32_TILE;
+  if (ntiles <= p.qrun) return;
+  const int runs = (ntiles + p.qrun - 1) / p.qrun;
+  const int R = wave * 32 + (lane & 31);
+  const int g = R / p.BM, qi = q0 + R - g * p.BM;
+  const floatx4* po = reinterpret_cast<const floatx4*>(p.part) +
+                      ((int64_t)wg * p.qsplit * BF32_NW + wave) * (NDO * 256) + dd * 256 + lane;
+  floatx4 a[4] = {floatx4{}, floatx4{}, floatx4{}, floatx4{}};
+#pragma unroll 4
+  for (int s = 0; s < runs; ++s) {
+#pragma unroll
+    for (int gq = 0; gq < 4; ++gq) a[gq] += po[(int64_t)s * (BF32_NW * NDO * 256) + gq * 64];
+  }
+  if (qi >= p.S) return;
+  float* dq = reinterpret_cast<float*>(p.dq) + b * p.dqsb + (kvh * p.G + g) * p.dqsh + (int64_t)qi * p.dqss +
+              dd * 32 + (lane >> 5) * 4;
+#pragma unroll
+  for (int gq = 0; gq < 4; ++gq) *reinterpret_cast<floatx4*>(dq + gq * 8) = a[gq] * p.scale;
 }
 
 // ---------------------------------------------------------------------------
@@ -380,13 +429,23 @@ static hipError_t launch_f32(const BwdParams& p, bool causal, hipStream_t st) {
     }
     return hipGetLastError();
   }
-  const dim3 gs(gk.x * p.nsplit);
-  if (causal) {
+  const dim3 gs(gk.x * p.nsplit), gqs(gq.x * p.qsplit), gqm(gq.x * BF32_NW), bqm(2 * D);
+  if (p.qsplit > 1) {
+    if (causal) hipLaunchKernelGGL((bwd_dq_f32_kernel<D, true, false, true>), gqs, block, 0, st, p);
+    else hipLaunchKernelGGL((bwd_dq_f32_kernel<D, false, false, true>), gqs, block, 0, st, p);
+    const hipError_t e = hipGetLastError();
+    if (e != hipSuccess) return e;
+    if (causal) hipLaunchKernelGGL((bwd_dq_f32_merge_kernel<D, true>), gqm, bqm, 0, st, p);
+    else hipLaunchKernelGGL((bwd_dq_f32_merge_kernel<D, false>), gqm, bqm, 0, st, p);
+  } else if (causal) {
     hipLaunchKernelGGL((bwd_dq_f32_kernel<D, true>), gq, block, 0, st, p);
+  } else {
+    hipLaunchKernelGGL((bwd_dq_f32_kernel<D, false>), gq, block, 0, st, p);
+  }
+  if (causal) {
     if (p.nsplit > 1) hipLaunchKernelGGL((bwd_dkdv_f32_kernel<D, true, false, true>), gs, block, 0, st, p);
     else hipLaunchKernelGGL((bwd_dkdv_f32_kernel<D, true>), gk, block, 0, st, p);
   } else {
-    hipLaunchKernelGGL((bwd_dq_f32_kernel<D, false>), gq, block, 0, st, p);
     if (p.nsplit > 1) hipLaunchKernelGGL((bwd_dkdv_f32_kernel<D, false, false, true>), gs, block, 0, st, p);
     else hipLaunchKernelGGL((bwd_dkdv_f32_kernel<D, false>), gk, block, 0, st, p);
   }

@@ -1009,6 +1009,16 @@ static int prefill_entry(const void* q, const int64_t* q_strides, const void* k,
   if (f32) {
     p.BM = 128 / G;
     p.nqb = (S + p.BM - 1) / p.BM;
+    const KeyRuns kr = workspace && !key_lens && !bias ? f32_key_runs(B, Hq, Hkv, S, T) : KeyRuns{1, 1};
+    p.nsplit = kr.n;
+    p.run = kr.len;
+    if (p.nsplit > 1) {
+      const int64_t need = nq_attn_prefill_workspace_bytes(B, Hq, Hkv, S, T, D, NQ_DTYPE_F32);
+      if (workspace_bytes < need || !nq_aligned16(workspace))
+        return nq_fail(NQ_ERR_WORKSPACE, "workspace of %lld bytes (16-byte aligned) required, %lld given",
+                       (long long)need, (long long)workspace_bytes);
+      p.ws = reinterpret_cast<float*>(workspace);
+    }
     return nq_check_launch(launch_prefill_f32(p, D, causal != 0, fuse, st));
   }
   // 256 rows per workgroup when that still gives enough workgroups, else 128
@@ -1032,8 +1042,12 @@ static int prefill_entry(const void* q, const int64_t* q_strides, const void* k,
 }
 
 extern "C" int64_t nq_attn_prefill_workspace_bytes(int B, int Hq, int Hkv, int S, int T, int D, int dtype) {
-  if (B <= 0 || Hq <= 0 || Hkv <= 0 || S <= 0 || T <= 0 || Hq % Hkv || !head_dim_ok(D) || dtype != NQ_DTYPE_BF16)
+  if (B <= 0 || Hq <= 0 || Hkv <= 0 || S <= 0 || T <= 0 || Hq % Hkv || !head_dim_ok(D) || !nq_dtype_ok(dtype))
     return 0;
+  if (dtype == NQ_DTYPE_F32) {
+    const KeyRuns kr = f32_key_runs(B, Hq, Hkv, S, T);  // 128 rows' accumulators, max and sum per workgroup
+    return kr.n > 1 ? prefill_wgs4(B, Hq, Hkv, S) * kr.n * (f32_part(D) + 256) * (int64_t)sizeof(float) : 0;
+  }
   const int ns = prefill_splits(B, Hq, Hkv, S, T);
   return ns > 1 ? pf_split_bytes(prefill_wgs4(B, Hq, Hkv, S), ns, D) : 0;
 }

@@ -50,7 +50,31 @@ struct PrefillParams {
   // whose partials go to ws
   int nsplit;
   float* ws;
+  int run;  // fp32 form: tiles per workgroup of a split launch
 };
+
+// How the fp32 kernels that own query rows (the prefill, the backward's dQ)
+// deal a query block's 32-key tiles to workgroups: runs of `len` tiles, `n` for
+// the longest block, n = 1 for none.  A launch of fewer workgroups than two per
+// CU leaves the device to its heaviest blocks (B2 S1000 8/2 heads D64: 128
+// workgroups of 1 to 32 tiles, ~2 us a tile): runs of the length that gives two
+// workgroups per CU the same work, at least F32_MIN_RUN tiles, at most
+// F32_MAX_RUNS of them, whose partials the merge adds one after another.
+constexpr int F32_MIN_RUN = 4, F32_MAX_RUNS = 32;
+struct KeyRuns { int n, len; };
+inline KeyRuns f32_key_runs(int B, int Hq, int Hkv, int S, int T) {
+  if (128 % (Hq / Hkv)) return {1, 1};
+  const int BM = 128 / (Hq / Hkv);
+  const int64_t wgs = (int64_t)B * Hkv * ((S + BM - 1) / BM);
+  const int64_t most = ((int64_t)T + 31) / 32;
+  if (wgs >= 512) return {1, 1};
+  int64_t len = (wgs * ((int64_t)T - (S < T ? S : T) / 2) / 32 + 511) / 512;  // a causal row's keys on average
+  if (len < F32_MIN_RUN) len = F32_MIN_RUN;
+  if (len * F32_MAX_RUNS < most) len = (most + F32_MAX_RUNS - 1) / F32_MAX_RUNS;
+  return {(int)((most + len - 1) / len), (int)len};
+}
+// Floats of one workgroup's partial accumulators, 4 waves of 32 rows.
+constexpr int64_t f32_part(int D) { return 128 * (int64_t)D; }
 
 // Keys of sequence b (-1: a length out of range).
 __device__ __forceinline__ int pf_keys(const PrefillParams& p, int b) {

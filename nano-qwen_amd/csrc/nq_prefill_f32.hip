@@ -41,9 +41,18 @@ struct F32Tile {
   __device__ static int vswz(int r) { return CPR >= 16 ? (((r >> 2) & 1) << 3) : 0; }
 };
 
+// (max, sum) of the rows of a split launch's partials, after the accumulators.
+template <int D>
+__device__ __forceinline__ floatx2* f32_max_sum(const PrefillParams& p) {
+  return reinterpret_cast<floatx2*>(p.ws + (int64_t)p.nqb * p.B * p.Hkv * p.nsplit * f32_part(D));
+}
+
 // BIAS: p.bias (fp32) is added to every score; a row may then see no finite
 // score in a tile, or in any (zeros out, LSE -inf, as SDPA gives).
-template <int D, bool CAUSAL, bool FUSE_Q, bool BIAS = false>
+// SPLIT: a block's tiles in runs of p.run (f32_key_runs).  A row may see no key of
+// a run; a block of several runs leaves O, row max and row sum in the workspace
+// for prefill_f32_merge_kernel.
+template <int D, bool CAUSAL, bool FUSE_Q, bool BIAS = false, bool SPLIT = false>
 __global__ void __launch_bounds__(64 * PF32_NW) prefill_f32_kernel(PrefillParams p) {
   using Tl = F32Tile<D>;
   constexpr int CPR = Tl::CPR;
@@ -61,7 +70,8 @@ __global__ void __launch_bounds__(64 * PF32_NW) prefill_f32_kernel(PrefillParams
 
   const int npairs = p.B * p.Hkv;
   const int L = blockIdx.x;
-  const int pair = L % npairs, qrank = L / npairs;
+  const int pair = L % npairs, split = SPLIT ? L / npairs % p.nsplit : 0;
+  const int qrank = L / npairs / (SPLIT ? p.nsplit : 1);
   const int qblk = CAUSAL ? (p.nqb - 1 - qrank) : qrank;  // heaviest first
   const int b = pair / p.Hkv, kvh = pair % p.Hkv;
   const int q0 = qblk * p.BM;
@@ -73,6 +83,8 @@ __global__ void __launch_bounds__(64 * PF32_NW) prefill_f32_kernel(PrefillParams
   const int coff = p.T - p.S;
   const int kv_end = max(0, CAUSAL ? min(T, q0 + p.BM + coff) : T);
   const int ntiles = (kv_end + PF32_BN - 1) / PF32_BN;
+  const int jbeg = SPLIT ? split * p.run : 0, jend = SPLIT ? min(ntiles, jbeg + p.run) : ntiles;
+  if (SPLIT && jbeg >= ntiles) return;  // (ntiles > 0: no key counts in a split launch)
 
   // row `key` of this (batch, kv head): dense strides, or through the block table
   auto krow = [&](const void* base, int64_t sb, int64_t sh, int64_t ss, int key) {
@@ -106,7 +118,7 @@ __global__ void __launch_bounds__(64 * PF32_NW) prefill_f32_kernel(PrefillParams
       vt[row * CPR + (c ^ Tl::vswz(row))] = vr[u];
     }
   };
-  if (ntiles > 0) fetch(0);
+  if (jbeg < jend) fetch(jbeg);
 
   // this lane's query row: column r32 of this wave's 32 rows
   const int R = wave * 32 + r32;
@@ -164,11 +176,11 @@ __global__ void __launch_bounds__(64 * PF32_NW) prefill_f32_kernel(PrefillParams
 #pragma unroll
   for (int dd = 0; dd < NDO; ++dd) oacc[dd] = floatx16{};
 
-  for (int j = 0; j < ntiles; ++j) {
+  for (int j = jbeg; j < jend; ++j) {
     __syncthreads();  // every wave is done with the previous tile
     stash();
     __syncthreads();
-    if (j + 1 < ntiles) fetch(j + 1);
+    if (j + 1 < jend) fetch(j + 1);
 
     // S^T = K Q^T for this tile's 32 keys (MFMA row = key r32)
     floatx16 s = floatx16{};
@@ -200,13 +212,14 @@ __global__ void __launch_bounds__(64 * PF32_NW) prefill_f32_kernel(PrefillParams
     }
 
     // online softmax in the log2 domain (tile 0 holds key 0 for every row,
-    // so m_i is finite from the first tile on, unless a bias masks it: a row
-    // with no finite score yet keeps m_i = -inf and exponentiates against 0)
+    // so m_i is finite from the first tile on, unless a bias masks it or the run
+    // starts later: a row with no finite score yet keeps m_i = -inf and
+    // exponentiates against 0)
     float mx = -INFINITY;
 #pragma unroll
     for (int i = 0; i < 16; ++i) mx = fmaxf(mx, s[i]);
     const float m_new = fmaxf(m_i, xor32_max(mx) * (BIAS ? 1.f : p.scale_log2));
-    const float m_use = (BIAS && !(m_new > -INFINITY)) ? 0.f : m_new;
+    const float m_use = ((BIAS || SPLIT) && !(m_new > -INFINITY)) ? 0.f : m_new;
     const float alpha = fast_exp2(m_i - m_use);
     l_i *= alpha;
 #pragma unroll
@@ -216,7 +229,7 @@ __global__ void __launch_bounds__(64 * PF32_NW) prefill_f32_kernel(PrefillParams
     float ls = 0.f;
 #pragma unroll
     for (int i = 0; i < 16; ++i) {
-      pv[i] = BIAS ? fast_exp2(s[i] - m_use) : fast_exp2(s[i] * p.scale_log2 - m_i);
+      pv[i] = BIAS ? fast_exp2(s[i] - m_use) : fast_exp2(s[i] * p.scale_log2 - m_use);
       ls += pv[i];
     }
     l_i += ls;
@@ -235,6 +248,18 @@ __global__ void __launch_bounds__(64 * PF32_NW) prefill_f32_kernel(PrefillParams
   }
 
   l_i = xor32_sum(l_i);
+  if (SPLIT && ntiles > p.run) {  // in the accumulators' lane order
+    const int64_t slot = (((int64_t)qblk * npairs + pair) * p.nsplit + split) * PF32_NW + wave;
+    floatx4* po = reinterpret_cast<floatx4*>(p.ws) + slot * (NDO * 256) + lane;
+#pragma unroll
+    for (int dd = 0; dd < NDO; ++dd)
+#pragma unroll
+      for (int gq = 0; gq < 4; ++gq)
+        po[(dd * 4 + gq) * 64] = floatx4{oacc[dd][gq * 4 + 0], oacc[dd][gq * 4 + 1], oacc[dd][gq * 4 + 2],
+                                         oacc[dd][gq * 4 + 3]};
+    if (hh == 0) f32_max_sum<D>(p)[slot * 32 + r32] = floatx2{m_i, l_i};
+    return;
+  }
   if (!qvalid) return;
   float* orow = reinterpret_cast<float*>(p.o) + b * p.osb + head * p.osh + (int64_t)qi * p.oss;
   if (kv_end == 0) {  // no keys: zeros; a length out of range: NaN
@@ -261,6 +286,50 @@ __global__ void __launch_bounds__(64 * PF32_NW) prefill_f32_kernel(PrefillParams
     p.lse[((int64_t)b * p.Hq + head) * p.S + qi] = none ? -INFINITY : (m_i + __log2f(l_i)) * kLn2;
 }
 
+// Adds the partials of the blocks with several runs: a workgroup takes the 32 rows
+// of one wave, its wave dd their dims 32dd .. 32dd + 31.  Reads each partial once,
+// HBM- or L2-bound.
+template <int D, bool CAUSAL>
+__global__ void __launch_bounds__(2 * D) prefill_f32_merge_kernel(PrefillParams p) {
+  constexpr int NDO = D / 32;
+  const int lane = threadIdx.x & 63, dd = threadIdx.x >> 6;
+  const int r32 = lane & 31, hh = lane >> 5;
+  const int npairs = p.B * p.Hkv;
+  const int wave = blockIdx.x % PF32_NW, wg = blockIdx.x / PF32_NW;
+  const int qblk = wg / npairs, pair = wg % npairs;
+  const int b = pair / p.Hkv, kvh = pair % p.Hkv;
+  const int q0 = qblk * p.BM;
+  const int kv_end = CAUSAL ? min(p.T, q0 + p.BM + p.T - p.S) : p.T;
+  const int ntiles = (kv_end + PF32_BN - 1) / PF32_BN;
+  if (ntiles <= p.run) return;
+  const int runs = (ntiles + p.run - 1) / p.run;
+  const int R = wave * 32 + r32;
+  const int g = R / p.BM, qi = q0 + R - g * p.BM;
+  const int64_t slot = ((int64_t)wg * p.nsplit) * PF32_NW + wave;
+  const floatx2* ml = f32_max_sum<D>(p) + slot * 32 + r32;
+  const floatx4* po = reinterpret_cast<const floatx4*>(p.ws) + slot * (NDO * 256) + dd * 256 + lane;
+  float M = -INFINITY;
+#pragma unroll 4
+  for (int s = 0; s < runs; ++s) M = fmaxf(M, ml[s * (PF32_NW * 32)][0]);
+  float l = 0.f;
+  floatx4 o[4] = {floatx4{}, floatx4{}, floatx4{}, floatx4{}};
+#pragma unroll 4
+  for (int s = 0; s < runs; ++s) {
+    const floatx2 m_l = ml[s * (PF32_NW * 32)];
+    const float w = fast_exp2(m_l[0] - M);
+    l = __builtin_fmaf(m_l[1], w, l);
+#pragma unroll
+    for (int gq = 0; gq < 4; ++gq) o[gq] += po[(int64_t)s * (PF32_NW * NDO * 256) + gq * 64] * w;
+  }
+  if (qi >= p.S) return;
+  const int head = kvh * p.G + g;
+  const float inv_l = 1.f / l;
+  float* orow = reinterpret_cast<float*>(p.o) + b * p.osb + head * p.osh + (int64_t)qi * p.oss + dd * 32 + hh * 4;
+#pragma unroll
+  for (int gq = 0; gq < 4; ++gq) *reinterpret_cast<floatx4*>(orow + gq * 8) = o[gq] * inv_l;
+  if (p.lse && dd == 0 && hh == 0) p.lse[((int64_t)b * p.Hq + head) * p.S + qi] = (M + __log2f(l)) * kLn2;
+}
+
 template <int D>
 static hipError_t launch_f32(const PrefillParams& p, bool causal, bool fuse, hipStream_t st) {
   dim3 grid((unsigned)(p.nqb * p.B * p.Hkv));
@@ -268,6 +337,21 @@ static hipError_t launch_f32(const PrefillParams& p, bool causal, bool fuse, hip
   if (p.bias) {
     if (causal) hipLaunchKernelGGL((prefill_f32_kernel<D, true, true, true>), grid, block, 0, st, p);
     else hipLaunchKernelGGL((prefill_f32_kernel<D, false, true, true>), grid, block, 0, st, p);
+    return hipGetLastError();
+  }
+  if (p.nsplit > 1) {
+    const dim3 gs(grid.x * p.nsplit), gm(grid.x * PF32_NW), bm(2 * D);
+    if (causal) {
+      if (fuse) hipLaunchKernelGGL((prefill_f32_kernel<D, true, true, false, true>), gs, block, 0, st, p);
+      else hipLaunchKernelGGL((prefill_f32_kernel<D, true, false, false, true>), gs, block, 0, st, p);
+    } else {
+      if (fuse) hipLaunchKernelGGL((prefill_f32_kernel<D, false, true, false, true>), gs, block, 0, st, p);
+      else hipLaunchKernelGGL((prefill_f32_kernel<D, false, false, false, true>), gs, block, 0, st, p);
+    }
+    const hipError_t e = hipGetLastError();
+    if (e != hipSuccess) return e;
+    if (causal) hipLaunchKernelGGL((prefill_f32_merge_kernel<D, true>), gm, bm, 0, st, p);
+    else hipLaunchKernelGGL((prefill_f32_merge_kernel<D, false>), gm, bm, 0, st, p);
     return hipGetLastError();
   }
   if (causal) {

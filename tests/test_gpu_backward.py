@@ -439,13 +439,15 @@ def test_split_dkdv_backward(Hq, Hkv, D, S, T, causal, dtype):
     # the order of fp32 additions is all that differs
     ws = torch.empty(base, dtype=torch.uint8, device=DEV)
     whole = ops.attention_backward(dv(q), dv(k), dv(v), o, dv(do), lse, causal=causal, workspace=ws)
-    assert torch.equal(split[0], whole[0])
-    for a, b in zip(split[1:], whole[1:]):
+    if dtype == torch.bfloat16:  # the fp32 dQ splits its keys too
+        assert torch.equal(split[0], whole[0])
+    for a, b in zip(split, whole):
         _close_rel(a, b, "split against whole", dtype)
     # key padding: blocks of padding alone have no steps and zero gradients
     o, lse = ops.attention_prefill(dv(q), dv(k), dv(v), causal=causal, key_lens=dv(lens), return_lse=True)
     split = ops.attention_backward(dv(q), dv(k), dv(v), o, dv(do), lse, causal=causal, key_lens=dv(lens))
     whole = ops.attention_backward(dv(q), dv(k), dv(v), o, dv(do), lse, causal=causal, key_lens=dv(lens), workspace=ws)
+    _close_rel(split[0], whole[0], "padded split dq against whole", dtype)
     for a, b in zip(split[1:], whole[1:]):
         _close_rel(a, b, "padded split against whole", dtype)
         assert not a[:, :, int(lens[0]):].any()

@@ -399,3 +399,43 @@ def test_split_keys_prefill(Hq, Hkv, D, S, T, causal, paged):
     # scores carry Q-hat's bf16 rounding: 2^-9 relative over D products of unit
     # variance, so a row's LSE moves by a few 2^-9 at most
     torch.testing.assert_close(lse.cpu().double(), torch.logsumexp(sc, -1).view(1, Hq, S), rtol=0, atol=2e-2)
+
+
+@pytest.mark.parametrize("fused", [False, True])
+@pytest.mark.parametrize("causal", [True, False])
+@pytest.mark.parametrize("Hq,Hkv,D,S,T", [
+    (8, 2, 64, 1, 129),        # one query row, five tiles: a run of four and one of a single key
+    (8, 2, 64, 545, 545),      # blocks of one run beside blocks of many; a last block of one position
+    (2, 2, 128, 129, 1664),    # 128 positions a block: rows that see no key of the last run
+    (32, 1, 32, 70, 12345),    # 4 positions a block, the most runs
+])
+def test_split_keys_prefill_f32(Hq, Hkv, D, S, T, causal, fused):
+    """fp32 launches of few query blocks split their keys into runs of tiles; paged reads give the same bits."""
+    say(f"split fp32 prefill Hq={Hq} Hkv={Hkv} D={D} S={S} T={T} causal={causal} fused={fused}")
+    assert ops._lib.load().nq_attn_prefill_workspace_bytes(1, Hq, Hkv, S, T, D, 1) > 0
+    q, k, v = randn(1, Hq, S, D, seed=411), randn(1, Hkv, T, D, seed=412), randn(1, Hkv, T, D, seed=413)
+    w = 1 + 0.02 * randn(D, seed=414)
+    cos, sin = rope_tables(D, T, 1e6)
+    args = dict(causal=causal, return_lse=True)
+    qh = q.double()
+    if fused:
+        args.update(q_weight=w.to(DEV), eps=1e-6, cos=cos.to(DEV), sin=sin.to(DEV), pos_offset=T - S)
+        qh = rotate_half(rms_norm(q.double(), w.double(), 1e-6, compute_dtype=torch.float64),
+                         cos.double()[T - S:], sin.double()[T - S:])
+    o, lse = ops.attention_prefill(q.to(DEV), k.to(DEV), v.to(DEV), **args)
+    sc = qh.view(1, Hkv, -1, S, D) @ k.double()[:, :, None].transpose(-1, -2) / D ** 0.5
+    if causal:
+        sc = sc.masked_fill(torch.arange(T) > torch.arange(S)[:, None] + T - S, float("-inf"))
+    ref = (torch.softmax(sc, -1) @ v.double()[:, :, None]).view(1, Hq, S, D)
+    torch.testing.assert_close(o.cpu().double(), ref, rtol=0, atol=1e-5)
+    torch.testing.assert_close(lse.cpu().double(), torch.logsumexp(sc, -1).view(1, Hq, S), rtol=0, atol=1e-5)
+    P = 96
+    n = -(-T // P)
+    kp, vp = (torch.full((n + 1, Hkv, P, D), float("nan"), device=DEV) for _ in range(2))
+    bt = torch.randperm(n + 1, generator=torch.Generator().manual_seed(415))[:n].to(torch.int32)
+    for src, pool in ((k, kp), (v, vp)):
+        for i in range(n):
+            rows = src[0, :, i * P:(i + 1) * P].to(DEV)
+            pool[int(bt[i]), :, :rows.shape[1]] = rows
+    po, plse = ops.attention_prefill_paged(q.to(DEV), kp, vp, bt.view(1, n).to(DEV), T=T, **args)
+    assert torch.equal(po, o) and torch.equal(plse, lse)
