@@ -127,6 +127,14 @@ int nq_swiglu_bwd(const void* gate, const void* up, const void* dy, void* dgate,
                   int dtype, void* stream);
 
 /*
+ * A bool keep-mask (a byte per element, nonzero = attend) as the bias of
+ * nq_attn_prefill_bias_fwd: 0 or -inf, bias (B, H, S, T padded to a multiple of 8)
+ * contiguous, the padding 0.  mask_strides: {batch, head, query, key}.
+ */
+int nq_mask_bias(const void* mask, const int64_t* mask_strides, void* bias, int B, int H, int S, int T,
+                 int dtype, void* stream);
+
+/*
  * Causal / full GQA prefill attention (FlashAttention-2 style forward).
  *
  * Replaces kernels/flash_attn.py:130-143 (flash_attention) and the

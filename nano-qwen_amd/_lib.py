@@ -60,6 +60,7 @@ SIGNATURES = {
     ]),
     "nq_swiglu": (_i32, [_p, _p, _p, _i64, _i32, _p]),  # gate, up, y, n, dtype, stream
     "nq_swiglu_bwd": (_i32, [_p, _p, _p, _p, _p, _i64, _i32, _p]),  # gate, up, dy, dgate, dup, n, dtype, stream
+    "nq_mask_bias": (_i32, [_p, _i64p, _p, _i32, _i32, _i32, _i32, _i32, _p]),  # mask, strides, bias, B, H, S, T, dtype
     "nq_attn_prefill_fwd": (_i32, [
         _p, _i64p, _p, _i64p, _p, _i64p, _p, _i64p,  # q, k, v, o (+ strides)
         _p, _p,                                      # lse, key_lens

@@ -333,16 +333,23 @@ class AttnBias:
                 raise ValueError(f"attn_mask of shape {tuple(mask.shape)} does not broadcast to "
                                  f"(B, Hq, S, T) = {(B, Hq, S, T)} on the {name} axis")
         m = m.to(device)
-        if m.dtype == torch.bool:
+        Bm, Hm, Sm = m.shape[:3]
+        self.shape = (B, Hq, S, T)
+        if m.dtype == torch.bool and m.is_cuda and dtype in _DTYPES and m.numel() > 0:
+            self.bias = torch.empty(Bm, Hm, Sm, -(-T // 8) * 8, dtype=dtype, device=device)
+            strides = (ctypes.c_int64 * 4)(*m.expand(Bm, Hm, Sm, T).stride())
+            _lib.check(_lib.load().nq_mask_bias(_ptr(m), strides, _ptr(self.bias), Bm, Hm, Sm, T, _DTYPES[dtype],
+                                                _stream(m)), "nq_mask_bias")
+            add = self.bias[..., :T]
+        elif m.dtype == torch.bool:
             add = torch.zeros(m.shape, dtype=dtype, device=device).masked_fill_(~m, float("-inf"))
         elif m.is_floating_point():
             add = m.to(dtype)
         else:
             raise TypeError(f"attn_mask must be bool or floating point, got {m.dtype}")
-        Bm, Hm, Sm = add.shape[:3]
-        self.shape = (B, Hq, S, T)
-        self.bias = torch.zeros(Bm, Hm, Sm, -(-T // 8) * 8, dtype=dtype, device=device)
-        self.bias[..., :T] = add
+        if not hasattr(self, "bias"):
+            self.bias = torch.zeros(Bm, Hm, Sm, -(-T // 8) * 8, dtype=dtype, device=device)
+            self.bias[..., :T] = add
         self.strides = self._strides(self.bias, (Bm, Hm, Sm))
         self.bias_t, self.t_strides = None, None
         if transpose:

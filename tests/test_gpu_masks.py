@@ -468,3 +468,23 @@ def test_prefill_bias_shapes(dtype, D, Hq, Hkv, causal):
         o = ops.attention_prefill(q.to(DEV), k.to(DEV), v.to(DEV), causal=causal, bias=bias)
         ref = attention(q.float(), k.float(), v.float(), causal=causal, causal_offset=T - S, mask=m.float())
         assert_close_for(dtype, o, ref, f"bias {tuple(m.shape)}")
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("shape,make", [
+    ((1, 1, 1, 8), lambda m: m),
+    ((2, 1, 5, 13), lambda m: m),                                # rows that start unaligned, a ragged last chunk
+    ((2, 3, 33, 64), lambda m: m.transpose(-1, -2).contiguous().transpose(-1, -2)),  # keys far apart
+    ((1, 1, 7, 24), lambda m: m[..., :1]),                       # one column for every key
+    ((2, 1, 300, 1030), lambda m: m[:, :, :, 3:]),               # a slice of wider rows
+])
+def test_bool_mask_as_bias(shape, make, dtype):
+    """The bias of a bool mask: 0 / -inf per element, zeros in the padding, whatever the mask's strides."""
+    say(f"mask bias {shape} {dtype}")
+    base = randn(*shape, seed=71) > 0
+    m, md = make(base), make(base.to(DEV))
+    B, H, S, T = shape[0], shape[1], shape[2], shape[3] if m.shape[3] == 1 else m.shape[3]
+    got = ops.AttnBias(md, B, H, S, T, dtype, torch.device(DEV), transpose=True)
+    ref = ops.AttnBias(m, B, H, S, T, dtype, torch.device("cpu"), transpose=True)
+    assert torch.equal(got.bias.cpu(), ref.bias) and torch.equal(got.bias_t.cpu(), ref.bias_t)
+    assert got.strides == ref.strides and got.t_strides == ref.t_strides
