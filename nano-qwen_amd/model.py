@@ -54,6 +54,8 @@ class LayerRMSNorm(nn.Module):
     autograd may keep the input itself (the kernels' backward) where the tensor
     operations keep an fp32 copy."""
 
+    input_kept = False  # of a module that was pickled without it
+
     def __init__(self, hidden_size: int, eps: float = 1e-6, input_kept: bool = False):
         super().__init__()
         self.weight = nn.Parameter(torch.ones(hidden_size))
@@ -65,11 +67,12 @@ class LayerRMSNorm(nn.Module):
         # as tensor operations eight launches forward and some twenty backward, each a
         # pass over fp32 rows: a training block at 4096 x 2048 bf16, with SwiGLU's
         # product below, 2296 -> 1863 us; four layers on 173 tokens 1420 -> 1286 us
-        if ops.plain_rows(x, w) and w.dim() == 1 and x.shape[-1] == w.shape[0]:
-            if not (torch.is_grad_enabled() and (x.requires_grad or w.requires_grad)):
-                return plain_rms_norm(x, w, self.eps)
-            if self.input_kept and w.shape[0] <= 4096:
-                return LayerRMSNormFn.apply(x, w, self.eps)
+        if not torch.jit.is_scripting():
+            if ops.plain_rows(x, w) and w.dim() == 1 and x.shape[-1] == w.shape[0]:
+                if not (torch.is_grad_enabled() and (x.requires_grad or w.requires_grad)):
+                    return plain_rms_norm(x, w, self.eps)
+                if self.input_kept and w.shape[0] <= 4096:
+                    return LayerRMSNormFn.apply(x, w, self.eps)
         return layer_rms_norm(x, w, self.eps)
 
 
@@ -112,8 +115,9 @@ class SwiGLU(nn.Module):
 
     def forward(self, x: torch.Tensor) -> torch.Tensor:
         gate, up = self.gate_proj(x), self.up_proj(x)
-        if gate.dtype == up.dtype and gate.shape == up.shape and ops.plain_rows(gate, up):
-            return self.down_proj(_SwiGLUProduct.apply(gate, up))
+        if not torch.jit.is_scripting():
+            if gate.dtype == up.dtype and gate.shape == up.shape and ops.plain_rows(gate, up):
+                return self.down_proj(_SwiGLUProduct.apply(gate, up))
         return self.down_proj(F.silu(gate) * up)
 
 

@@ -72,6 +72,7 @@ def test_layer_rmsnorm_other_routes():
     dys = torch.stack([torch.ones_like(y), 2 * torch.ones_like(y)])
     (b,) = torch.autograd.grad(norm(x), x, dys, is_grads_batched=True)
     torch.testing.assert_close(b[1], 2 * b[0])
+    torch.testing.assert_close(torch.jit.script(norm)(x), z)
     odd = LayerRMSNorm(63).to(DEV)
     assert odd(x[:, :63]).shape == (6, 63) and norm(x[:0]).shape == (0, 64)
     xt = randn(64, 6, seed=22).to(DEV).t()
@@ -108,6 +109,7 @@ def test_swiglu_other_routes():
         return ffn.down_proj(F.silu(ffn.gate_proj(t)) * ffn.up_proj(t))
     torch.testing.assert_close(ffn(x), plain(x))
     torch.testing.assert_close(torch.vmap(ffn)(x[None])[0], plain(x))
+    torch.testing.assert_close(torch.jit.script(ffn)(x), plain(x))
     for f in (ffn, plain):
         torch.func.jvp(f, (x,), (x,))
     xs = x.clone().requires_grad_()
