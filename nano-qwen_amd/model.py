@@ -51,8 +51,8 @@ class LayerRMSNorm(nn.Module):
     fp32 statistic, cast back to the input dtype before the weight multiply.
 
     ``input_kept``: the caller does not write to the input before the backward, so
-    autograd may keep the input itself (the kernels' backward) where the tensor
-    operations keep an fp32 copy."""
+    autograd keeps the input itself.  Without it a bf16 input is copied first (the tensor
+    operations keep an fp32 copy; of an fp32 input they keep the input itself too)."""
 
     input_kept = False  # of a module that was pickled without it
 
@@ -71,8 +71,9 @@ class LayerRMSNorm(nn.Module):
             if ops.plain_rows(x, w) and w.dim() == 1 and x.shape[-1] == w.shape[0]:
                 if not (torch.is_grad_enabled() and (x.requires_grad or w.requires_grad)):
                     return plain_rms_norm(x, w, self.eps)
-                if self.input_kept and w.shape[0] <= 4096:
-                    return LayerRMSNormFn.apply(x, w, self.eps)
+                if w.shape[0] <= 4096:
+                    kept = self.input_kept or x.dtype == torch.float32
+                    return LayerRMSNormFn.apply(x if kept else x.clone(), w, self.eps)
         return layer_rms_norm(x, w, self.eps)
 
 
@@ -145,7 +146,8 @@ class TransformerBlock(nn.Module):
         _check_dense(config)
         self.layer_idx = layer_idx
         self.config = config
-        self.input_layernorm = LayerRMSNorm(config.hidden_size, eps=config.rms_norm_eps, input_kept=True)
+        # its input is the block's caller's, who may reuse the memory before the backward
+        self.input_layernorm = LayerRMSNorm(config.hidden_size, eps=config.rms_norm_eps)
         self.attention = Attention(config, layer_idx=layer_idx)
         self.post_attention_layernorm = LayerRMSNorm(config.hidden_size, eps=config.rms_norm_eps, input_kept=True)
         self.feed_forward = SwiGLU(config.hidden_size, config.intermediate_size)

@@ -49,6 +49,9 @@ def _code(t: torch.Tensor) -> int:
         raise TypeError(f"unsupported dtype {t.dtype}; the kernels take bfloat16 or float32") from None
 
 
+_MAX_ELEMENTS = 2 ** 34  # of a kernel with a thread per 8 elements: a launch has fewer than 2^32 threads
+
+
 # What every call goes through takes plain ints where ctypes does (the signatures
 # convert them) and builds no object it drops again: of the ~30 us that the host
 # takes for one decode step, the two launches are ~10.
@@ -83,8 +86,8 @@ def _aligned(t: torch.Tensor) -> bool:
 def plain_rows(*ts: torch.Tensor) -> bool:
     """Whether a kernel may stand in for tensor operations on these operands: contiguous
     bf16 or fp32 tensors of the current device, not empty, 16-byte aligned, rows of whole
-    16-byte pieces, outside tracing, compilation, vmap, forward-mode and dispatch modes
-    (which the tensor operations go through)."""
+    16-byte pieces, no larger than one launch takes, outside tracing, compilation, vmap,
+    forward-mode and dispatch modes (which the tensor operations go through)."""
     if (torch.compiler.is_compiling() or torch.jit.is_tracing() or _forward_ad._current_level >= 0
             or torch._C._functorch.peek_interpreter_stack() is not None
             or torch._C._len_torch_dispatch_stack() > 0):
@@ -93,7 +96,7 @@ def plain_rows(*ts: torch.Tensor) -> bool:
         if (type(t) not in (torch.Tensor, torch.nn.Parameter) or torch._C._functorch.is_legacy_batchedtensor(t)
                 or not t.is_cuda or t.dtype not in _DTYPES
                 or t.layout != torch.strided or not t.is_contiguous() or t.dim() == 0 or t.numel() == 0
-                or t.shape[-1] % 8 or t.data_ptr() % 16):
+                or t.numel() >= _MAX_ELEMENTS or t.shape[-1] % 8 or t.data_ptr() % 16):
             return False
     return all(t.device == ts[0].device for t in ts) and ts[0].device.index == torch.cuda.current_device()
 
@@ -335,7 +338,8 @@ class AttnBias:
         m = m.to(device)
         Bm, Hm, Sm = m.shape[:3]
         self.shape = (B, Hq, S, T)
-        if m.dtype == torch.bool and m.is_cuda and dtype in _DTYPES and m.numel() > 0:
+        if (m.dtype == torch.bool and m.is_cuda and dtype in _DTYPES and m.numel() > 0
+                and Bm * Hm * Sm * T < _MAX_ELEMENTS):
             self.bias = torch.empty(Bm, Hm, Sm, -(-T // 8) * 8, dtype=dtype, device=device)
             strides = (ctypes.c_int64 * 4)(*m.expand(Bm, Hm, Sm, T).stride())
             _lib.check(_lib.load().nq_mask_bias(_ptr(m), strides, _ptr(self.bias), Bm, Hm, Sm, T, _DTYPES[dtype],

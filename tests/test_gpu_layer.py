@@ -5,7 +5,7 @@ import pytest
 import torch
 import torch.nn.functional as F
 
-from nano_qwen_amd.model import LayerRMSNorm, SwiGLU, _SwiGLUProduct
+from nano_qwen_amd.model import LayerRMSNorm, ModelConfig, SwiGLU, TransformerBlock, _SwiGLUProduct
 from nano_qwen_amd.norm import layer_rms_norm
 from tests.helpers import randn, say
 
@@ -83,6 +83,25 @@ def test_layer_rmsnorm_other_routes():
     out = free(h)
     h.add_(1)
     out.sum().backward()
+
+
+def test_block_input_may_change_before_backward():
+    """A block's caller may reuse its bf16 input's memory: gradients are those of the forward's input."""
+    say("block input overwritten before the backward")
+    cfg = ModelConfig(vocab_size=64, hidden_size=64, intermediate_size=128, num_hidden_layers=1,
+                      num_attention_heads=4, num_key_value_heads=2, head_dim=32)
+    block = TransformerBlock(cfg).to(DEV, BF)
+    grads = []
+    for overwrite in (False, True):
+        x = randn(2, 9, 64, seed=24, dtype=BF).to(DEV).requires_grad_()
+        h = x * 1
+        y = block(h)
+        y = y[0] if isinstance(y, tuple) else y
+        if overwrite:
+            h.zero_()
+        grads.append(torch.autograd.grad(y.float().sum(), [x, *block.parameters()]))
+    for a, b in zip(*grads):
+        _close(b, a.double().cpu(), BF, 1, "gradient")
 
 
 @pytest.mark.parametrize("shape", [(1, 8), (3, 683, 8), (2, 5, 6144)])
