@@ -53,7 +53,8 @@ def _ref_params(path, name):
     raise AssertionError(f"{name} not found in {path}")
 
 
-@pytest.mark.skipif(not os.path.isdir(REF), reason="reference tree not present")
+@pytest.mark.skipif(not all(os.path.isfile(os.path.join(REF, rel)) for rel, _ in EXPECTED),
+                    reason="reference tree not present")
 @pytest.mark.parametrize("key", list(EXPECTED))
 def test_expected_signature_is_the_reference_source(key):
     rel, name = key
