@@ -38,8 +38,11 @@ def rms_norm(x: torch.Tensor, weight: torch.Tensor, eps: float) -> torch.Tensor:
 def _rms_norm_into(x: torch.Tensor, w: torch.Tensor, y: torch.Tensor, eps: float) -> torch.Tensor:
     """The launch: x and y hold equally spaced rows (all but the last dim are rows), y contiguous."""
     W = x.shape[-1]
-    rc = _lib.load().nq_rmsnorm(ops._ptr(x), x.stride(0) if x.dim() == 2 else W, ops._ptr(w), ops._ptr(y), W,
-                                x.numel() // W, W, ops._code(x), ops._code(w), ops._code(y), eps, ops._stream(x))
+    rows = x.numel() // W
+    # the stride of a single row is anything, also in a tensor that counts as contiguous
+    pitch = x.stride(0) if x.dim() == 2 and rows > 1 else W
+    rc = _lib.load().nq_rmsnorm(ops._ptr(x), pitch, ops._ptr(w), ops._ptr(y), W, rows, W,
+                                ops._code(x), ops._code(w), ops._code(y), eps, ops._stream(x))
     _lib.check(rc, "nq_rmsnorm")
     return y
 

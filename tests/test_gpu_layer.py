@@ -6,7 +6,7 @@ import torch
 import torch.nn.functional as F
 
 from nano_qwen_amd.model import LayerRMSNorm, ModelConfig, SwiGLU, TransformerBlock, _SwiGLUProduct
-from nano_qwen_amd.norm import layer_rms_norm
+from nano_qwen_amd.norm import layer_rms_norm, rms_norm
 from tests.helpers import randn, say
 
 pytestmark = pytest.mark.gpu
@@ -51,6 +51,31 @@ def test_layer_rmsnorm(rows, width, xdt, wdt):
     # a bf16 n may round the other way: 2^-8 of a term now and then
     _close(dw, (d6 * n.to(xdt).double()).sum(0), BF if BF in (xdt, wdt) else F32, rows, "dw")
     assert dx.dtype == xdt and dw.dtype == wdt
+
+
+@pytest.mark.parametrize("xdt", [BF, F32])
+def test_one_row_of_a_wider_tensor(xdt):
+    """A single row counts as contiguous whatever its stride, here no multiple of 16 bytes."""
+    say(f"one row of a wider tensor {xdt}")
+    big = randn(4, 71, seed=14, dtype=xdt)
+    w = (1 + 0.1 * randn(64, seed=15)).to(xdt)
+    norm = LayerRMSNorm(64).to(DEV, xdt)
+    with torch.no_grad():
+        norm.weight.copy_(w)
+    x = big.to(DEV)[:1, :64]
+    assert x.is_contiguous() and x.stride(0) == 71
+    want = (big[:1, :64].double() * torch.rsqrt(big[:1, :64].double().square().mean(-1, keepdim=True) + 1e-6))
+    want = want.to(xdt).double() * w.double()
+    with torch.no_grad():
+        _close(norm(x), want, xdt, 64, "y")
+    _close(rms_norm(x, norm.weight.detach(), 1e-6), want, xdt, 64, "rms_norm")
+    xg = x.detach().requires_grad_()
+    y = norm(xg)
+    _close(y, want, xdt, 64, "y with a gradient")
+    (dx,) = torch.autograd.grad(y, xg, torch.ones_like(y))
+    z = layer_rms_norm(xg, norm.weight, 1e-6)
+    (want,) = torch.autograd.grad(z, xg, torch.ones_like(z))
+    _close(dx, want.double().cpu(), xdt, 64, "dx")
 
 
 def test_layer_rmsnorm_other_routes():
