@@ -117,7 +117,8 @@ class SwiGLU(nn.Module):
     def forward(self, x: torch.Tensor) -> torch.Tensor:
         gate, up = self.gate_proj(x), self.up_proj(x)
         if not torch.jit.is_scripting():
-            if gate.dtype == up.dtype and gate.shape == up.shape and ops.plain_rows(gate, up):
+            # plain_rows first: the proxies of torch.fx's symbolic trace cannot be compared
+            if ops.plain_rows(gate, up) and gate.dtype == up.dtype and gate.shape == up.shape:
                 return self.down_proj(_SwiGLUProduct.apply(gate, up))
         return self.down_proj(F.silu(gate) * up)
 

@@ -4,6 +4,7 @@ import pytest
 import torch
 
 from nano_qwen_amd import KVCache, ModelConfig, Qwen3Model, generate_greedy_batch
+from nano_qwen_amd.model import LayerRMSNorm, SwiGLU
 from tests.golden.make_golden_model import MODEL, make_model_weights
 
 
@@ -20,6 +21,14 @@ def test_reference_state_dict_loads_strict():
     m.load_state_dict(w, strict=True)
     assert set(m.state_dict()) == set(w)
     assert m.count_parameters()["total"] == sum(v.numel() for v in w.values())
+
+
+@pytest.mark.parametrize("make", [lambda: LayerRMSNorm(16), lambda: SwiGLU(16, 24)])
+def test_layers_trace_symbolically(make):
+    """torch.fx's symbolic trace goes through the layers' tensor operations."""
+    mod, x = make(), torch.randn(3, 16)
+    traced = torch.fx.symbolic_trace(mod)
+    assert torch.equal(traced(x), mod(x))
 
 
 def test_forward_on_cpu_fails_loudly():
