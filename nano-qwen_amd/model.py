@@ -50,9 +50,11 @@ class LayerRMSNorm(nn.Module):
     """RMSNorm over the hidden size, the reference's arithmetic (model/norm.py:17-22):
     fp32 statistic, cast back to the input dtype before the weight multiply.
 
-    ``input_kept``: the caller does not write to the input before the backward, so
-    autograd keeps the input itself.  Without it a bf16 input is copied first (the tensor
-    operations keep an fp32 copy; of an fp32 input they keep the input itself too)."""
+    Under autograd a bf16 input is copied, so that its owner may write to it before the
+    backward (the tensor operations keep an fp32 copy; of an fp32 input they keep the input
+    itself, and so does this).  The model's own norms do too: a program may call them by
+    themselves, and hooks see their inputs.  ``input_kept`` says that nobody writes to the
+    input until then, and autograd keeps the input itself."""
 
     input_kept = False  # of a module that was pickled without it
 
@@ -147,10 +149,9 @@ class TransformerBlock(nn.Module):
         _check_dense(config)
         self.layer_idx = layer_idx
         self.config = config
-        # its input is the block's caller's, who may reuse the memory before the backward
         self.input_layernorm = LayerRMSNorm(config.hidden_size, eps=config.rms_norm_eps)
         self.attention = Attention(config, layer_idx=layer_idx)
-        self.post_attention_layernorm = LayerRMSNorm(config.hidden_size, eps=config.rms_norm_eps, input_kept=True)
+        self.post_attention_layernorm = LayerRMSNorm(config.hidden_size, eps=config.rms_norm_eps)
         self.feed_forward = SwiGLU(config.hidden_size, config.intermediate_size)
 
     def forward(self, hidden_states: torch.Tensor, position_ids: Optional[torch.Tensor] = None,
@@ -175,7 +176,7 @@ class Qwen3Model(nn.Module):
         self.embed = TokenEmbedding(config)
         self.layers = nn.ModuleList([TransformerBlock(config, layer_idx=i)
                                      for i in range(config.num_hidden_layers)])
-        self.norm = LayerRMSNorm(config.hidden_size, eps=config.rms_norm_eps, input_kept=True)
+        self.norm = LayerRMSNorm(config.hidden_size, eps=config.rms_norm_eps)
         self.lm_head = nn.Linear(config.hidden_size, config.vocab_size, bias=False)
         if getattr(config, "tie_word_embeddings", False):
             self.lm_head.weight = self.embed.embed_tokens.weight

@@ -5,7 +5,7 @@ import pytest
 import torch
 import torch.nn.functional as F
 
-from nano_qwen_amd.model import LayerRMSNorm, ModelConfig, SwiGLU, TransformerBlock, _SwiGLUProduct
+from nano_qwen_amd.model import LayerRMSNorm, ModelConfig, Qwen3Model, SwiGLU, TransformerBlock, _SwiGLUProduct
 from nano_qwen_amd.norm import layer_rms_norm, rms_norm
 from tests.helpers import randn, say
 
@@ -127,6 +127,25 @@ def test_block_input_may_change_before_backward():
         grads.append(torch.autograd.grad(y.float().sum(), [x, *block.parameters()]))
     for a, b in zip(*grads):
         _close(b, a.double().cpu(), BF, 1, "gradient")
+
+
+@pytest.mark.parametrize("name", ["norm", "layers.0.post_attention_layernorm", "layers.0.input_layernorm"])
+def test_models_norms_let_their_input_change(name):
+    """A program that calls one of a model's norms may write to its bf16 input before the backward."""
+    say(f"input of {name} overwritten before the backward")
+    cfg = ModelConfig(vocab_size=64, hidden_size=64, intermediate_size=128, num_hidden_layers=1,
+                      num_attention_heads=4, num_key_value_heads=2, head_dim=32)
+    norm = Qwen3Model(cfg).to(DEV, BF).get_submodule(name)
+    grads = []
+    for overwrite in (False, True):
+        x = randn(5, 64, seed=25, dtype=BF).to(DEV).requires_grad_()
+        h = x * 1
+        y = norm(h)
+        if overwrite:
+            h.mul_(3)
+        grads.append(torch.autograd.grad(y.float().square().sum(), [x, norm.weight]))
+    for a, b in zip(*grads):
+        assert torch.equal(a, b)
 
 
 @pytest.mark.parametrize("shape", [(1, 8), (3, 683, 8), (2, 5, 6144)])
