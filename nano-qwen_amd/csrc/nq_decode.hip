@@ -882,14 +882,17 @@ decode_stream_f32_kernel(DecodeParams p) {
         for (int i = 0; i < 4; ++i) mx = fmaxf(mx, sc[kb][i]);
       mx = fmaxf(mx, shfl_xor_f(mx, 16));
       mx = fmaxf(mx, shfl_xor_f(mx, 32));
-      const float m_new = fmaxf(m_i, mx * p.scale_log2);  // finite: a step holds a key below kend
-      const float alpha = fast_exp2(m_i - m_new);
+      // a step holds a key below kend, but its scores may have overflowed to -inf:
+      // without a finite one so far the row keeps m = -inf and exponentiates against 0
+      const float m_new = fmaxf(m_i, mx * p.scale_log2);
+      const float m_use = m_new > -INFINITY ? m_new : 0.f;
+      const float alpha = fast_exp2(m_i - m_use);
       float rs = 0.f;
 #pragma unroll
       for (int kb = 0; kb < 2; ++kb)
 #pragma unroll
         for (int i = 0; i < 4; ++i) {
-          sc[kb][i] = fast_exp2(__builtin_fmaf(sc[kb][i], p.scale_log2, -m_new));
+          sc[kb][i] = fast_exp2(__builtin_fmaf(sc[kb][i], p.scale_log2, -m_use));
           rs += sc[kb][i];
         }
       l_i = __builtin_fmaf(l_i, alpha, rs);
@@ -971,7 +974,7 @@ __global__ void __launch_bounds__(DC_MERGE_MAX_THREADS) decode_merge_kernel(Deco
   if (wf == wl) return;  // one wave covered the row and wrote it
   const int ns = (int)(wl - wf + 1);
   // one pass with a running max, so every partial's (m, l) and outputs are
-  // loaded together (every partial holds at least one key: its m is finite)
+  // loaded together (a partial whose scores are all -inf has m = -inf and l = 0)
   float M = -INFINITY, wsum = 0.f;
   float acc[DPT];
 #pragma unroll
@@ -996,8 +999,9 @@ __global__ void __launch_bounds__(DC_MERGE_MAX_THREADS) decode_merge_kernel(Deco
         }
       }
       const float Mn = fmaxf(M, m_l[0]);
-      const float a = fast_exp2(M - Mn);  // 0 for the first partial
-      const float sc = fast_exp2(m_l[0] - Mn);
+      const float Mu = Mn > -INFINITY ? Mn : 0.f;
+      const float a = fast_exp2(M - Mu);  // 0 for the first partial
+      const float sc = fast_exp2(m_l[0] - Mu);
       wsum = wsum * a + m_l[1] * sc;
 #pragma unroll
       for (int e = 0; e < DPT; ++e) acc[e] = acc[e] * a + o[e] * sc;

@@ -95,9 +95,9 @@ __device__ __forceinline__ int key_perm32(int r) {
 }
 
 // ---- split keys.  A query block's tiles [0, ntiles) start at those whose first
-// key every row of the block sees, so that no row of a split is without a
-// finite score; these are dealt to the splits in equal runs, and the tiles
-// after them (the block's diagonal) stay with the last run.
+// key every row of the block sees, so that every row sees a key in the first tile
+// of a split; these are dealt to the splits in equal runs, and the tiles after
+// them (the block's diagonal) stay with the last run.
 // The keys [kofs, kend) of split s; false: it has none.
 template <bool CAUSAL>
 __device__ __forceinline__ bool pf_split(const PrefillParams& p, int q0, int s, int& kofs, int& kend) {
@@ -570,9 +570,16 @@ prefill_kernel(PrefillParams p) {
   // here; later tiles carry the offset from their MFMAs.)  mx_cur is the row
   // max of the next tile to be exponentiated, relative to m_i.
   float mx_cur = 0.f;
-  // BIAS: a row with no finite score yet holds the placeholder max 0 (ph);
-  // its first finite tile max then replaces it outright (O and l are still 0)
+  // BIAS, SPLIT: a row with no finite score yet holds the placeholder max 0 (ph);
+  // its first finite tile max then replaces it outright (O and l are still 0).
+  // In a split that is a row whose scores overflow to -inf over its run's first
+  // tiles: other runs may hold finite ones.  There raise_at, the mx_cur above which
+  // the row max is raised, is -inf meanwhile and stands for ph: a ph of its own in
+  // the loop cost 0.9% (500 queries on 12345 paged keys, 32/8 heads: 117.7 ->
+  // 118.7 us); with raise_at the bias kernel spills more (causal D = 128, B4
+  // S1024: 67.3 -> 68.8 us).
   bool ph = false;
+  float raise_at = PF_RESCALE_LOG2;
   {
     mask_tile(sA, 0);
     float mx = -INFINITY;
@@ -581,11 +588,11 @@ prefill_kernel(PrefillParams p) {
 #pragma unroll
       for (int i = 0; i < 16; i += 2) mx = fmaxf(mx, fmaxf(sA[kb][i], sA[kb][i + 1]));
     mx = xor32_max(mx);
-    if constexpr (BIAS) {
+    if constexpr (BIAS || SPLIT) {
       ph = !(mx > -INFINITY);
       if (ph) mx = 0.f;
       // S[0] relative to the placeholder is all -inf: no max to take from it
-      if (ph) mx_cur = -INFINITY;
+      if (ph) mx_cur = raise_at = -INFINITY;
     }
     set_max(mx);
 #pragma unroll
@@ -617,20 +624,22 @@ prefill_kernel(PrefillParams p) {
 
     // online softmax (log2 domain); each lane owns one query row
     (void)n0;
-    bool raise = mx_cur > PF_RESCALE_LOG2;
+    bool raise = mx_cur > (SPLIT ? raise_at : PF_RESCALE_LOG2);
     if constexpr (BIAS) raise = raise || (ph && mx_cur > -INFINITY);
     if (wave_any(raise)) {
       const float m_old = m_i;
       float inc = fmaxf(mx_cur, 0.f);
-      if constexpr (BIAS) {
+      if constexpr (SPLIT) ph = raise_at < 0.f;
+      if constexpr (BIAS || SPLIT) {
         if (ph) inc = mx_cur > -INFINITY ? mx_cur : 0.f;
       }
       set_max(m_i + inc);
       const float delta = m_i - m_old;
       float alpha = fast_exp2(-delta);
-      if constexpr (BIAS) {
+      if constexpr (BIAS || SPLIT) {
         if (ph) alpha = 0.f;  // nothing accumulated yet (avoids 0 * inf)
         ph = ph && !(mx_cur > -INFINITY);
+        if (SPLIT && !ph) raise_at = PF_RESCALE_LOG2;
       }
       l_i *= alpha;
 #pragma unroll
@@ -761,7 +770,8 @@ prefill_kernel(PrefillParams p) {
       for (int gq = 0; gq < 4; ++gq)
         po[(dd * 4 + gq) * 64] = floatx4{oacc[dd][gq * 4 + 0], oacc[dd][gq * 4 + 1], oacc[dd][gq * 4 + 2],
                                          oacc[dd][gq * 4 + 3]};
-    if (sl < 32) pf_split_ml(p, D, NW)[grp * 32 + sl] = floatx2{m_i, l_i};
+    // a run without a finite score (m = -inf, l = 0, O = 0) weighs nothing in the merge
+    if (sl < 32) pf_split_ml(p, D, NW)[grp * 32 + sl] = floatx2{raise_at < 0.f ? -INFINITY : m_i, l_i};
     return;
   }
   // (BIAS: a row the bias masks entirely has l = 0 and gets zeros, as SDPA gives)

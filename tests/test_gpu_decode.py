@@ -167,3 +167,25 @@ def test_decode_merge_of_many_partials(dtype, Hq, Hkv, keys, chunk):
         ref = decode_path(q.float(), kc.float(), vc.float(), lens, q_weight=qw, eps=1e-6, cos=cos, sin=sin,
                           q_pos=lens.long() - 1)
         assert_close_for(dtype, o, ref, f"D={D}")
+
+
+@pytest.mark.parametrize("D", [32, 64, 128])
+@pytest.mark.parametrize("dropped", ["odd", "most"])
+def test_decode_f32_scores_overflowing(D, dropped):
+    """Steps of 32 keys whose scores all overflow to -inf weigh nothing, wherever the waves' ranges begin."""
+    say(f"fp32 decode, overflowing scores D={D} {dropped}")
+    B, Hq, Hkv, T = 2, 8, 2, 1700
+    lens = torch.tensor([T, 1001], dtype=torch.int32)
+    q, kc, vc = randn(B, Hq, D, seed=96), randn(B, Hkv, T, D, seed=97), randn(B, Hkv, T, D, seed=98)
+    step = torch.arange(T) // 32
+    drop = (step >= 1) & ((step % 2 == 1) if dropped == "odd" else True)
+    q[..., 0] = 1e20
+    kc[..., 0] = torch.where(drop, -1e25, 0.0)  # products beyond fp32's range
+    for chunk in (0, 32, 128):
+        o = nq.attention_decode(q.to(DEV), kc.to(DEV), vc.to(DEV), lens.to(DEV), max_len=T, chunk=chunk)
+        qd, kd = q.double(), kc.double()
+        qd[..., 0] = kd[..., 0] = 0
+        sc = qd.view(B, Hkv, -1, 1, D) @ kd[:, :, None].transpose(-1, -2) / D ** 0.5
+        gone = drop | (torch.arange(T) >= lens.view(B, 1, 1, 1, 1))
+        ref = (torch.softmax(sc.masked_fill(gone, float("-inf")), -1) @ vc.double()[:, :, None]).view(B, Hq, D)
+        assert_close_for(torch.float32, o, ref, f"chunk={chunk}")

@@ -439,3 +439,45 @@ def test_split_keys_prefill_f32(Hq, Hkv, D, S, T, causal, fused):
             pool[int(bt[i]), :, :rows.shape[1]] = rows
     po, plse = ops.attention_prefill_paged(q.to(DEV), kp, vp, bt.view(1, n).to(DEV), T=T, **args)
     assert torch.equal(po, o) and torch.equal(plse, lse)
+
+
+@pytest.mark.parametrize("paged", [False, True])
+@pytest.mark.parametrize("Hq,Hkv,D,S,T,dropped", [
+    (8, 2, 128, 33, 1600, "most"),   # every run but the first without a finite score
+    (8, 2, 64, 500, 5003, "odd"),    # finite scores from a run's second tile on
+    (2, 2, 128, 129, 1664, "odd"),
+])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+def test_split_keys_prefill_scores_overflowing(dtype, Hq, Hkv, D, S, T, dropped, paged):
+    """Keys whose scores overflow to -inf, over whole runs or their first tiles, weigh nothing."""
+    say(f"split prefill, overflowing scores D={D} S={S} T={T} {dropped} paged={paged} {dtype}")
+    lib = ops._lib.load()
+    assert lib.nq_attn_prefill_workspace_bytes(1, Hq, Hkv, S, T, D, ops._code(torch.empty(0, dtype=dtype))) > 0
+    q, k, v = (randn(1, H, n, D, seed=421 + i, dtype=dtype) for i, (H, n) in enumerate(((Hq, S), (Hkv, T), (Hkv, T))))
+    tile = torch.arange(T) // 64
+    drop = (tile >= 1) & (torch.arange(T) < T - S) & ((tile % 2 == 1) if dropped == "odd" else True)
+    # the products of dim 0 are 0 for kept keys and beyond fp32's range, negative, for the others
+    q[..., 0] = 1e20
+    k[..., 0] = torch.where(drop, -1e25, 0.0).to(dtype)
+    args = dict(causal=True, return_lse=True)
+    if paged:
+        P = 64
+        n = -(-T // P)
+        pools = torch.zeros(2, n, Hkv, P, D, dtype=dtype, device=DEV)
+        for src, pool in ((k, pools[0]), (v, pools[1])):
+            for i in range(n):
+                rows = src[0, :, i * P:(i + 1) * P].to(DEV)
+                pool[i, :, :rows.shape[1]] = rows
+        bt = torch.arange(n, dtype=torch.int32, device=DEV).view(1, n)
+        o, lse = ops.attention_prefill_paged(q.to(DEV), pools[0], pools[1], bt, T=T, **args)
+    else:
+        o, lse = ops.attention_prefill(q.to(DEV), k.to(DEV), v.to(DEV), **args)
+    qd, kd = q.double(), k.double()
+    qd[..., 0] = kd[..., 0] = 0
+    sc = qd.view(1, Hkv, -1, S, D) @ kd[:, :, None].transpose(-1, -2) / D ** 0.5
+    sc = sc.masked_fill(drop | (torch.arange(T) > torch.arange(S)[:, None] + T - S), float("-inf"))
+    ref = (torch.softmax(sc, -1) @ v.double()[:, :, None]).view(1, Hq, S, D)
+    assert_close_for(dtype, o, ref, "overflowing o")
+    # bf16: the query is rounded again after its scaling, 2^-9 of D products of unit variance
+    torch.testing.assert_close(lse.cpu().double(), torch.logsumexp(sc, -1).view(1, Hq, S), rtol=0,
+                               atol=2e-2 if dtype == torch.bfloat16 else 1e-5)
