@@ -801,6 +801,15 @@ def attention_merge_(o: torch.Tensor, lse: torch.Tensor, o_part: torch.Tensor,
 # Backward
 # ---------------------------------------------------------------------------
 
+def _backward_workspace_bytes(B: int, Hq: int, Hkv: int, S: int, T: int, D: int, dt: int, causal: bool,
+                              biased: bool) -> int:
+    """With room for the partial sums of dK/dV, whose steps a small launch splits; one with a bias never does."""
+    lib = _lib.load()
+    if biased:
+        return int(lib.nq_attn_bwd_workspace_bytes(B, Hq, S))
+    return int(lib.nq_attn_bwd_split_workspace_bytes(B, Hq, Hkv, S, T, D, dt, int(bool(causal))))
+
+
 def attention_backward(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, o: torch.Tensor,
                        dout: torch.Tensor, lse: torch.Tensor, *, causal: bool = True,
                        sm_scale: Optional[float] = None, key_lens: Optional[torch.Tensor] = None,
@@ -838,8 +847,7 @@ def attention_backward(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, o: tor
     lib = _lib.load()
     if workspace is None or (workspace.numel() * workspace.element_size()
                              < int(lib.nq_attn_bwd_workspace_bytes(B, Hq, S))):
-        # with room for the partial sums of dK/dV, whose steps a small launch splits
-        need = int(lib.nq_attn_bwd_split_workspace_bytes(B, Hq, Hkv, S, T, D, _code(q), int(bool(causal))))
+        need = _backward_workspace_bytes(B, Hq, Hkv, S, T, D, _code(q), causal, bias is not None)
         workspace = torch.empty(need, dtype=torch.uint8, device=dev)
     st = _lib.strides3
     head = (_ptr(q), st(q.stride()[:3]), _ptr(k), st(k.stride()[:3]), _ptr(v), st(v.stride()[:3]),

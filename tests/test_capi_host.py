@@ -98,6 +98,15 @@ def test_fp32_side_inputs_are_realigned():
     assert _f32(aligned, base.device).data_ptr() == aligned.data_ptr()
 
 
+def test_backward_with_a_bias_takes_no_room_for_partials():
+    """A launch of few key blocks splits dK/dV's steps, but not under a bias: its workspace holds no partials."""
+    from nano_qwen_amd import ops
+    sizes = (1, 32, 8, 1024, 1024, 128, _lib.NQ_DTYPE_BF16, True)
+    base = _lib.load().nq_attn_bwd_workspace_bytes(1, 32, 1024)
+    assert ops._backward_workspace_bytes(*sizes, False) > base
+    assert ops._backward_workspace_bytes(*sizes, True) == base
+
+
 def test_cpu_tensors_are_refused():
     q = torch.zeros(1, 2, 4, 64)
     with pytest.raises(RuntimeError, match="HIP device"):
