@@ -391,11 +391,13 @@ __global__ void __launch_bounds__(256, D == 64 ? 3 : 2) bwd_dkdv_kernel(BwdParam
   } else {
     kblk = blockIdx.x / npairs;
     pair = blockIdx.x % npairs;
-    // one to two workgroups per CU, all resident from the start: the second half
-    // goes lightest first, so that the CU with the heaviest block gets the
-    // lightest as its other one (B2 S4096 32/8 heads, 512 blocks: 915 -> 799 us)
-    const int half = (nkb + 1) / 2;
-    if (CAUSAL && nkb * npairs > 256 && nkb * npairs <= 512 && kblk >= half) kblk = nkb - 1 - (kblk - half);
+    // one to two workgroups per CU, all resident from the start: the ones beyond
+    // one per CU, the lightest blocks, go lightest first, so that the CU with the
+    // heaviest block gets the lightest as its other one (B2 32/8 heads D128, dK/dV
+    // with dQ: 512 blocks 1228 -> 1127 us, 384 817 -> 772, 320 644 -> 625, 272 513 ->
+    // 514; with the second half of the blocks reversed, those last took 664 and 560)
+    const int first = (256 + npairs - 1) / npairs;
+    if (CAUSAL && nkb * npairs > 256 && nkb * npairs <= 512 && kblk >= first) kblk = nkb - 1 - (kblk - first);
   }
   const int b = pair / p.Hkv, kvh = pair % p.Hkv;
   const int k0 = kblk * BW_KEYS;

@@ -451,3 +451,37 @@ def test_split_dkdv_backward(Hq, Hkv, D, S, T, causal, dtype):
     for a, b in zip(split[1:], whole[1:]):
         _close_rel(a, b, "padded split against whole", dtype)
         assert not a[:, :, int(lens[0]):].any()
+
+
+@pytest.mark.parametrize("B,Hkv,G,D,S,T", [
+    (4, 8, 1, 64, 1400, 1400),   # 11 key blocks x 32 pairs
+    (2, 8, 2, 32, 2100, 2177),   # 18 x 16, the last block one key; T > S
+    (3, 43, 1, 64, 385, 385),    # 4 x 129: 516 blocks, beyond the range
+    (3, 29, 1, 64, 385, 385),    # 4 x 87: a pair count that does not divide 256
+    (5, 8, 1, 128, 1537, 1600),  # 13 x 40 = 520, beyond too
+    (5, 8, 1, 128, 1400, 1410),  # 12 x 40 = 480
+])
+def test_backward_block_order(B, Hkv, G, D, S, T):
+    """Causal dK/dV launches of one to two key blocks per CU take the blocks beyond one per CU
+    in another order: each key's rows are written, and are those of the reference."""
+    say(f"block order B={B} Hkv={Hkv} G={G} D={D} S={S} T={T}")
+    dt = torch.bfloat16
+    Hq = Hkv * G
+    q, k, v, do = (randn(B, H, n, D, seed=591 + i, dtype=dt).to(DEV)
+                   for i, (H, n) in enumerate(((Hq, S), (Hkv, T), (Hkv, T), (Hq, S))))
+    lens = torch.randint(T // 2, T + 1, (B,), generator=torch.Generator().manual_seed(590)).to(torch.int32)
+    for kl in (None, lens.to(DEV)):
+        o, lse = ops.attention_prefill(q, k, v, causal=True, key_lens=kl, return_lse=True)
+        got = ops.attention_backward(q, k, v, o, do, lse, causal=True, key_lens=kl)
+        for b in range(B):
+            for h in range(0, Hkv, 7):  # fp64 autograd of one pair at a time
+                hs = slice(h * G, h * G + G)
+                leaves = [t.double().detach().requires_grad_() for t in (q[b, hs], k[b, h], v[b, h])]
+                sc = leaves[0] @ leaves[1].t() / D ** 0.5
+                gone = torch.arange(T, device=DEV) > torch.arange(S, device=DEV)[:, None] + T - S
+                if kl is not None:
+                    gone = gone | (torch.arange(T, device=DEV) >= kl[b])
+                p = torch.softmax(sc.masked_fill(gone, float("-inf")), -1)
+                ref = torch.autograd.grad((p @ leaves[2] * do[b, hs].double()).sum(), leaves)
+                for name, g, r in zip(("dq", "dk", "dv"), (got[0][b, hs], got[1][b, h], got[2][b, h]), ref):
+                    _close_rel(g, r, name, dt)
