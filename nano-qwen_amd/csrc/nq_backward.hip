@@ -630,7 +630,11 @@ __global__ void __launch_bounds__(256, D == 64 ? 3 : 2) bwd_dkdv_kernel(BwdParam
     bw_store_part<D>(p, kblk, pair, split, wave, fresh_lane(), dkacc, dvacc);
     return;
   }
-  const int el = fresh_lane(), ehh = el >> 5;  // no lane value held through the loop: it would spill
+  // no lane value held through the loop: it would spill.  (The causal bias kernel
+  // at D = 128 holds its lane there anyway, and a fresh one made it spill 12
+  // registers where the held one spills 5: causal masked backward with dQ, B2
+  // 32/8 heads S1024, 386 against 366 us.)
+  const int el = BIAS && CAUSAL && D == 128 ? lane : fresh_lane(), ehh = el >> 5;
   const int ekey = k0 + wave * 32 + (el & 31);
   if (ekey >= p.T) return;
   T* dko = reinterpret_cast<T*>(p.dk) + b * p.dksb + kvh * p.dksh + (int64_t)ekey * p.dkss;
