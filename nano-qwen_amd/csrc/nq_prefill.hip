@@ -1019,7 +1019,7 @@ static int prefill_entry(const void* q, const int64_t* q_strides, const void* k,
   if (f32) {
     p.BM = 128 / G;
     p.nqb = (S + p.BM - 1) / p.BM;
-    const KeyRuns kr = workspace && !key_lens && !bias ? f32_key_runs(B, Hq, Hkv, S, T) : KeyRuns{1, 1};
+    const KeyRuns kr = workspace && !key_lens && !bias ? f32_key_runs(B, Hq, Hkv, S, T, D) : KeyRuns{1, 1};
     p.nsplit = kr.n;
     p.run = kr.len;
     if (p.nsplit > 1) {
@@ -1055,7 +1055,7 @@ extern "C" int64_t nq_attn_prefill_workspace_bytes(int B, int Hq, int Hkv, int S
   if (B <= 0 || Hq <= 0 || Hkv <= 0 || S <= 0 || T <= 0 || Hq % Hkv || !head_dim_ok(D) || !nq_dtype_ok(dtype))
     return 0;
   if (dtype == NQ_DTYPE_F32) {
-    const KeyRuns kr = f32_key_runs(B, Hq, Hkv, S, T);  // 128 rows' accumulators, max and sum per workgroup
+    const KeyRuns kr = f32_key_runs(B, Hq, Hkv, S, T, D);  // 128 rows' accumulators, max and sum per workgroup
     return kr.n > 1 ? prefill_wgs4(B, Hq, Hkv, S) * kr.n * (f32_part(D) + 256) * (int64_t)sizeof(float) : 0;
   }
   const int ns = prefill_splits(B, Hq, Hkv, S, T);

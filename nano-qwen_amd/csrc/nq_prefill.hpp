@@ -57,21 +57,40 @@ struct PrefillParams {
 // deal a query block's 32-key tiles to workgroups: runs of `len` tiles, `n` for
 // the longest block, n = 1 for none.  A launch of fewer workgroups than two per
 // CU leaves the device to its heaviest blocks (B2 S1000 8/2 heads D64: 128
-// workgroups of 1 to 32 tiles, ~2 us a tile): runs of the length that gives two
-// workgroups per CU the same work, at least F32_MIN_RUN tiles, at most
+// workgroups of 1 to 32 tiles, 90 us whole and 54 in runs): runs of the length that
+// gives two workgroups per CU the same work, at least F32_MIN_RUN tiles, at most
 // F32_MAX_RUNS of them, whose partials the merge adds one after another.
-constexpr int F32_MIN_RUN = 4, F32_MAX_RUNS = 32;
+//
+// They are taken where this estimate says that they pay, from the prefill's tile
+// time tile_us (a workgroup alone on its CU; those that share one take turns).
+// Whole, a launch lasts as long as its longest block or an even share of the
+// tiles.  Split, it lasts one run if the runs have a CU each, else the even share,
+// the run that ends last, and a tile for each run's start; then 5 us for the merge
+// and the partials' way to memory and back at 3 TB/s.  Over 110 launches of 1 to 496
+// workgroups no split it takes was slower than the whole launch; without it 22 were:
+// B16 1/1 heads S3863 D128 (496 workgroups) 703 us whole and 1002 split, B1 16/8 S2000
+// D128 320 and 348, B3 64/16 S277 D32 22 and 29.  Below ~12 us of tiles a call is as
+// long as the host takes to launch it, and a second launch only adds to that.
+constexpr int F32_MIN_RUN = 3, F32_MAX_RUNS = 32;
 struct KeyRuns { int n, len; };
-inline KeyRuns f32_key_runs(int B, int Hq, int Hkv, int S, int T) {
+inline KeyRuns f32_key_runs(int B, int Hq, int Hkv, int S, int T, int D) {
   if (128 % (Hq / Hkv)) return {1, 1};
   const int BM = 128 / (Hq / Hkv);
   const int64_t wgs = (int64_t)B * Hkv * ((S + BM - 1) / BM);
   const int64_t most = ((int64_t)T + 31) / 32;
   if (wgs >= 512) return {1, 1};
-  int64_t len = (wgs * ((int64_t)T - (S < T ? S : T) / 2) / 32 + 511) / 512;  // a causal row's keys on average
+  const int64_t tiles = wgs * ((int64_t)T - (S < T ? S : T) / 2) / 32;  // a causal row's keys on average
+  int64_t len = (tiles + 511) / 512;
   if (len < F32_MIN_RUN) len = F32_MIN_RUN;
   if (len * F32_MAX_RUNS < most) len = (most + F32_MAX_RUNS - 1) / F32_MAX_RUNS;
-  return {(int)((most + len - 1) / len), (int)len};
+  const double tile_us = D == 32 ? 1.62 : D == 64 ? 2.78 : 5.05;
+  const double share = tiles / 256.0, each = (double)((most + len - 1) / len);
+  const double mean = (double)tiles / wgs / len + 0.5;
+  const double runs = wgs * (mean < each ? mean : each);
+  const double whole = (most > share ? most : share) * tile_us;
+  const double split = (runs <= 256 ? len : share + len + runs / 256) * tile_us + 5.0 + runs * 1024 * D / 3e6;
+  if (whole < 12.4 || split >= whole) return {1, 1};
+  return {(int)each, (int)len};
 }
 // Floats of one workgroup's partial accumulators, 4 waves of 32 rows.
 constexpr int64_t f32_part(int D) { return 128 * (int64_t)D; }

@@ -179,3 +179,19 @@ def test_bench_refuses_more_than_one_gpu():
                        capture_output=True, text=True, timeout=120, cwd=ROOT)
     assert r.returncode == 2
     assert "one GPU" in r.stderr and r.stdout == ""
+
+
+@pytest.mark.parametrize("B,Hq,Hkv,S,T,D,splits", [
+    (1, 8, 2, 1, 129, 64, True),       # five tiles
+    (1, 8, 2, 1, 160, 32, False),      # five tiles, too short for a second launch
+    (2, 8, 2, 1000, 1000, 64, True),   # 128 workgroups
+    (16, 1, 1, 3863, 3985, 128, False),  # 496, evenly loaded as they are
+    (1, 16, 8, 2000, 2000, 128, False),  # 256 of 16 to 63 tiles, two rounds of runs
+    (3, 64, 16, 277, 277, 32, False),    # 432 of up to nine tiles
+    (4, 64, 4, 1, 8000, 128, True),      # 16 long rows
+    (512, 8, 1, 1, 8000, 128, False),    # two workgroups per CU
+])
+def test_fp32_prefill_splits_where_it_pays(B, Hq, Hkv, S, T, D, splits):
+    """fp32 prefills of few workgroups split their keys unless the runs and the merge take longer."""
+    need = _lib.load().nq_attn_prefill_workspace_bytes(B, Hq, Hkv, S, T, D, _lib.NQ_DTYPE_F32)
+    assert (need > 0) == splits
