@@ -61,17 +61,22 @@ struct PrefillParams {
 // gives two workgroups per CU the same work, at least F32_MIN_RUN tiles, at most
 // F32_MAX_RUNS of them, whose partials the merge adds one after another.
 //
-// They are taken where this estimate says that they pay, from the prefill's tile
-// time tile_us (a workgroup alone on its CU; those that share one take turns).
-// Whole, a launch lasts as long as its longest block or an even share of the
-// tiles.  Split, it lasts one run if the runs have a CU each, else the even share,
-// the run that ends last, and a tile for each run's start; then 5 us for the merge
-// and the partials' way to memory and back at 3 TB/s.  Over 110 launches of 1 to 496
-// workgroups no split it takes was slower than the whole launch; without it 22 were:
-// B16 1/1 heads S3863 D128 (496 workgroups) 703 us whole and 1002 split, B1 16/8 S2000
-// D128 320 and 348, B3 64/16 S277 D32 22 and 29.  Below ~12 us of tiles a call is as
-// long as the host takes to launch it, and a second launch only adds to that.
-constexpr int F32_MIN_RUN = 3, F32_MAX_RUNS = 32;
+// They are taken where this estimate says that they pay.  Unit: the prefill's time
+// for a tile of a workgroup that has its CU to itself, tile_us (dQ's products are in
+// the same proportion).  Whole, a launch lasts as long as its longest block or an
+// even share of all tiles.  Split, it lasts
+//   - one run where every run has a CU to itself;
+//   - up to `fit` runs per CU (by registers): two runs, as they take turns, or the share;
+//   - beyond that the share, and on average half of a run that ends last; at D = 128,
+//     where fit is 1, and a multiple of 4 runs per block, the first runs of all blocks
+//     come to lie on the same CUs, and the launch lasts as if every block had them all;
+// and 5 us for the merge launch, and the partials' way out and back at 4 TB/s.
+// Of 200 prefills drawn at random, 1 to 511 workgroups, none is 2% slower than whole
+// (22 of 110 were without this) and they take 0.56 of the time.  Left out are, whole /
+// split: B16 1/1 heads S3863 D128 703 / 1002 us, B1 16/2 S2461 D128 392 / 537, B16 8/1
+// S239 D128 50 / 63, B3 64/16 S277 D32 22 / 29.  Below ~12 us of tiles a call lasts as
+// long as the host takes to launch it, and a second launch adds to that.
+constexpr int F32_MIN_RUN = 4, F32_MAX_RUNS = 32;
 struct KeyRuns { int n, len; };
 inline KeyRuns f32_key_runs(int B, int Hq, int Hkv, int S, int T, int D) {
   if (128 % (Hq / Hkv)) return {1, 1};
@@ -81,16 +86,21 @@ inline KeyRuns f32_key_runs(int B, int Hq, int Hkv, int S, int T, int D) {
   if (wgs >= 512) return {1, 1};
   const int64_t tiles = wgs * ((int64_t)T - (S < T ? S : T) / 2) / 32;  // a causal row's keys on average
   int64_t len = (tiles + 511) / 512;
-  if (len < F32_MIN_RUN) len = F32_MIN_RUN;
+  const int least = most <= 6 ? 3 : F32_MIN_RUN;
+  if (len < least) len = least;
   if (len * F32_MAX_RUNS < most) len = (most + F32_MAX_RUNS - 1) / F32_MAX_RUNS;
+  const int64_t n = (most + len - 1) / len;
+  const int fit = D == 32 ? 4 : D == 64 ? 2 : 1;
   const double tile_us = D == 32 ? 1.62 : D == 64 ? 2.78 : 5.05;
-  const double share = tiles / 256.0, each = (double)((most + len - 1) / len);
-  const double mean = (double)tiles / wgs / len + 0.5;
-  const double runs = wgs * (mean < each ? mean : each);
-  const double whole = (most > share ? most : share) * tile_us;
-  const double split = (runs <= 256 ? len : share + len + runs / 256) * tile_us + 5.0 + runs * 1024 * D / 3e6;
-  if (whole < 12.4 || split >= whole) return {1, 1};
-  return {(int)each, (int)len};
+  const double share = tiles / 256.0, mean = (double)tiles / wgs / len + 1;
+  const double runs = wgs * (mean < n ? mean : n);
+  const double whole = most > share ? most : share;
+  double split = len;
+  if (runs > 256 * fit) split = share + 0.5 * len / fit;
+  else if (runs > 256) split = 2 * len > share ? 2 * len : share;
+  if (fit == 1 && n % 4 == 0 && runs > 256 && wgs * n * len > 256 * split) split = wgs * n * len / 256.0;
+  if (whole * tile_us < 12.4 || split * tile_us + 5.0 + runs * 1024 * D / 4e6 >= whole * tile_us) return {1, 1};
+  return {(int)n, (int)len};
 }
 // Floats of one workgroup's partial accumulators, 4 waves of 32 rows.
 constexpr int64_t f32_part(int D) { return 128 * (int64_t)D; }
