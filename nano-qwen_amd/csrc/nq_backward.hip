@@ -817,28 +817,49 @@ extern "C" int64_t nq_attn_bwd_workspace_bytes(int B, int Hq, int S) {
 }
 
 // How dK/dV splits the key blocks' steps when there are fewer blocks than CUs:
-// runs of the length that gives every resident workgroup the same work (at least
-// DKDV_MIN_RUN steps, ~25 us), where some block is longer than that.  fp32 B2
-// S1000 8/2 heads D64, 32 blocks of up to 128 steps: 666 us whole, 93 + 6 for the
-// merge in runs of 16.  From a block per CU on the sums keep the query order, so
-// that a sequence's gradients do not depend on the batch it is in.
+// runs of the length that gives every resident workgroup the same work, at least
+// DKDV_MIN_RUN steps.  fp32 B2 S1000 8/2 heads D64, 32 blocks of up to 128 steps: 666
+// us whole, 93 + 6 for the merge in runs of 16.  The runs follow from the launch's
+// block count, so that a sequence's gradients depend in their last bits on the batch
+// it is in; from a block per CU on nothing is split and they do not.
+//
+// They are taken where they pay: whole, a launch lasts as long as its longest block;
+// split, a run or the CUs' even share of the steps, where every block has all its
+// steps (no causal mask) and the runs do not fit at once, as many equal runs as
+// there are rounds.  The steps saved, step_us each, are set against the merge: 3.5 us
+// and the partials' way out and back at 4 TB/s.  Left out so, whole / split: fp32 B4
+// 8/4 heads S986 T1059 D128 full 928 / 1037 us, bf16 B8 2/2 S543 D64 full 37 / 42,
+// B4 8/8 S750 D128 full 80 / 84.
 struct DkdvSplit { int nsplit, run; };
 constexpr int DKDV_MIN_RUN = 16;
 static DkdvSplit dkdv_split(int B, int Hq, int Hkv, int S, int T, int D, int dtype, bool causal) {
   const int G = Hq / Hkv, nkb = (T + BW_KEYS - 1) / BW_KEYS;
+  const int64_t pairs = (int64_t)B * Hkv;
+  if (nkb * pairs >= 256) return {1, 1};
+  auto steps = [&](int i) {
+    const int lo = i * BW_KEYS - (T - S), q = causal && lo > 0 ? lo / BW_BQ * BW_BQ : 0;
+    return q < S ? (int64_t)G * ((S - q + BW_BQ - 1) / BW_BQ) : 0;
+  };
   int64_t total = 0, most = 0;
   for (int i = 0; i < nkb; ++i) {
-    const int lo = i * BW_KEYS - (T - S), q = causal && lo > 0 ? lo / BW_BQ * BW_BQ : 0;
-    const int64_t steps = q < S ? (int64_t)G * ((S - q + BW_BQ - 1) / BW_BQ) : 0;
-    total += steps;
-    if (steps > most) most = steps;
+    total += steps(i) * pairs;
+    if (steps(i) > most) most = steps(i);
   }
+  const bool f32 = dtype == NQ_DTYPE_F32;
   // resident workgroups: 256 CUs x (bf16 D = 64: 3, else 2; fp32: 1)
-  const int slots = 256 * (dtype == NQ_DTYPE_F32 ? 1 : (D == 64 ? 3 : 2));
-  const int64_t even = (total * B * Hkv + slots - 1) / slots;
+  const int slots = 256 * (f32 ? 1 : (D == 64 ? 3 : 2));
+  const int64_t even = (total + slots - 1) / slots;
   const int64_t run = even > DKDV_MIN_RUN ? even : DKDV_MIN_RUN;
-  if ((int64_t)nkb * B * Hkv >= 256 || run >= most || most > 0x7fffffff) return {1, 1};
-  return {(int)((most + run - 1) / run), (int)run};
+  if (run >= most || most > 0x7fffffff) return {1, 1};
+  int64_t runs = 0;
+  for (int i = 0; i < nkb; ++i) runs += (steps(i) + run - 1) / run * pairs;
+  const int64_t each = (most + run - 1) / run;
+  double split = run;
+  if (!causal && runs > slots) split = (double)((runs + slots - 1) / slots) * ((most + each - 1) / each);
+  if (total > 256 * split) split = total / 256.0;
+  const double step_us = f32 ? (D == 32 ? 4.2 : D == 64 ? 5.8 : 10.6) : (D == 32 ? 0.8 : D == 64 ? 1.1 : 1.6);
+  if ((most - split) * step_us <= 3.5 + runs * 2048 * D / 4e6) return {1, 1};
+  return {(int)each, (int)run};
 }
 
 extern "C" int64_t nq_attn_bwd_split_workspace_bytes(int B, int Hq, int Hkv, int S, int T, int D, int dtype,

@@ -195,3 +195,21 @@ def test_fp32_prefill_splits_where_it_pays(B, Hq, Hkv, S, T, D, splits):
     """fp32 prefills of few workgroups split their keys unless the runs and the merge take longer."""
     need = _lib.load().nq_attn_prefill_workspace_bytes(B, Hq, Hkv, S, T, D, _lib.NQ_DTYPE_F32)
     assert (need > 0) == splits
+
+
+@pytest.mark.parametrize("dt,B,Hq,Hkv,S,T,D,causal,splits", [
+    (_lib.NQ_DTYPE_BF16, 1, 8, 2, 545, 545, 64, 1, True),
+    (_lib.NQ_DTYPE_BF16, 8, 2, 2, 543, 543, 64, 0, False),    # 17 steps: a run of 16 saves one
+    (_lib.NQ_DTYPE_BF16, 4, 8, 8, 750, 750, 128, 0, False),   # 192 even blocks
+    (_lib.NQ_DTYPE_BF16, 1, 16, 16, 1522, 1522, 128, 1, True),  # 192 blocks of 1 to 48 steps
+    (_lib.NQ_DTYPE_F32, 4, 8, 8, 750, 750, 128, 0, False),    # two rounds of half a block
+    (_lib.NQ_DTYPE_BF16, 8, 32, 8, 1024, 1024, 128, 1, False),  # two blocks per CU
+])
+def test_dkdv_splits_where_it_pays(dt, B, Hq, Hkv, S, T, D, causal, splits):
+    """dK/dV launches of fewer blocks than CUs split their steps unless the runs and the merge take longer."""
+    lib = _lib.load()
+    need = lib.nq_attn_bwd_split_workspace_bytes(B, Hq, Hkv, S, T, D, dt, causal)
+    base = lib.nq_attn_bwd_workspace_bytes(B, Hq, S)
+    if dt == _lib.NQ_DTYPE_F32:  # dQ's partials use the same memory
+        base += lib.nq_attn_prefill_workspace_bytes(B, Hq, Hkv, S, T, D, dt) * D // (D + 2)
+    assert (need > base) == splits
