@@ -870,7 +870,7 @@ extern "C" int64_t nq_attn_bwd_split_workspace_bytes(int B, int Hq, int Hkv, int
   const int64_t nkb = (T + BW_KEYS - 1) / BW_KEYS;
   int64_t part = sp.nsplit > 1 ? nkb * B * Hkv * sp.nsplit * (BW_KEYS * 2 * (int64_t)D) : 0;
   if (dtype == NQ_DTYPE_F32) {  // dQ's partials, in the same memory before dK/dV's
-    const KeyRuns kr = f32_key_runs(B, Hq, Hkv, S, T, D);
+    const KeyRuns kr = f32_key_runs(B, Hq, Hkv, S, T, D, true, causal != 0);
     if (kr.n > 1) {
       const int BM = 128 / (Hq / Hkv);
       const int64_t dq = (int64_t)B * Hkv * ((S + BM - 1) / BM) * kr.n * f32_part(D);
@@ -978,7 +978,7 @@ static int bwd_entry(const void* q, const int64_t* q_strides, const void* k, con
     }
     p.part = p.ws + need / (int64_t)sizeof(float);  // need is a multiple of 256
     if (f32) {
-      const KeyRuns kr = f32_key_runs(B, Hq, Hkv, S, T, D);
+      const KeyRuns kr = f32_key_runs(B, Hq, Hkv, S, T, D, true, causal != 0);
       p.qsplit = kr.n;
       p.qrun = kr.len;
     }

@@ -1019,7 +1019,8 @@ static int prefill_entry(const void* q, const int64_t* q_strides, const void* k,
   if (f32) {
     p.BM = 128 / G;
     p.nqb = (S + p.BM - 1) / p.BM;
-    const KeyRuns kr = workspace && !key_lens && !bias ? f32_key_runs(B, Hq, Hkv, S, T, D) : KeyRuns{1, 1};
+    KeyRuns kr = workspace && !key_lens && !bias ? f32_key_runs(B, Hq, Hkv, S, T, D) : KeyRuns{1, 1};
+    if (!causal && f32_key_runs(B, Hq, Hkv, S, T, D, false, false).n == 1) kr = {1, 1};
     p.nsplit = kr.n;
     p.run = kr.len;
     if (p.nsplit > 1) {

@@ -61,44 +61,49 @@ struct PrefillParams {
 // gives two workgroups per CU the same work, at least F32_MIN_RUN tiles, at most
 // F32_MAX_RUNS of them, whose partials the merge adds one after another.
 //
-// They are taken where this estimate says that they pay.  Unit: the prefill's time
-// for a tile of a workgroup that has its CU to itself, tile_us (dQ's products are in
-// the same proportion).  Whole, a launch lasts as long as its longest block or an
+// They are taken where this estimate says that they pay.  Unit: the time for a tile
+// of a workgroup that has its CU to itself, tile_us; dQ takes twice the prefill's.  The
+// prefill's workspace is sized without knowing the mask, so that counts on a causal
+// one; a full launch then leaves it unused where its own estimate says so.  Whole, a launch lasts as long as its longest block or an
 // even share of all tiles.  Split, it lasts
 //   - one run where every run has a CU to itself;
 //   - up to `fit` runs per CU (by registers): two runs, as they take turns, or the share;
-//   - beyond that the share, and on average half of a run that ends last; at D = 128,
-//     where fit is 1, and a multiple of 4 runs per block, the first runs of all blocks
-//     come to lie on the same CUs, and the launch lasts as if every block had them all;
+//   - beyond that the share, and on average half of a run that ends last;
+//   - with a multiple of 4 runs per causal block, where they have no CU each and fit <= 2:
+//     the first runs of all blocks come to lie on the same CUs, and the launch lasts as
+//     if every block had them all;
 // and 5 us for the merge launch, and the partials' way out and back at 4 TB/s.
 // Of 200 prefills drawn at random, 1 to 511 workgroups, none is 2% slower than whole
 // (22 of 110 were without this) and they take 0.56 of the time.  Left out are, whole /
 // split: B16 1/1 heads S3863 D128 703 / 1002 us, B1 16/2 S2461 D128 392 / 537, B16 8/1
-// S239 D128 50 / 63, B3 64/16 S277 D32 22 / 29.  Below ~12 us of tiles a call lasts as
+// S239 D128 50 / 63, B3 64/16 S277 D32 22 / 29; the backward by dQ's, B16 32/4 S53 T172
+// D128 241 / 262, B4 8/1 S1239 D64 1779 / 1825.  Below ~12 us of tiles a call lasts as
 // long as the host takes to launch it, and a second launch adds to that.
 constexpr int F32_MIN_RUN = 4, F32_MAX_RUNS = 32;
 struct KeyRuns { int n, len; };
-inline KeyRuns f32_key_runs(int B, int Hq, int Hkv, int S, int T, int D) {
+inline KeyRuns f32_key_runs(int B, int Hq, int Hkv, int S, int T, int D, bool dq = false, bool causal = true) {
   if (128 % (Hq / Hkv)) return {1, 1};
   const int BM = 128 / (Hq / Hkv);
   const int64_t wgs = (int64_t)B * Hkv * ((S + BM - 1) / BM);
   const int64_t most = ((int64_t)T + 31) / 32;
   if (wgs >= 512) return {1, 1};
-  const int64_t tiles = wgs * ((int64_t)T - (S < T ? S : T) / 2) / 32;  // a causal row's keys on average
-  int64_t len = (tiles + 511) / 512;
+  const int64_t half = wgs * ((int64_t)T - (S < T ? S : T) / 2) / 32;  // a causal row's keys on average
+  int64_t len = (half + 511) / 512;
   const int least = most <= 6 ? 3 : F32_MIN_RUN;
   if (len < least) len = least;
   if (len * F32_MAX_RUNS < most) len = (most + F32_MAX_RUNS - 1) / F32_MAX_RUNS;
   const int64_t n = (most + len - 1) / len;
   const int fit = D == 32 ? 4 : D == 64 ? 2 : 1;
-  const double tile_us = D == 32 ? 1.62 : D == 64 ? 2.78 : 5.05;
-  const double share = tiles / 256.0, mean = (double)tiles / wgs / len + 1;
+  const double tile_us = (D == 32 ? 1.62 : D == 64 ? 2.78 : 5.05) * (dq ? 2 : 1);
+  const double tiles = causal ? half : wgs * (T / 32.0), share = tiles / 256;
+  const double mean = tiles / wgs / len + (dq ? 0.5 : 1);  // runs of a block
   const double runs = wgs * (mean < n ? mean : n);
-  const double whole = most > share ? most : share;
+  double whole = most > share ? most : share;
+  if (!causal && fit == 1) whole = (double)((wgs + 255) / 256 * most);  // all blocks alike
   double split = len;
   if (runs > 256 * fit) split = share + 0.5 * len / fit;
   else if (runs > 256) split = 2 * len > share ? 2 * len : share;
-  if (fit == 1 && n % 4 == 0 && runs > 256 && wgs * n * len > 256 * split) split = wgs * n * len / 256.0;
+  if (causal && fit <= 2 && n % 4 == 0 && runs > 256 && wgs * n * len > 256 * split) split = wgs * n * len / 256.0;
   if (whole * tile_us < 12.4 || split * tile_us + 5.0 + runs * 1024 * D / 4e6 >= whole * tile_us) return {1, 1};
   return {(int)n, (int)len};
 }
