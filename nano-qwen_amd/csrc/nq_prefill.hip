@@ -918,15 +918,22 @@ static int64_t prefill_wgs4(int B, int Hq, int Hkv, int S) {
   return BM > 0 ? (int64_t)B * Hkv * ((S + BM - 1) / BM) : 0;
 }
 
-// Workgroups per query block that the keys are split over: as many as the
-// device holds, two per CU.  A launch of up to half a workgroup per CU gains
-// from runs of 6 tiles on (B1 32/8 heads D128, 16 queries on 1000 keys: 19.7 ->
-// 17.2 us; 500 on 12345: 180 -> 112), up to 16 of them (16 queries on 12000 keys:
-// 165 us whole, 36 at 15 runs, 46 at 31, whose merge takes longer).  Above that a
-// split only puts a second workgroup on each CU: 2 x 500 queries on 2000 keys,
-// 32/4 heads, 35 tiles in two went 45.8 -> 50.7 us, 250 tiles 327 -> 307.
+// Workgroups per query block that the keys are split over: as many as the device
+// holds, two per CU, in runs of at least 6 tiles, up to 16 of them (B1 32/8 heads
+// D128, 16 queries on 1000 keys: 19.7 -> 17.2 us; 500 on 12345: 180 -> 112; 16 on 12000:
+// 165 us whole, 36 at 15 runs, 46 at 31, whose merge takes longer).  From half a
+// workgroup per CU on the second runs share CUs, and 32 tiles are the least (two runs
+// at D128: 136 workgroups of 17 tiles 22.2 -> 24.4 us, 160 of 24 28.3 -> 32.5, 180 of
+// 30 36.5 -> 41.5, 162 of 113 109.5 -> 82.2; 256 of 35 45.8 -> 50.7, of 250 327 -> 307).
+//
+// And only where this estimate says that they pay: a tile takes 0.5 to 0.88 us, a fifth
+// more where runs share a CU, or as long as the K and V tiles of all pairs and runs take
+// at 5 TB/s (query blocks of a pair find each other's in the L2); the merge launch takes
+// 6 us and the partials' way out and back 8 TB/s.  Left out so, whole / split, D128 but
+// for the first: 2 queries of 8 x 16 heads on 1193 keys D64 17.8 / 20.0 us; one query of
+// 16 x 8 heads on 1000 20.9 / 23.6; 64 of 4 x 32/8 on 900 20.4 / 22.5.
 constexpr int PF_SPLIT_SLOTS = 512, PF_SPLIT_MAX = 16;
-static int prefill_splits(int B, int Hq, int Hkv, int S, int T) {
+static int prefill_splits(int B, int Hq, int Hkv, int S, int T, int D) {
   if (128 % (Hq / Hkv)) return 1;
   const int64_t wgs = prefill_wgs4(B, Hq, Hkv, S);
   const int64_t fit = PF_SPLIT_SLOTS / wgs;
@@ -934,7 +941,15 @@ static int prefill_splits(int B, int Hq, int Hkv, int S, int T) {
   const int64_t most = (T - S / 2) / (PF_BN * tiles);  // T - S/2: a causal row's keys on average
   int64_t n = fit < most ? fit : most;
   if (n > PF_SPLIT_MAX) n = PF_SPLIT_MAX;
-  return n > 1 ? (int)n : 1;
+  if (n < 2) return 1;
+  auto tile_us = [&](int64_t runs) {  // per query block
+    const double alone = (D == 32 ? 0.5 : D == 64 ? 0.63 : 0.88) * (wgs * runs > 256 ? 1.2 : 1.0);
+    const double fed = (double)B * Hkv * runs * 256 * D / 5e6;
+    return alone > fed ? alone : fed;
+  };
+  const double m = (double)T / PF_BN;  // tiles of the longest block
+  const double split = m / n * tile_us(n) + 6.0 + wgs * n * 1024 * D / 8e6;
+  return split < m * tile_us(1) ? (int)n : 1;
 }
 
 // Shared by the dense, paged and bias entry points: bt == NULL for dense K/V,
@@ -1039,7 +1054,7 @@ static int prefill_entry(const void* q, const int64_t* q_strides, const void* k,
   const int nw = (128 % G == 0 && (wide_wgs < PF_WIDE_MIN_WGS || D == 32 || bias)) ? 4 : 8;
   p.BM = 32 * nw / G;
   p.nqb = (S + p.BM - 1) / p.BM;
-  p.nsplit = workspace && !key_lens && !bias ? prefill_splits(B, Hq, Hkv, S, T) : 1;
+  p.nsplit = workspace && !key_lens && !bias ? prefill_splits(B, Hq, Hkv, S, T, D) : 1;
   if (p.nsplit > 1) {
     const int64_t need = pf_split_bytes((int64_t)p.nqb * B * Hkv, p.nsplit, D);
     if (workspace_bytes < need || !nq_aligned16(workspace))
@@ -1059,7 +1074,7 @@ extern "C" int64_t nq_attn_prefill_workspace_bytes(int B, int Hq, int Hkv, int S
     const KeyRuns kr = f32_key_runs(B, Hq, Hkv, S, T, D);  // 128 rows' accumulators, max and sum per workgroup
     return kr.n > 1 ? prefill_wgs4(B, Hq, Hkv, S) * kr.n * (f32_part(D) + 256) * (int64_t)sizeof(float) : 0;
   }
-  const int ns = prefill_splits(B, Hq, Hkv, S, T);
+  const int ns = prefill_splits(B, Hq, Hkv, S, T, D);
   return ns > 1 ? pf_split_bytes(prefill_wgs4(B, Hq, Hkv, S), ns, D) : 0;
 }
 

@@ -213,3 +213,17 @@ def test_dkdv_splits_where_it_pays(dt, B, Hq, Hkv, S, T, D, causal, splits):
     if dt == _lib.NQ_DTYPE_F32:  # dQ's partials use the same memory
         base += lib.nq_attn_prefill_workspace_bytes(B, Hq, Hkv, S, T, D, dt) * D // (D + 2)
     assert (need > base) == splits
+
+
+@pytest.mark.parametrize("B,Hq,Hkv,S,T,D,splits", [
+    (1, 32, 8, 500, 12345, 128, True),   # 128 workgroups, long
+    (4, 32, 8, 64, 900, 128, False),     # 64, two runs of seven tiles
+    (16, 32, 8, 1, 1000, 128, False),    # 128 that stream keys of their own
+    (8, 16, 16, 2, 1193, 64, False),     # 128 of 19 short tiles
+    (8, 32, 8, 1, 4000, 128, True),      # 64 of 63 tiles
+    (1, 32, 8, 520, 2000, 128, False),   # 136 of 32 tiles
+])
+def test_prefill_splits_where_it_pays(B, Hq, Hkv, S, T, D, splits):
+    """bf16 prefills of few workgroups split their keys unless the runs and the merge take longer."""
+    need = _lib.load().nq_attn_prefill_workspace_bytes(B, Hq, Hkv, S, T, D, _lib.NQ_DTYPE_BF16)
+    assert (need > 0) == splits
