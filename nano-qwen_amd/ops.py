@@ -537,17 +537,29 @@ def decode_workspace_bytes(B: int, Hq: int, Hkv: int, D: int, max_len: int, chun
     return int(_lib.load().nq_attn_decode_workspace_bytes(B, Hq, Hkv, D, max_len, chunk))
 
 
+# Microseconds per 32 keys of an fp32 decode that walks a sequence's keys whole.
+_F32_TILE_US = {32: 1.62, 64: 2.78, 128: 5.05}
+
+
 def _decode_workspace(workspace: Optional[torch.Tensor], dt: int, B: int, Hq: int, Hkv: int, D: int,
-                      max_len: int, chunk: int, dev):
-    """The workspace of a decode's partials (the caller's when it is large enough), and the
-    call's dtype code.  An fp32 decode takes one of its own: its callers may hand the same
-    workspace to calls that overlap, which an fp32 cache never read."""
+                      max_len: int, chunk: int, dev, append: bool):
+    """The workspace of a decode's partials (the caller's when it is large enough), its bytes,
+    and the call's dtype code.  An fp32 decode takes one of its own: its callers may hand the
+    same workspace to calls that overlap, which an fp32 cache never read."""
     need = decode_workspace_bytes(B, Hq, Hkv, D, max_len, chunk)
     if dt == _lib.NQ_DTYPE_F32:
-        return torch.empty(max(need, 16), dtype=torch.uint8, device=dev), dt | _lib.NQ_DECODE_F32_SPLIT
+        # Short caches are walked whole, in one launch where the split takes two: 5 us
+        # and the tiles, times the rounds of (sequence, kv head) pairs, against the ~16.5 us
+        # in which the host makes two launches (B16 8/2 heads D64 with 100 keys of 128: 15.1
+        # us whole and 17.0 split; 32/8 heads D128, 24.8 and 17.1).  With an append
+        # either form takes two.
+        walk = -(-max_len // 32) * _F32_TILE_US.get(D, 0.0) * max(1.0, B * Hkv / 256)
+        if not append and 5.0 + walk <= 16.5:
+            return workspace, 0 if workspace is None else workspace.numel() * workspace.element_size(), dt
+        workspace, dt = None, dt | _lib.NQ_DECODE_F32_SPLIT
     if workspace is None or workspace.numel() * workspace.element_size() < need:
         workspace = torch.empty(max(need, 16), dtype=torch.uint8, device=dev)
-    return workspace, dt
+    return workspace, workspace.numel() * workspace.element_size(), dt
 
 
 def attention_decode(q: torch.Tensor, k_cache: torch.Tensor, v_cache: torch.Tensor,
@@ -584,8 +596,7 @@ def attention_decode(q: torch.Tensor, k_cache: torch.Tensor, v_cache: torch.Tens
     if out is None:
         out = torch.empty(B, Hq, D, dtype=q.dtype, device=q.device)
     dev = q.device
-    workspace, dt = _decode_workspace(workspace, dt, B, Hq, Hkv, D, max_len, chunk, dev)
-    wbytes = workspace.numel() * workspace.element_size()
+    workspace, wbytes, dt = _decode_workspace(workspace, dt, B, Hq, Hkv, D, max_len, chunk, dev, False)
     cos_t, sin_t, max_pos = _tables(cos, sin, dev)
     lens_t = _i32(lens, dev)
     qp = _decode_q_pos(q_pos, q_pos0, B, max_pos, dev)
@@ -741,8 +752,7 @@ def attention_decode_paged(q: torch.Tensor, k_pool: torch.Tensor, v_pool: torch.
             raise ValueError("lens_out must not alias lens")
     if out is None:
         out = torch.empty(B, Hq, D, dtype=q.dtype, device=dev)
-    workspace, dt = _decode_workspace(workspace, dt, B, Hq, Hkv, D, max_len, chunk, dev)
-    wbytes = workspace.numel() * workspace.element_size()
+    workspace, wbytes, dt = _decode_workspace(workspace, dt, B, Hq, Hkv, D, max_len, chunk, dev, k_new is not None)
     cos_t, sin_t, max_pos = _tables(cos, sin, dev)
     qp = _decode_q_pos(q_pos, q_pos0, B, max_pos, dev)
     qw, qf = _norm_weight(q_weight, dev, dt, _lib.NQ_QWEIGHT_BF16, plan)

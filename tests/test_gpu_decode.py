@@ -4,6 +4,7 @@ import pytest
 import torch
 
 import nano_qwen_amd as nq
+from nano_qwen_amd import ops
 from oracle import decode_path, rope_tables
 from tests.helpers import assert_bf16_close, assert_close_for, randn, say
 
@@ -189,3 +190,21 @@ def test_decode_f32_scores_overflowing(D, dropped):
         gone = drop | (torch.arange(T) >= lens.view(B, 1, 1, 1, 1))
         ref = (torch.softmax(sc.masked_fill(gone, float("-inf")), -1) @ vc.double()[:, :, None]).view(B, Hq, D)
         assert_close_for(torch.float32, o, ref, f"chunk={chunk}")
+
+
+@pytest.mark.parametrize("D,whole", [(32, 224), (64, 128), (128, 64)])
+def test_decode_f32_short_caches(D, whole):
+    """fp32 caches of up to ``whole`` keys are walked whole, longer ones split: at the line and beyond, every length."""
+    for cap in (1, 32, whole, whole + 1, 300):
+        say(f"fp32 decode D={D} cap={cap}")
+        lens = torch.tensor([cap, 1, max(1, cap // 2), 0], dtype=torch.int32)
+        q, kc, vc = (randn(4, *s, D, seed=101 + i) for i, s in enumerate(((8,), (2, cap), (2, cap))))
+        _poison_tail(kc, lens), _poison_tail(vc, lens)
+        _, _, dt = ops._decode_workspace(None, ops._code(q), 4, 8, 2, D, cap, 0, torch.device(DEV), False)
+        assert (dt == ops._code(q)) == (cap <= whole)
+        o = nq.attention_decode(q.to(DEV), kc.to(DEV), vc.to(DEV), lens.to(DEV), max_len=cap)
+        qd = q.double().view(4, 2, 4, 1, D)
+        sc = (qd @ kc.nan_to_num().double()[:, :, None].transpose(-1, -2) / D ** 0.5)
+        sc = sc.masked_fill(torch.arange(cap) >= lens.view(4, 1, 1, 1, 1), float("-inf"))
+        ref = (torch.softmax(sc, -1).nan_to_num() @ vc.nan_to_num().double()[:, :, None]).view(4, 8, D)
+        assert_close_for(torch.float32, o, ref, f"cap={cap}")
