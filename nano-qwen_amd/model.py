@@ -70,13 +70,29 @@ class LayerRMSNorm(nn.Module):
         # pass over fp32 rows: a training block at 4096 x 2048 bf16, with SwiGLU's
         # product below, 2296 -> 1863 us; four layers on 173 tokens 1420 -> 1286 us
         if not torch.jit.is_scripting():
-            if ops.plain_rows(x, w) and w.dim() == 1 and x.shape[-1] == w.shape[0]:
-                if not (torch.is_grad_enabled() and (x.requires_grad or w.requires_grad)):
+            grad = ops.takes_gradient(x, w)
+            if (grad is not None and w.dim() == 1 and not (grad and w.shape[0] > 4096)
+                    and x.shape[-1:] == w.shape and ops.plain_rows(x, w)):
+                if not grad:
                     return plain_rms_norm(x, w, self.eps)
-                if w.shape[0] <= 4096:
-                    kept = self.input_kept or x.dtype == torch.float32
-                    return LayerRMSNormFn.apply(x if kept else x.clone(), w, self.eps)
+                kept = self.input_kept or x.dtype == torch.float32
+                return LayerRMSNormFn.apply(x if kept else x.clone(), w, self.eps)
         return layer_rms_norm(x, w, self.eps)
+
+
+def _swiglu_product(gate: torch.Tensor, up: torch.Tensor) -> torch.Tensor:
+    y = torch.empty_like(gate)
+    rc = _lib.load().nq_swiglu(ops._ptr(gate), ops._ptr(up), ops._ptr(y), gate.numel(), ops._code(gate),
+                               ops._stream(gate))
+    _lib.check(rc, "nq_swiglu")
+    return y
+
+
+# Elements of gate from which a product with a gradient goes through the kernels.  An
+# autograd function's calls take the host ~35 us longer than the tensor operations' (2048
+# rows of 1024 -> 3072, forward and backward: 344 us against 309); from here on the
+# device takes longer than the host, and its passes count (4096 rows: 351 against 375).
+_SWIGLU_GRAD_ELEMENTS = 1 << 23
 
 
 class _SwiGLUProduct(torch.autograd.Function):
@@ -85,11 +101,7 @@ class _SwiGLUProduct(torch.autograd.Function):
     @staticmethod
     def forward(ctx, gate, up):
         ctx.save_for_backward(gate, up)
-        y = torch.empty_like(gate)
-        rc = _lib.load().nq_swiglu(ops._ptr(gate), ops._ptr(up), ops._ptr(y), gate.numel(), ops._code(gate),
-                                   ops._stream(gate))
-        _lib.check(rc, "nq_swiglu")
-        return y
+        return _swiglu_product(gate, up)
 
     @staticmethod
     def backward(ctx, dy):
@@ -119,9 +131,10 @@ class SwiGLU(nn.Module):
     def forward(self, x: torch.Tensor) -> torch.Tensor:
         gate, up = self.gate_proj(x), self.up_proj(x)
         if not torch.jit.is_scripting():
-            # plain_rows first: the proxies of torch.fx's symbolic trace cannot be compared
-            if ops.plain_rows(gate, up) and gate.dtype == up.dtype and gate.shape == up.shape:
-                return self.down_proj(_SwiGLUProduct.apply(gate, up))
+            grad = ops.takes_gradient(gate, up)
+            if (grad is not None and not (grad and gate.numel() < _SWIGLU_GRAD_ELEMENTS)
+                    and gate.dtype == up.dtype and gate.shape == up.shape and ops.plain_rows(gate, up)):
+                return self.down_proj(_SwiGLUProduct.apply(gate, up) if grad else _swiglu_product(gate, up))
         return self.down_proj(F.silu(gate) * up)
 
 

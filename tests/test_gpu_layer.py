@@ -184,3 +184,24 @@ def test_swiglu_other_routes():
     torch.testing.assert_close(res[0], res[1], rtol=1e-3, atol=1e-5)
     gates = torch.tensor([float("inf"), float("-inf"), float("nan"), 0.0, -100.0, 100.0, 1e30, -1e30], device=DEV)
     torch.testing.assert_close(_SwiGLUProduct.apply(gates, torch.ones_like(gates)), F.silu(gates), equal_nan=True)
+
+
+@pytest.mark.parametrize("rows,kernel", [(8191, False), (8192, True)])
+def test_swiglu_route_by_size(rows, kernel):
+    """A product with a gradient goes through the kernels from 2^23 elements on, one without always; the values agree."""
+    say(f"SwiGLU of {rows} x 1024, with a gradient and without")
+    ffn = SwiGLU(64, 1024).to(DEV, BF)
+    seen = []
+    ffn.down_proj.register_forward_pre_hook(lambda mod, args: seen.append(args[0]))
+    x = randn(rows, 64, seed=42, dtype=BF).to(DEV).requires_grad_()
+    y = ffn(x)
+    assert seen[0].grad_fn.name().startswith("_SwiGLUProduct") == kernel
+    with torch.no_grad():
+        ffn(x)
+    # one route rounds silu(gate) as the other does, which may fall the other way
+    for p in seen:
+        _close(p, (F.silu(ffn.gate_proj(x).double()).to(BF).double() * ffn.up_proj(x).double()).detach().cpu(), BF, 1, "product")
+    (dx,) = torch.autograd.grad(y, x, torch.ones_like(y))
+    g, u = ffn.gate_proj(x), ffn.up_proj(x)
+    (want,) = torch.autograd.grad(ffn.down_proj(F.silu(g) * u), x, torch.ones_like(y))
+    _close(dx, want.double().cpu(), BF, 1, "dx")
