@@ -481,3 +481,44 @@ def test_split_keys_prefill_scores_overflowing(dtype, Hq, Hkv, D, S, T, dropped,
     # bf16: the query is rounded again after its scaling, 2^-9 of D products of unit variance
     torch.testing.assert_close(lse.cpu().double(), torch.logsumexp(sc, -1).view(1, Hq, S), rtol=0,
                                atol=2e-2 if dtype == torch.bfloat16 else 1e-5)
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("paged", [False, True])
+@pytest.mark.parametrize("causal", [True, False])
+@pytest.mark.parametrize("B,Hq,Hkv,D,S,T", [
+    (2, 8, 2, 128, 33, 2500),
+    (3, 4, 4, 64, 300, 2700),  # 12 pairs, several query blocks
+])
+def test_split_keys_prefill_batches(B, Hq, Hkv, D, S, T, causal, paged, dtype):
+    """Split prefills of several sequences: each has its own rows, keys, pages, outputs and LSE."""
+    say(f"split prefill B={B} {Hq}/{Hkv} D={D} S={S} T={T} causal={causal} paged={paged} {dtype}")
+    lib = ops._lib.load()
+    assert lib.nq_attn_prefill_workspace_bytes(B, Hq, Hkv, S, T, D, ops._code(torch.empty(0, dtype=dtype))) > 0
+    # sequences of unlike scale, so that a row of another one's shows
+    size = torch.arange(1, B + 1).view(B, 1, 1, 1)
+    q, k, v = (randn(B, H, n, D, seed=431 + i) for i, (H, n) in enumerate(((Hq, S), (Hkv, T), (Hkv, T))))
+    q, k, v = q.to(dtype), k.to(dtype), (v * size).to(dtype)
+    args = dict(causal=causal, return_lse=True)
+    if paged:
+        P = 64
+        n = -(-T // P)
+        kp, vp = (torch.full((B * n + 1, Hkv, P, D), float("nan"), dtype=dtype, device=DEV) for _ in range(2))
+        bt = torch.randperm(B * n + 1, generator=torch.Generator().manual_seed(435))[:B * n].to(torch.int32).view(B, n)
+        for src, pool in ((k, kp), (v, vp)):
+            for b in range(B):
+                for i in range(n):
+                    rows = src[b, :, i * P:(i + 1) * P].to(DEV)
+                    pool[int(bt[b, i]), :, :rows.shape[1]] = rows
+        o, lse = ops.attention_prefill_paged(q.to(DEV), kp, vp, bt.to(DEV), T=T, **args)
+    else:
+        o, lse = ops.attention_prefill(q.to(DEV), k.to(DEV), v.to(DEV), **args)
+    sc = q.double().view(B, Hkv, -1, S, D) @ k.double()[:, :, None].transpose(-1, -2) / D ** 0.5
+    if causal:
+        sc = sc.masked_fill(torch.arange(T) > torch.arange(S)[:, None] + T - S, float("-inf"))
+    ref = (torch.softmax(sc, -1) @ v.double()[:, :, None]).view(B, Hq, S, D)
+    for b in range(B):
+        assert_close_for(dtype, o[b] / (b + 1), ref[b] / (b + 1), f"sequence {b}")
+    # bf16: the query is rounded again after its scaling, 2^-9 of D products of unit variance
+    torch.testing.assert_close(lse.cpu().double(), torch.logsumexp(sc, -1).view(B, Hq, S), rtol=0,
+                               atol=2e-2 if dtype == torch.bfloat16 else 1e-5)
