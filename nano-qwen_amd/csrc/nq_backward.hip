@@ -396,8 +396,7 @@ __global__ void __launch_bounds__(256, D == 64 ? 3 : 2) bwd_dkdv_kernel(BwdParam
     // heaviest block gets the lightest as its other one (B2 32/8 heads D128, dK/dV
     // with dQ: 512 blocks 1228 -> 1127 us, 384 817 -> 772, 320 644 -> 625, 272 513 ->
     // 514; with the second half of the blocks reversed, those last took 664 and 560)
-    const int first = (256 + npairs - 1) / npairs;
-    if (CAUSAL && nkb * npairs > 256 && nkb * npairs <= 512 && kblk >= first) kblk = nkb - 1 - (kblk - first);
+    if (CAUSAL && kblk >= p.kblk_turn) kblk = nkb - 1 - (kblk - p.kblk_turn);
   }
   const int b = pair / p.Hkv, kvh = pair % p.Hkv;
   const int k0 = kblk * BW_KEYS;
@@ -969,6 +968,8 @@ static int bwd_entry(const void* q, const int64_t* q_strides, const void* k, con
   p.scale_log2 = p.scale * kLog2e;
   hipStream_t st = reinterpret_cast<hipStream_t>(stream);
   p.nsplit = p.run = p.qsplit = p.qrun = 1;
+  const int64_t pairs = (int64_t)B * Hkv, blocks = (T + BW_KEYS - 1) / BW_KEYS * pairs;
+  p.kblk_turn = blocks > 256 && blocks <= 512 ? (int)((256 + pairs - 1) / pairs) : INT32_MAX;
   if (!wide && !bias && nq_aligned16(workspace) &&
       workspace_bytes >= nq_attn_bwd_split_workspace_bytes(B, Hq, Hkv, S, T, D, dtype, causal)) {
     const DkdvSplit sp = dkdv_split(B, Hq, Hkv, S, T, D, dtype, causal != 0);

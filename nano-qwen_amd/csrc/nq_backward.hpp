@@ -40,6 +40,7 @@ struct BwdParams {
   // each (1 = none), whose partial sums go to part
   int nsplit, run;
   float* part;
+  int kblk_turn;  // bf16 dK/dV, causal: the rank from which key blocks go lightest first
   // fp32 dQ: a query block's key tiles split likewise (f32_key_runs), whose
   // partials use the same memory before it
   int qsplit, qrun;
