@@ -354,7 +354,7 @@ class AttnBias:
         Bm, Hm, Sm = m.shape[:3]
         self.shape = (B, Hq, S, T)
         if (m.dtype == torch.bool and m.is_cuda and dtype in _DTYPES and m.numel() > 0
-                and Bm * Hm * Sm * T < _MAX_ELEMENTS):
+                and Bm * Hm * Sm * T < _MAX_ELEMENTS and m.device.index == torch.cuda.current_device()):
             self.bias = torch.empty(Bm, Hm, Sm, -(-T // 8) * 8, dtype=dtype, device=device)
             strides = (ctypes.c_int64 * 4)(*m.expand(Bm, Hm, Sm, T).stride())
             _lib.check(_lib.load().nq_mask_bias(_ptr(m), strides, _ptr(self.bias), Bm, Hm, Sm, T, _DTYPES[dtype],
@@ -402,7 +402,9 @@ def attention_prefill(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, *,
     contiguous (B, S, Hq, D) buffer, so ``o.transpose(1, 2).reshape(B, S, -1)``
     (o_proj's input, model/attention.py:117) costs nothing.  With
     ``return_lse`` also returns the fp32 (B, Hq, S) log-sum-exp.  With
-    ``plan=True`` returns a KernelCall whose ``launch()`` runs it.
+    ``plan=True`` returns a KernelCall whose ``launch()`` runs it.  A call gives
+    the same bits each time; one of few query blocks splits its keys by the batch
+    size among other things, so a sequence's last bits depend on the batch it is in.
     """
     _require_device(q, k, v, out)
     B, Hq, S, D = q.shape
@@ -848,7 +850,10 @@ def attention_backward(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, o: tor
     the same causal, sm_scale, key_lens and bias; the bias built with
     ``transpose=True``).  dk/dv sum the gradients of the
     G query heads that share a kv head; keys past key_lens[b] get zeros.
-    Returns fresh (dq, dk, dv) in q's dtype.
+    Returns fresh (dq, dk, dv) in q's dtype, the same bits on every call; in a
+    launch of fewer than 256 key blocks (fp32 dQ: 512 query blocks) the sums are
+    split by the batch size among other things, so a sequence's last bits depend
+    on the batch it is in.
     """
     _require_device(q, k, v, o, dout, lse)
     B, Hq, S, D = q.shape

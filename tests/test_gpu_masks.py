@@ -488,3 +488,13 @@ def test_bool_mask_as_bias(shape, make, dtype):
     ref = ops.AttnBias(m, B, H, S, T, dtype, torch.device("cpu"), transpose=True)
     assert torch.equal(got.bias.cpu(), ref.bias) and torch.equal(got.bias_t.cpu(), ref.bias_t)
     assert got.strides == ref.strides and got.t_strides == ref.t_strides
+
+
+def test_mask_on_another_device_than_the_current_one(monkeypatch):
+    """A launch goes to the current device: the bias of a mask elsewhere is made by tensor operations there."""
+    mask = (torch.rand(2, 1, 5, 21, generator=torch.Generator().manual_seed(71)) > 0.4).to(DEV)
+    here = ops.AttnBias(mask, 2, 4, 5, 21, torch.bfloat16, mask.device)
+    monkeypatch.setattr(torch.cuda, "current_device", lambda: mask.device.index + 1)
+    monkeypatch.setattr(ops._lib, "load", lambda: pytest.fail("launched from another device"))
+    there = ops.AttnBias(mask, 2, 4, 5, 21, torch.bfloat16, mask.device)
+    assert torch.equal(here.bias, there.bias) and here.strides == there.strides
