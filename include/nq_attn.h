@@ -230,7 +230,10 @@ int nq_attn_prefill_paged_fwd(const void* q, const int64_t* q_strides, const voi
  * block's keys over several workgroups, whose fp32 partials a second launch
  * adds (no counterpart in the reference).  nq_attn_prefill_workspace_bytes
  * gives the bytes needed (16-byte aligned), 0 where the keys are not split: the
- * workspace is then not used, and NULL is accepted anywhere for no split.
+ * workspace is then not used, and NULL is accepted anywhere for no split.  The
+ * runs follow from B, the heads, S, T, D and the dtype: a call gives the same
+ * bits each time, but a sequence's last bits depend on the batch it is in
+ * (without a workspace they do not).
  * block_table NULL: k and v are dense as in nq_attn_prefill_fwd; else they are
  * pools as in nq_attn_prefill_paged_fwd.  The other arguments are theirs.
  */
@@ -406,6 +409,9 @@ int64_t nq_attn_bwd_workspace_bytes(int B, int Hq, int S);
  * adds in a fixed order.  At least nq_attn_bwd_workspace_bytes, and equal to it
  * where nothing is gained (long key ranges that fill the device evenly).  With
  * a smaller workspace (or one that is not 16-byte aligned) nothing is split.
+ * For fp32 dQ's keys are split likewise, its partials in the same memory.  The
+ * runs follow from the arguments: the bits are the same on every run, but in a
+ * split launch a sequence's last bits depend on the batch it is in.
  */
 int64_t nq_attn_bwd_split_workspace_bytes(int B, int Hq, int Hkv, int S, int T, int D, int dtype,
                                           int causal);
